@@ -58,6 +58,16 @@ unsafe extern "C" {
         stream: *mut c_void) -> c_int;
     pub fn ullm_hip_qkv_proj_workspace_bytes(rows: c_int, n_head: c_int, n_kv_head: c_int,
         head_dim: c_int) -> usize;
+    pub fn ullm_hip_qkv_gemm_append(x: *const f32, in_dim: c_int, w_q: *const c_void,
+        w_k: *const c_void, w_v: *const c_void, w_dtype: c_int, x_bits: c_int,
+        q_bias: *const f32, k_bias: *const f32, v_bias: *const f32, q_norm: *const f32,
+        k_norm: *const f32, eps: f32, rope_cs: *const f32, rope_n_pos: c_int, rope_neox: c_int,
+        rotary_dim: c_int, rows: c_int, start_pos: c_int, n_head: c_int, n_kv_head: c_int,
+        head_dim: c_int, q_out: *mut c_void, q_dtype: c_int, k_cache: *mut c_void,
+        v_cache: *mut c_void, kv_dtype: c_int, kv_stride: i64, workspace: *mut c_void,
+        workspace_bytes: usize, stream: *mut c_void) -> c_int;
+    pub fn ullm_hip_qkv_gemm_workspace_bytes(rows: c_int, in_dim: c_int, w_dtype: c_int,
+        x_bits: c_int, n_head: c_int, n_kv_head: c_int, head_dim: c_int) -> usize;
     pub fn ullm_hip_paged_decode_workspace_bytes(batch: c_int, n_head: c_int, n_kv_head: c_int,
         head_dim: c_int, max_len: c_int, window: c_int) -> usize;
     pub fn ullm_hip_attn_decode_paged(q: *const f32, k_pages: *const c_void,

@@ -187,6 +187,29 @@ int ullm_hip_qkv_proj_append(const float *x, int in_dim, const void *w_q, const 
  * it does not split head vectors). */
 size_t ullm_hip_qkv_proj_workspace_bytes(int rows, int n_head, int n_kv_head, int head_dim);
 
+/* ullm_hip_qkv_proj_append for many rows: the projections run as one MFMA GEMM
+ * over the three weight matrices (the weights are read once per call, not per
+ * row) into the workspace, the append follows.  Same arguments and result as
+ * ullm_hip_qkv_proj_append (any number of rows), plus
+ * x_bits: significant bits of x that enter the products, 16 (as
+ *         ullm_hip_matmul) or 24; with f16 weights x carries 22 bits (relative
+ *         to no less than 2^-17 of its row's largest value) whatever x_bits is
+ * workspace: DEVICE memory of ullm_hip_qkv_gemm_workspace_bytes, 256-byte
+ *         aligned; needs no initialisation, one call at a time.
+ * An operand of 2 GiB or more (rows or outputs times in_dim, 16-bit) is
+ * refused, and ullm_hip_qkv_gemm_workspace_bytes returns 0 for it. */
+int ullm_hip_qkv_gemm_append(const float *x, int in_dim, const void *w_q, const void *w_k,
+                             const void *w_v, int w_dtype, int x_bits, const float *q_bias,
+                             const float *k_bias, const float *v_bias, const float *q_norm,
+                             const float *k_norm, float eps, const float *rope_cs,
+                             int rope_n_pos, int rope_neox, int rotary_dim, int rows,
+                             int start_pos, int n_head, int n_kv_head, int head_dim, void *q_out,
+                             int q_dtype, void *k_cache, void *v_cache, int kv_dtype,
+                             int64_t kv_stride, void *workspace, size_t workspace_bytes,
+                             void *stream);
+size_t ullm_hip_qkv_gemm_workspace_bytes(int rows, int in_dim, int w_dtype, int x_bits, int n_head,
+                                         int n_kv_head, int head_dim);
+
 /* Batched projection for prefill: y[s*out_dim + o] = sum_i w[o*in_dim + i] *
  * x[s*in_dim + i] for s < n_cols, o < out_dim.  Replaces the reference's
  * batched matmul (crates/ullm-metal/src/forward.rs:675-726, kernel

@@ -133,6 +133,29 @@ def test_proj_append_validation():
     assert wsz(2048, 32, 8, 128) == 0  # prefill rows: no split
 
 
+def test_qkv_gemm_validation():
+    f, wsz = L.lib().ullm_hip_qkv_gemm_append, L.lib().ullm_hip_qkv_gemm_workspace_bytes
+
+    def call(**kw):
+        a = dict(x=64, i=256, wq=64, wk=64, wv=64, wdt=L.DT_F16, bits=24, qb=None, kb=None, vb=None,
+                 qn=None, kn=None, eps=1e-6, cs=64, npos=99, neox=1, rd=64, rows=16, sp=0, h=4, hk=2,
+                 d=64, qo=64, qdt=L.DT_F32, kc=64, vc=64, kvdt=L.DT_F32, kvs=128, ws=None, wsb=0, st=None)
+        a.update(kw)
+        return f(*a.values())
+
+    assert call(wdt=5) == L.E_UNSUPPORTED and call(d=96) == L.E_UNSUPPORTED
+    for bad in (dict(bits=8), dict(i=252), dict(rows=-1), dict(sp=-1), dict(rd=66), dict(kvs=64),
+                dict(h=3), dict(x=None), dict(wk=72), dict(npos=15), dict(rows=1 << 24, npos=1 << 25)):
+        assert call(**bad) == L.E_INVALID, bad
+    assert call(rows=0) == L.OK
+    assert call() == L.E_WORKSPACE
+    n = wsz(16, 256, L.DT_F16, 24, 4, 2, 64)
+    assert call(ws=256, wsb=n - 1) == L.E_WORKSPACE and call(ws=264, wsb=n) == L.E_INVALID
+    for bad in ((0, 256, 1, 24, 4, 2, 64), (16, 252, 1, 24, 4, 2, 64), (16, 256, 1, 20, 4, 2, 64),
+                (1 << 24, 256, 1, 24, 4, 2, 64)):
+        assert wsz(*bad) == 0, bad
+
+
 def test_matmul_validation():
     f = L.lib().ullm_hip_matmul
 

@@ -1,0 +1,108 @@
+"""The many-row Q/K/V projection (ullm_hip_qkv_gemm_append): its GEMM against
+an f64 product of the same inputs, its append against qkv_append, and the rule
+that chooses it against the matvec path."""
+import pytest
+import torch
+
+from ullm_amd import attention as A
+
+pytestmark = pytest.mark.gpu
+
+DT = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
+
+
+def _inputs(dev, rows, in_dim, H, Hk, D, wdt, seed):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    x = torch.randn(rows, in_dim, device=dev, generator=g)
+    ws = [(torch.randn(n * D, in_dim, device=dev, generator=g) / in_dim ** 0.5).to(DT[wdt])
+          for n in (H, Hk, Hk)]
+    return x, ws
+
+
+def _raw(x, ws, H, Hk, D, bits, start=0):
+    """The projections alone: no bias or norm, and a RoPE table of zero angles."""
+    rows = x.shape[0]
+    cs = torch.zeros(start + rows, D // 2, 2, device=x.device)
+    cs[..., 0] = 1
+    kc = torch.full((start + rows + 1, Hk * D), 7.0, device=x.device)
+    vc, q = kc.clone(), torch.empty(rows, H * D, device=x.device)
+    assert A._proj_gemm(x, *ws, kc, vc, cs, start, H, Hk, D, D, True, None, None, 1e-6, None, None,
+                        None, q, Hk * D, bits, None)
+    for c in (kc, vc):  # rows outside start.. are untouched
+        assert bool((c[:start] == 7).all()) and bool((c[start + rows:] == 7).all())
+    return q, kc[start:start + rows], vc[start:start + rows]
+
+
+# Rows on both sides of the token tiles (32, 64, 128), outputs that leave part
+# of every output tile (128, 256, 384) empty, in_dim below a step, with a tail
+# of 8, 24 and 40 dims, and long enough to be split over several key ranges.
+@pytest.mark.parametrize("wdt,bits", [("bf16", 16), ("bf16", 24), ("f16", 24), ("f32", 24)])
+@pytest.mark.parametrize("rows,in_dim,H,Hk,D", [
+    (1, 8, 1, 1, 64), (31, 40, 3, 1, 64), (33, 264, 4, 2, 64), (64, 1048, 2, 2, 256),
+    (65, 2560, 8, 4, 128), (129, 1032, 9, 3, 128), (383, 544, 32, 8, 64), (1025, 512, 16, 4, 128),
+])
+def test_projection_vs_f64(dev, rows, in_dim, H, Hk, D, wdt, bits):
+    print(f"[qkv-gemm] rows{rows} in{in_dim} H{H} Hk{Hk} D{D} {wdt} bits{bits}", flush=True)
+    x, ws = _inputs(dev, rows, in_dim, H, Hk, D, wdt, 5)
+    # rows over 2^-60 .. 2^60, the largest element 2^20 times the others in one
+    x *= torch.exp2(torch.randint(-60, 61, (rows, 1), device=dev, dtype=torch.float32))
+    x[0, 0] *= 2.0 ** 20
+    # relative residual of the planes, plus the f32 additions (in_dim of them
+    # at most); f16 planes also lose 2^-39 of the row's largest |x|
+    eps = (2.0 ** -16 if bits == 16 else 2.0 ** -21) + in_dim * 2.0 ** -24
+    for y, w in zip(_raw(x, ws, H, Hk, D, bits, start=2), ws):
+        w64 = w.double()
+        ref = x.double() @ w64.t().contiguous()
+        bound = eps * (x.double().abs() @ w64.abs().t().contiguous())
+        if wdt == "f16":
+            bound += 2.0 ** -39 * x.double().abs().amax(1, keepdim=True) * w64.abs().sum(1)
+        assert bool(((y.double() - ref).abs() <= bound + 1e-37).all())
+
+
+@pytest.mark.parametrize("wdt,bits", [("bf16", 16), ("bf16", 24), ("f16", 24), ("f32", 24)])
+def test_infinities_and_nans_stay_in_their_rows(dev, wdt, bits):
+    rows, in_dim, H, Hk, D = 40, 96, 2, 1, 64
+    print(f"[qkv-gemm-inf] {wdt} bits{bits}", flush=True)
+    x, ws = _inputs(dev, rows, in_dim, H, Hk, D, wdt, 6)
+    clean = _raw(x, ws, H, Hk, D, bits)
+    x2 = x.clone()
+    x2[3, 5], x2[7, 0], x2[9, 90] = float("inf"), float("nan"), -3.4028e38
+    x2[11] = 0
+    got = _raw(x2, ws, H, Hk, D, bits)
+    for y, c in zip(got, clean):
+        keep = [r for r in range(rows) if r not in (3, 7, 9, 11)]
+        assert torch.equal(y[keep], c[keep])
+        assert bool((y[11] == 0).all())
+    y, w = got[2], ws[2]  # v: no RoPE (whose zero sines make NaN of an infinity)
+    assert torch.equal(y[3], torch.where(w[:, 5] > 0, float("inf"), -float("inf")))
+    assert bool(torch.isnan(y[7]).all())
+    ref = x2[9].double() @ w.double().t().contiguous()
+    assert bool(((y[9].double() - ref).abs() <= 1e-4 * ref.abs()).all())
+
+
+@pytest.mark.parametrize("kvdt", ["f32", "bf16"])
+@pytest.mark.parametrize("rows,D,wdt,neox,rd", [(11, 256, "f16", True, 256), (50, 128, "bf16", False, 128),
+                                                (70, 64, "f32", True, 32)])
+def test_append_and_rule_match_matvec(dev, rows, D, wdt, neox, rd, kvdt, monkeypatch):
+    """qkv_proj_append gives the same rows on both sides of its rule."""
+    print(f"[qkv-gemm-append] rows{rows} D{D} {wdt} kv={kvdt}", flush=True)
+    H, Hk, in_dim, start = 6, 2, 1536, 9
+    x, ws = _inputs(dev, rows, in_dim, H, Hk, D, wdt, 8)
+    cs = A.rope_table(start + rows, rd, 1e4, device=dev)
+    g = torch.Generator(device=dev).manual_seed(9)
+    qn, kn = (torch.randn(D, device=dev, generator=g) for _ in range(2))
+    qb, kb, vb = (torch.randn(n * D, device=dev, generator=g) for n in (H, Hk, Hk))
+    got = []
+    for pays in (True, False):
+        monkeypatch.setattr(A, "_gemm_pays", lambda *a: pays)
+        kc = torch.zeros(start + rows, Hk * D, device=dev, dtype=DT[kvdt])
+        vc = torch.zeros_like(kc)
+        q = A.qkv_proj_append(x, *ws, kc, vc, cs, start_pos=start, n_head=H, n_kv_head=Hk, head_dim=D,
+                              rotary_dim=rd, neox=neox, q_norm=qn, k_norm=kn, q_bias=qb, k_bias=kb,
+                              v_bias=vb, q_dtype=DT[kvdt])
+        got.append((q.float(), kc.float(), vc.float()))
+    # f32 sums in another order; a 16-bit store can round one step (2^-7) apart
+    for a, b in zip(*got):
+        assert float((a - b).norm() / b.norm()) <= (2e-6 if kvdt == "f32" else 5e-4)
+        step = 2.0 ** -7 * b.abs() if kvdt == "bf16" else 0
+        assert bool(((a - b).abs() <= 2e-5 + step).all())

@@ -276,6 +276,42 @@ def proj_workspace(rows, n_head, n_kv_head, head_dim, device="cuda"):
     return _proj_ws[key]
 
 
+def _gemm_pays(rows, n, in_dim, head_dim, w_dtype):
+    """Whether `rows` token rows of an [n, in_dim] projection run faster as
+    ullm_hip_qkv_gemm_append (every weight read once, three launches) than as
+    qkv_proj_append's matvec per row.  Measured (us, matvec / GEMM, 24 bits):
+    bf16 2560 -> 6144: 8 rows 20.8 / 24.5, 12 rows 29.3 / 24.7, 300 rows 509 /
+    48; f16 2048 -> 3072: 16 rows 15.8 / 20.1, 40 rows 36.4 / 21.5; f32 2560 ->
+    6144: 16 rows 49 / 62, 40 rows 126 / 58; head_dim 256 from 256 head vectors
+    on (16 rows of 16, 2560 -> 4096): 112..117 / 24 (16-bit), 105 / 49 (f32)."""
+    if head_dim == 256 and rows * (n // head_dim) >= 256:
+        return True
+    return rows * n * in_dim >= (320_000_000 if w_dtype == torch.float32 else 160_000_000)
+
+
+def _proj_gemm(x, w_q, w_k, w_v, k_cache, v_cache, rope_cs, start_pos, n_head, n_kv_head, head_dim,
+               rotary_dim, neox, q_norm, k_norm, eps, q_bias, k_bias, v_bias, q_out, kv_stride,
+               x_bits, stream):
+    """ullm_hip_qkv_gemm_append with its scratch from the caching allocator;
+    False (nothing done) where an operand is too large for it."""
+    rows, in_dim = x.shape
+    lib = L.lib()
+    n = int(lib.ullm_hip_qkv_gemm_workspace_bytes(rows, in_dim, _dt(w_q), x_bits, n_head,
+                                                  n_kv_head, head_dim))
+    if n == 0:
+        return False
+    ws = torch.empty(n, dtype=torch.uint8, device=x.device)
+    if stream is not None:
+        ws.record_stream(stream)
+    L.check(lib.ullm_hip_qkv_gemm_append(
+        _ptr(x), in_dim, _ptr(w_q), _ptr(w_k), _ptr(w_v), _dt(w_q), x_bits, _ptr(q_bias),
+        _ptr(k_bias), _ptr(v_bias), _ptr(q_norm), _ptr(k_norm), float(eps), _ptr(rope_cs),
+        rope_cs.shape[0], int(bool(neox)), rotary_dim, rows, start_pos, n_head, n_kv_head, head_dim,
+        _ptr(q_out), _DT[q_out.dtype], _ptr(k_cache), _ptr(v_cache), _dt(k_cache), kv_stride,
+        _ptr(ws), n, _stream(stream)))
+    return True
+
+
 def qkv_proj_append(x, w_q, w_k, w_v, k_cache, v_cache, rope_cs, *, start_pos, n_head,
                     n_kv_head, head_dim, rotary_dim=None, neox=True, q_norm=None, k_norm=None,
                     eps=1e-6, q_bias=None, k_bias=None, v_bias=None, q_out=None, q_dtype=None,
@@ -302,6 +338,12 @@ def qkv_proj_append(x, w_q, w_k, w_v, k_cache, v_cache, rope_cs, *, start_pos, n
         q_out = torch.empty(rows, n_head * head_dim, dtype=q_dtype, device=x.device)
     if kv_stride is None:
         kv_stride = n_kv_head * head_dim
+    n = (n_head + 2 * n_kv_head) * head_dim
+    if rows <= 65535 and _gemm_pays(rows, n, in_dim, head_dim, w_q.dtype) and _proj_gemm(
+            x, w_q, w_k, w_v, k_cache, v_cache, rope_cs, start_pos, n_head, n_kv_head, head_dim,
+            rotary_dim, neox, q_norm, k_norm, eps, q_bias, k_bias, v_bias, q_out, kv_stride, 24,
+            stream):
+        return q_out
     if workspace is None:
         workspace = proj_workspace(rows, n_head, n_kv_head, head_dim, x.device)
     wsb = 0 if workspace is None else workspace.numel() * workspace.element_size()
@@ -402,6 +444,36 @@ class GpuAttention:
                           q_norm=qn, k_norm=kn, eps=p.eps, q_bias=qb, k_bias=kb, v_bias=vb,
                           q_dtype=q_dtype)
 
+    def _project_append(self, layer, xbs, wq, wk, wv, start_pos, norms, biases):
+        """The prompt's bf16 projections and append: a few rows as matvecs (f32
+        sums), more as one GEMM over the three weights (16 significant bits of
+        xbs, as ullm_hip_matmul).  None where the operands are not what those
+        take.  2560 -> 6144, us: 8 rows 21 (matvec), 40 rows 21, 2048 rows 129,
+        against 87, 89 and 171 of three matmuls and the append."""
+        p = self.p
+        D, n = p.head_dim, (p.n_head + 2 * p.n_kv_head) * p.head_dim
+        if not (xbs.is_cuda and xbs.dim() == 2 and xbs.dtype == torch.float32 and xbs.is_contiguous()
+                and xbs.shape[0] > 0 and xbs.shape[1] >= 8 and xbs.shape[1] % 8 == 0
+                and xbs.data_ptr() % 16 == 0):
+            return None
+        for w, m in ((wq, p.n_head), (wk, p.n_kv_head), (wv, p.n_kv_head)):
+            if not (w.is_cuda and w.dtype == torch.bfloat16 and tuple(w.shape) == (m * D, xbs.shape[1])
+                    and w.is_contiguous() and w.data_ptr() % 16 == 0):
+                return None
+        rows = xbs.shape[0]
+        kc, vc = self.key_cache[layer], self.val_cache[layer]
+        if rows < 32 and not _gemm_pays(rows, n, xbs.shape[1], D, wq.dtype):
+            return qkv_proj_append(xbs, wq, wk, wv, kc, vc, self.rope_cs, start_pos=start_pos,
+                                   n_head=p.n_head, n_kv_head=p.n_kv_head, head_dim=D,
+                                   rotary_dim=self.rotary_dim, neox=p.rope_neox, q_norm=norms[0],
+                                   k_norm=norms[1], eps=p.eps, q_bias=biases[0],
+                                   k_bias=biases[1], v_bias=biases[2], q_dtype=p.kv_dtype)
+        qr = torch.empty(rows, p.n_head * D, dtype=p.kv_dtype, device=xbs.device)
+        ok = _proj_gemm(xbs, wq, wk, wv, kc, vc, self.rope_cs, start_pos, p.n_head, p.n_kv_head, D,
+                        self.rotary_dim, p.rope_neox, norms[0], norms[1], p.eps, *biases, qr,
+                        self.kv_dim, 16, None)
+        return qr if ok else None
+
     def forward(self, layer: int, q, k, v, pos: int, q_norm=None, k_norm=None, q_bias=None,
                 k_bias=None, v_bias=None):
         """Decode one token: q [n_head*D], k/v [n_kv_head*D] f32 projections.
@@ -465,6 +537,12 @@ class GpuAttention:
         if start_pos + S > p.n_ctx:
             raise L.UllmHipError(L.E_INVALID, "prompt exceeds the context")
         if wq.dtype == torch.bfloat16:
+            qr = self._project_append(layer, xbs, wq, wk, wv, start_pos, (q_norm, k_norm),
+                                      (q_bias, k_bias, v_bias))
+            if qr is not None:
+                return attn_prefill(qr, self.key_cache[layer], self.val_cache[layer], p.n_head,
+                                    p.n_kv_head, p.head_dim, start_pos=start_pos,
+                                    window=self._window(layer), scale=self.scale)
             q = matmul(wq, xbs)
             k = matmul(wk, xbs)
             v = matmul(wv, xbs)

@@ -282,7 +282,7 @@ __global__ __launch_bounds__(kAppendWaves * 64) void qkv_append_kernel(
     const float *__restrict__ v_bias, const float *__restrict__ q_norm,
     const float *__restrict__ k_norm, float eps, const float *__restrict__ cs, int neox,
     int rotary_dim, int rows, int start_pos, int n_head, int n_kv_head, void *q_out,
-    void *k_cache, void *v_cache, int64_t kv_stride, PageMap pm, int gpw) {
+    void *k_cache, void *v_cache, int64_t kv_stride, PageMap pm, int gpw, AppendSrc as) {
     using Epi = SplitEpi<D>;
     constexpr int L = Epi::L, HPW = Epi::HPW;
     __shared__ float buf[kAppendWaves][HPW * D];
@@ -291,7 +291,7 @@ __global__ __launch_bounds__(kAppendWaves * 64) void qkv_append_kernel(
     const int row = blockIdx.x;
     const int gq = (n_head + HPW - 1) / HPW, gk = (n_kv_head + HPW - 1) / HPW;
     const int groups = gq + 2 * gk;
-    const int64_t q_dim = (int64_t)n_head * D, kv_dim = (int64_t)n_kv_head * D;
+    const int64_t q_dim = (int64_t)n_head * D;
     int pos = start_pos + row;
     int64_t crow = pos;
     if (pm.pos) {  // wave-uniform
@@ -324,13 +324,18 @@ __global__ __launch_bounds__(kAppendWaves * 64) void qkv_append_kernel(
             ok[b] = kind[b] != 3 && head[b] < (kind[b] == 0 ? n_head : n_kv_head);
             // uniform base + a 32-bit lane offset; a lane past the kind's last
             // head re-reads head h0 (in bounds) and stores nothing
-            const float *src = (kind[b] == 0 ? q_in + row * q_dim : (kind[b] == 1 ? k_in : v_in) + row * kv_dim) + (int64_t)h0 * D;
+            const float *src = (kind[b] == 0 ? q_in + row * as.q_ld : (kind[b] == 1 ? k_in : v_in) + row * as.kv_ld) + (int64_t)h0 * D;
             const float *bias = kind[b] == 0 ? q_bias : (kind[b] == 1 ? k_bias : v_bias);
             const unsigned lo = ok[b] ? loff : (unsigned)c0;
             float2 a{0.f, 0.f}, c{0.f, 0.f}, ba{0.f, 0.f}, bc{0.f, 0.f};
             if (kind[b] != 3) {
                 a = *(const float2 *)(src + lo);
                 c = *(const float2 *)(src + lo + D / 2);
+                for (int p = 1; p < as.ns; p++) {  // partial sums of a split projection
+                    src += as.ss;
+                    const float2 a2 = *(const float2 *)(src + lo), c2 = *(const float2 *)(src + lo + D / 2);
+                    a.x += a2.x, a.y += a2.y, c.x += c2.x, c.y += c2.y;
+                }
                 if (bias) {
                     ba = *(const float2 *)(bias + (int64_t)h0 * D + lo);
                     bc = *(const float2 *)(bias + (int64_t)h0 * D + lo + D / 2);
@@ -538,13 +543,13 @@ static void launch_kv(int kvdt, dim3 g, dim3 b, hipStream_t st, const float *qi,
                       const float *vi, const float *qb, const float *kb, const float *vb,
                       const float *qn, const float *kn, float eps, const float *cs, int neox,
                       int rd, int rows, int sp, int nh, int nkv, void *qo, void *kc, void *vc,
-                      int64_t kvs, PageMap pm, int gpw) {
+                      int64_t kvs, PageMap pm, int gpw, AppendSrc as) {
     if (kvdt == ULLM_DT_F32)
-        hipLaunchKernelGGL((qkv_append_kernel<D, QDT, ULLM_DT_F32>), g, b, 0, st, qi, ki, vi, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, pm, gpw);
+        hipLaunchKernelGGL((qkv_append_kernel<D, QDT, ULLM_DT_F32>), g, b, 0, st, qi, ki, vi, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, pm, gpw, as);
     else if (kvdt == ULLM_DT_F16)
-        hipLaunchKernelGGL((qkv_append_kernel<D, QDT, ULLM_DT_F16>), g, b, 0, st, qi, ki, vi, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, pm, gpw);
+        hipLaunchKernelGGL((qkv_append_kernel<D, QDT, ULLM_DT_F16>), g, b, 0, st, qi, ki, vi, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, pm, gpw, as);
     else
-        hipLaunchKernelGGL((qkv_append_kernel<D, QDT, ULLM_DT_BF16>), g, b, 0, st, qi, ki, vi, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, pm, gpw);
+        hipLaunchKernelGGL((qkv_append_kernel<D, QDT, ULLM_DT_BF16>), g, b, 0, st, qi, ki, vi, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, pm, gpw, as);
 }
 
 template <int D>
@@ -552,10 +557,10 @@ static void launch_q(int qdt, int kvdt, dim3 g, dim3 b, hipStream_t st, const fl
                      const float *ki, const float *vi, const float *qb, const float *kb,
                      const float *vb, const float *qn, const float *kn, float eps,
                      const float *cs, int neox, int rd, int rows, int sp, int nh, int nkv,
-                     void *qo, void *kc, void *vc, int64_t kvs, PageMap pm, int gpw) {
-    if (qdt == ULLM_DT_F32) launch_kv<D, ULLM_DT_F32>(kvdt, g, b, st, qi, ki, vi, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, pm, gpw);
-    else if (qdt == ULLM_DT_F16) launch_kv<D, ULLM_DT_F16>(kvdt, g, b, st, qi, ki, vi, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, pm, gpw);
-    else launch_kv<D, ULLM_DT_BF16>(kvdt, g, b, st, qi, ki, vi, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, pm, gpw);
+                     void *qo, void *kc, void *vc, int64_t kvs, PageMap pm, int gpw, AppendSrc as) {
+    if (qdt == ULLM_DT_F32) launch_kv<D, ULLM_DT_F32>(kvdt, g, b, st, qi, ki, vi, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, pm, gpw, as);
+    else if (qdt == ULLM_DT_F16) launch_kv<D, ULLM_DT_F16>(kvdt, g, b, st, qi, ki, vi, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, pm, gpw, as);
+    else launch_kv<D, ULLM_DT_BF16>(kvdt, g, b, st, qi, ki, vi, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, pm, gpw, as);
 }
 
 // Grid of qkv_append_kernel: one token row per blockIdx.x; a row's head
@@ -570,6 +575,20 @@ static dim3 append_grid(int rows, int n_head, int n_kv_head, int head_dim, int &
     gpw = rows < kAppendSplitBelow ? kAppendWaves * kBatch : groups;
     if (env > 0) gpw = env;
     return dim3((unsigned)rows, (unsigned)((groups + gpw - 1) / gpw));
+}
+
+int append_rows(const float *q, const float *k, const float *v, AppendSrc as, const float *qb,
+                const float *kb, const float *vb, const float *qn, const float *kn, float eps,
+                const float *cs, int neox, int rd, int rows, int sp, int nh, int nkv, int D, void *qo,
+                int qdt, void *kc, void *vc, int kvdt, int64_t kvs, hipStream_t st) {
+    int gpw;
+    const dim3 g = append_grid(rows, nh, nkv, D, gpw), b(kAppendWaves * 64);
+    switch (D) {
+        case 64: launch_q<64>(qdt, kvdt, g, b, st, q, k, v, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, PageMap{}, gpw, as); break;
+        case 128: launch_q<128>(qdt, kvdt, g, b, st, q, k, v, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, PageMap{}, gpw, as); break;
+        default: launch_q<256>(qdt, kvdt, g, b, st, q, k, v, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, PageMap{}, gpw, as); break;
+    }
+    return check_hip(hipGetLastError(), "qkv_append launch");
 }
 
 }  // namespace ullm
@@ -625,15 +644,11 @@ extern "C" int ullm_hip_qkv_append(const float *q_in, const float *k_in, const f
                          rope_n_pos, start_pos + rows);
     if (q_out == (void *)q_in && q_dtype != ULLM_DT_F32)
         return set_error(ULLM_HIP_E_INVALID, "qkv_append: in-place q needs q_dtype f32");
-    int gpw;
-    const dim3 grid = append_grid(rows, n_head, n_kv_head, head_dim, gpw), block(kAppendWaves * 64);
-    hipStream_t st = (hipStream_t)stream;
-    switch (head_dim) {
-        case 64: launch_q<64>(q_dtype, kv_dtype, grid, block, st, q_in, k_in, v_in, q_bias, k_bias, v_bias, q_norm, k_norm, eps, rope_cs, rope_neox, rotary_dim, rows, start_pos, n_head, n_kv_head, q_out, k_cache, v_cache, kv_stride, PageMap{}, gpw); break;
-        case 128: launch_q<128>(q_dtype, kv_dtype, grid, block, st, q_in, k_in, v_in, q_bias, k_bias, v_bias, q_norm, k_norm, eps, rope_cs, rope_neox, rotary_dim, rows, start_pos, n_head, n_kv_head, q_out, k_cache, v_cache, kv_stride, PageMap{}, gpw); break;
-        default: launch_q<256>(q_dtype, kv_dtype, grid, block, st, q_in, k_in, v_in, q_bias, k_bias, v_bias, q_norm, k_norm, eps, rope_cs, rope_neox, rotary_dim, rows, start_pos, n_head, n_kv_head, q_out, k_cache, v_cache, kv_stride, PageMap{}, gpw); break;
-    }
-    return check_hip(hipGetLastError(), "qkv_append launch");
+    return append_rows(q_in, k_in, v_in,
+                       AppendSrc{(int64_t)n_head * head_dim, (int64_t)n_kv_head * head_dim, 1, 0},
+                       q_bias, k_bias, v_bias, q_norm, k_norm, eps, rope_cs, rope_neox, rotary_dim,
+                       rows, start_pos, n_head, n_kv_head, head_dim, q_out, q_dtype, k_cache,
+                       v_cache, kv_dtype, kv_stride, (hipStream_t)stream);
 }
 
 extern "C" int ullm_hip_qkv_append_paged(const float *q_in, const float *k_in, const float *v_in,
@@ -670,13 +685,14 @@ extern "C" int ullm_hip_qkv_append_paged(const float *q_in, const float *k_in, c
         return set_error(ULLM_HIP_E_INVALID, "qkv_append_paged: in-place q needs q_dtype f32");
     const PageMap pm{positions, block_table, table_stride, __builtin_ctz(page_size), n_pages,
                      rope_n_pos};
+    const AppendSrc as{(int64_t)n_head * head_dim, (int64_t)n_kv_head * head_dim, 1, 0};
     int gpw;
     const dim3 grid = append_grid(rows, n_head, n_kv_head, head_dim, gpw), block(kAppendWaves * 64);
     hipStream_t st = (hipStream_t)stream;
     switch (head_dim) {
-        case 64: launch_q<64>(q_dtype, kv_dtype, grid, block, st, q_in, k_in, v_in, q_bias, k_bias, v_bias, q_norm, k_norm, eps, rope_cs, rope_neox, rotary_dim, rows, 0, n_head, n_kv_head, q_out, k_pages, v_pages, kv_stride, pm, gpw); break;
-        case 128: launch_q<128>(q_dtype, kv_dtype, grid, block, st, q_in, k_in, v_in, q_bias, k_bias, v_bias, q_norm, k_norm, eps, rope_cs, rope_neox, rotary_dim, rows, 0, n_head, n_kv_head, q_out, k_pages, v_pages, kv_stride, pm, gpw); break;
-        default: launch_q<256>(q_dtype, kv_dtype, grid, block, st, q_in, k_in, v_in, q_bias, k_bias, v_bias, q_norm, k_norm, eps, rope_cs, rope_neox, rotary_dim, rows, 0, n_head, n_kv_head, q_out, k_pages, v_pages, kv_stride, pm, gpw); break;
+        case 64: launch_q<64>(q_dtype, kv_dtype, grid, block, st, q_in, k_in, v_in, q_bias, k_bias, v_bias, q_norm, k_norm, eps, rope_cs, rope_neox, rotary_dim, rows, 0, n_head, n_kv_head, q_out, k_pages, v_pages, kv_stride, pm, gpw, as); break;
+        case 128: launch_q<128>(q_dtype, kv_dtype, grid, block, st, q_in, k_in, v_in, q_bias, k_bias, v_bias, q_norm, k_norm, eps, rope_cs, rope_neox, rotary_dim, rows, 0, n_head, n_kv_head, q_out, k_pages, v_pages, kv_stride, pm, gpw, as); break;
+        default: launch_q<256>(q_dtype, kv_dtype, grid, block, st, q_in, k_in, v_in, q_bias, k_bias, v_bias, q_norm, k_norm, eps, rope_cs, rope_neox, rotary_dim, rows, 0, n_head, n_kv_head, q_out, k_pages, v_pages, kv_stride, pm, gpw, as); break;
     }
     return check_hip(hipGetLastError(), "qkv_append_paged launch");
 }

@@ -128,6 +128,20 @@ int decode_f32_paged(const float *q, const void *kp, const void *vp, int64_t kvs
                      const int32_t *lens, int max_len, int win, int batch, int nh, int nkv, int D,
                      float qs, float *out, void *ws, size_t ws_bytes, hipStream_t st);
 
+// Rows read by the fused append: row r of q (k, v) starts q_ld (kv_ld)
+// elements after row r - 1, and is the sum of ns partials ss elements apart.
+struct AppendSrc {
+    int64_t q_ld, kv_ld;
+    int ns;
+    int64_t ss;
+};
+// The append of qkv_append over such rows (append.hip), arguments checked by
+// the caller.
+int append_rows(const float *q, const float *k, const float *v, AppendSrc src, const float *qb,
+                const float *kb, const float *vb, const float *qn, const float *kn, float eps,
+                const float *cs, int neox, int rd, int rows, int sp, int nh, int nkv, int D, void *qo,
+                int qdt, void *kc, void *vc, int kvdt, int64_t kvs, hipStream_t st);
+
 constexpr float kLog2e = 1.4426950408889634f;
 
 }  // namespace ullm
