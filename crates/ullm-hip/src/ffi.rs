@@ -88,6 +88,18 @@ unsafe extern "C" {
         block_table: *const i32, table_len: c_int, s: c_int, start_pos: c_int, window: c_int,
         n_head: c_int, n_kv_head: c_int, head_dim: c_int, scale: f32, out: *mut f32,
         stream: *mut c_void) -> c_int;
+    pub fn ullm_hip_attn_prefill_paged_ws(q: *const c_void, k_pages: *const c_void,
+        v_pages: *const c_void, dtype: c_int, kv_stride: i64, page_size: c_int, n_pages: c_int,
+        block_table: *const i32, table_len: c_int, s: c_int, start_pos: c_int, window: c_int,
+        n_head: c_int, n_kv_head: c_int, head_dim: c_int, scale: f32, out: *mut f32,
+        workspace: *mut c_void, workspace_bytes: usize, stream: *mut c_void) -> c_int;
+    pub fn ullm_hip_attn_prefill_ws(q: *const c_void, k_cache: *const c_void,
+        v_cache: *const c_void, dtype: c_int, kv_stride: i64, s: c_int, start_pos: c_int,
+        window: c_int, n_head: c_int, n_kv_head: c_int, head_dim: c_int, scale: f32,
+        out: *mut f32, workspace: *mut c_void, workspace_bytes: usize,
+        stream: *mut c_void) -> c_int;
+    pub fn ullm_hip_prefill_workspace_bytes(dtype: c_int, s: c_int, start_pos: c_int,
+        window: c_int, n_head: c_int, n_kv_head: c_int, head_dim: c_int) -> usize;
     pub fn ullm_hip_matmul(w: *const c_void, w_dtype: c_int, x: *const f32, y: *mut f32,
         in_dim: c_int, out_dim: c_int, n_cols: c_int, stream: *mut c_void) -> c_int;
 }

@@ -128,6 +128,21 @@ int ullm_hip_attn_prefill(const void *q, const void *k_cache, const void *v_cach
                           int64_t kv_stride, int S, int start_pos, int window, int n_head,
                           int n_kv_head, int head_dim, float scale, float *out, void *stream);
 
+/* The two prefill entry points with scratch: where few rows attend many keys (a
+ * short prompt, or a chunk of one at a large start_pos) the key range of a
+ * row is then split over several workgroups and their partial results are
+ * merged in a second launch.  Same arguments and result otherwise; workspace
+ * is DEVICE memory, 256-byte aligned, of ullm_hip_prefill_workspace_bytes
+ * (contiguous and paged alike; 0: the call is not split), needs no
+ * initialisation and serves one call at a time.  NULL or a smaller one: the
+ * call runs unsplit, as the entry point without it does. */
+int ullm_hip_attn_prefill_ws(const void *q, const void *k_cache, const void *v_cache, int dtype,
+                             int64_t kv_stride, int S, int start_pos, int window, int n_head,
+                             int n_kv_head, int head_dim, float scale, float *out,
+                             void *workspace, size_t workspace_bytes, void *stream);
+size_t ullm_hip_prefill_workspace_bytes(int dtype, int S, int start_pos, int window, int n_head,
+                                        int n_kv_head, int head_dim);
+
 /* Fills host memory `cs` ([n_pos][rotary_dim/2][2] f32, (cos, sin)) with the
  * RoPE angles of the CPU reference: freq_i = theta.powf(2i/rd).recip() and
  * (sin, cos) = (pos*freq_i).sin_cos() in f32
@@ -290,6 +305,14 @@ int ullm_hip_attn_prefill_paged(const void *q, const void *k_pages, const void *
                                 const int32_t *block_table, int table_len, int s, int start_pos,
                                 int window, int n_head, int n_kv_head, int head_dim, float scale,
                                 float *out, void *stream);
+
+/* ullm_hip_attn_prefill_paged with scratch (see ullm_hip_attn_prefill_ws). */
+int ullm_hip_attn_prefill_paged_ws(const void *q, const void *k_pages, const void *v_pages,
+                                   int dtype, int64_t kv_stride, int page_size, int n_pages,
+                                   const int32_t *block_table, int table_len, int s,
+                                   int start_pos, int window, int n_head, int n_kv_head,
+                                   int head_dim, float scale, float *out, void *workspace,
+                                   size_t workspace_bytes, void *stream);
 
 /* Measurement calibration (no counterpart in the reference): reads `bytes`
  * bytes of DEVICE memory at `src` (16-byte aligned) once, with 16-byte loads

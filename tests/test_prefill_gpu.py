@@ -89,7 +89,7 @@ def p16_geometry(S, H, Hk, start_pos=0, window=0):
     hw1 = hw_of(8)
     grid1 = (S + 128 // hw1 - 1) // (128 // hw1) * (H // hw1)
     binding = 0 < window < start_pos + S
-    ks = 2 if grid1 < 256 or (grid1 == 256 and not binding) else 1
+    ks = 2 if grid1 <= (128 if binding else 256) else 1
     hw = hw_of(8 // ks)
     ur = 16 * (8 // ks) // hw
     ds = 2 if ks == 2 and (S + ur - 1) // ur * (H // hw) * 2 <= 256 else 1

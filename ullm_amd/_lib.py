@@ -30,6 +30,10 @@ SIGNATURES = {
     "ullm_hip_attn_prefill": (
         _i, [_vp, _vp, _vp, _i, _i64, _i, _i, _i, _i, _i, _i, _f, _vp, _vp]
     ),
+    "ullm_hip_attn_prefill_ws": (
+        _i, [_vp, _vp, _vp, _i, _i64, _i, _i, _i, _i, _i, _i, _f, _vp, _vp, _sz, _vp]
+    ),
+    "ullm_hip_prefill_workspace_bytes": (_sz, [_i, _i, _i, _i, _i, _i, _i]),
     "ullm_hip_rope_table": (_i, [_vp, _i, _i, _f]),
     "ullm_hip_stream_read": (_i, [_vp, _sz, _i, _vp, _vp]),
     "ullm_hip_qkv_append": (
@@ -52,6 +56,9 @@ SIGNATURES = {
     "ullm_hip_matmul": (_i, [_vp, _i, _vp, _vp, _i, _i, _i, _vp]),
     "ullm_hip_attn_prefill_paged": (
         _i, [_vp, _vp, _vp, _i, _i64, _i, _i, _vp, _i, _i, _i, _i, _i, _i, _i, _f, _vp, _vp]
+    ),
+    "ullm_hip_attn_prefill_paged_ws": (
+        _i, [_vp, _vp, _vp, _i, _i64, _i, _i, _vp, _i, _i, _i, _i, _i, _i, _i, _f, _vp, _vp, _sz, _vp]
     ),
     "ullm_hip_qkv_append_paged": (
         _i,

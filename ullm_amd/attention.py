@@ -8,6 +8,7 @@ PyTorch fallback: without the library or a GPU the calls raise.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import math
 from dataclasses import dataclass
 from typing import Optional
@@ -155,6 +156,31 @@ def qkv_append_paged(q, k, v, k_pages, v_pages, rope_cs, positions, block_table,
     return q_out
 
 
+# The scratch sizes depend on these numbers alone.
+@functools.lru_cache(maxsize=1024)
+def _prefill_bytes(dtype, S, start_pos, window, n_head, n_kv_head, head_dim):
+    return int(L.lib().ullm_hip_prefill_workspace_bytes(dtype, S, start_pos, window, n_head,
+                                                        n_kv_head, head_dim))
+
+
+@functools.lru_cache(maxsize=1024)
+def _gemm_bytes(rows, in_dim, w_dtype, x_bits, n_head, n_kv_head, head_dim):
+    return int(L.lib().ullm_hip_qkv_gemm_workspace_bytes(rows, in_dim, w_dtype, x_bits, n_head,
+                                                         n_kv_head, head_dim))
+
+
+def _prefill_scratch(q, S, start_pos, window, n_head, n_kv_head, head_dim, stream):
+    """Scratch for a prefill call that splits its key ranges: (tensor, bytes),
+    or (None, 0) where it does not."""
+    n = _prefill_bytes(_dt(q), S, start_pos, window, n_head, n_kv_head, head_dim)
+    if n == 0:
+        return None, 0
+    ws = torch.empty(n, dtype=torch.uint8, device=q.device)
+    if stream is not None:
+        ws.record_stream(stream)
+    return ws, n
+
+
 def attn_prefill_paged(q, k_pages, v_pages, block_table, n_head, n_kv_head, head_dim, *,
                        start_pos=0, window=0, scale=None, out=None, stream=None):
     """Causal prefill of S rows (positions start_pos..) of one sequence whose
@@ -174,10 +200,11 @@ def attn_prefill_paged(q, k_pages, v_pages, block_table, n_head, n_kv_head, head
         scale = 1.0 / math.sqrt(head_dim)
     if out is None:
         out = torch.empty(S, n_head * head_dim, dtype=torch.float32, device=q.device)
-    rc = L.lib().ullm_hip_attn_prefill_paged(
+    ws, wsb = _prefill_scratch(q, S, start_pos, window, n_head, n_kv_head, head_dim, stream)
+    rc = L.lib().ullm_hip_attn_prefill_paged_ws(
         _ptr(q), _ptr(k_pages), _ptr(v_pages), _dt(q), kv_stride, page_size, n_pages,
         _ptr(block_table), block_table.numel(), S, start_pos, window, n_head, n_kv_head, head_dim,
-        float(scale), _ptr(out), _stream(stream))
+        float(scale), _ptr(out), _ptr(ws), wsb, _stream(stream))
     L.check(rc)
     return out
 
@@ -214,10 +241,11 @@ def attn_prefill(q, k_cache, v_cache, n_head, n_kv_head, head_dim, *, start_pos=
     rows = max(1, PREFILL_Q_MAX_BYTES // row_bytes)
     for r0 in range(0, max(S, 1), rows):
         n = min(rows, S - r0)
-        rc = L.lib().ullm_hip_attn_prefill(
+        ws, wsb = _prefill_scratch(q, n, start_pos + r0, window, n_head, n_kv_head, head_dim, stream)
+        rc = L.lib().ullm_hip_attn_prefill_ws(
             _ptr(q[r0:r0 + n]), _ptr(k_cache), _ptr(v_cache), _dt(q), kv_stride, n,
             start_pos + r0, window, n_head, n_kv_head, head_dim, float(scale),
-            _ptr(out[r0:r0 + n]), _stream(stream))
+            _ptr(out[r0:r0 + n]), _ptr(ws), wsb, _stream(stream))
         L.check(rc)
     return out
 
@@ -296,8 +324,7 @@ def _proj_gemm(x, w_q, w_k, w_v, k_cache, v_cache, rope_cs, start_pos, n_head, n
     False (nothing done) where an operand is too large for it."""
     rows, in_dim = x.shape
     lib = L.lib()
-    n = int(lib.ullm_hip_qkv_gemm_workspace_bytes(rows, in_dim, _dt(w_q), x_bits, n_head,
-                                                  n_kv_head, head_dim))
+    n = _gemm_bytes(rows, in_dim, _dt(w_q), x_bits, n_head, n_kv_head, head_dim)
     if n == 0:
         return False
     ws = torch.empty(n, dtype=torch.uint8, device=x.device)

@@ -227,13 +227,119 @@ __device__ __forceinline__ void page_tile(const KvPages &pg, const char *kc, con
     so = __builtin_amdgcn_readfirstlane((key0 & ((1 << pg.shift) - 1)) * rbg);
 }
 
+// Prefill with the key ranges split over workgroups.  The query rows are taken
+// in units of UR rows and the keys in tiles of `tile`; a unit of more than
+// `chunk` tiles is cut into parts of equal tile counts, each a workgroup of its
+// own that leaves (m, l) and the unnormalised O of its rows, which
+// launch_prefill_merge adds up.  Part p's O is a whole [S][n_head*D] plane,
+// its (m, l) a [S][n_head] plane of pairs.
+struct KeySplit {
+    int chunk, tile;
+    float *o;
+    float2 *ml;
+};
+// Key tiles [t0, t1) of unit u: the window start of its first row to the
+// causal end of its last.
+__host__ __device__ __forceinline__ void unit_tiles(int u, int UR, int S, int start_pos, int window,
+                                                    int tile, int &t0, int &t1) {
+    const int hi = start_pos + (u * UR + UR < S ? u * UR + UR : S);
+    const int lo = window > 0 && start_pos + u * UR + 1 - window > 0 ? start_pos + u * UR + 1 - window : 0;
+    t0 = lo / tile;
+    t1 = (hi + tile - 1) / tile;
+}
+// The unit's parts, and part `part`'s share of [t0, t1).
+__device__ __forceinline__ int part_tiles(const KeySplit &sp, int part, int &t0, int &t1) {
+    const int parts = (t1 - t0 + sp.chunk - 1) / sp.chunk, per = (t1 - t0 + parts - 1) / parts;
+    t0 += part * per;
+    t1 = min(t1, t0 + per);
+    return parts;
+}
+int launch_prefill_merge(int D, KeySplit sp, int UR, int S, int start_pos, int window, int n_head,
+                         float *out, hipStream_t st);
+// Host: the split of a call.  chunk: tiles per part of the longest unit, which
+// has `parts` of them (1: unsplit); bytes: the scratch for O and (m, l).
+struct SplitPlan {
+    int chunk, parts;
+    size_t ml_off, bytes;
+};
+// The units of a call: n workgroups' worth of them when unsplit (row units
+// times head groups), the longest and the average one in key tiles.
+struct UnitLoad {
+    double n, longest, avg;
+};
+inline UnitLoad unit_load(int S, int UR, int n_hg, int start_pos, int window, int tile) {
+    const int n = (S + UR - 1) / UR;
+    int a0, a1, b0, b1;
+    unit_tiles(0, UR, S, start_pos, window, tile, a0, a1);
+    unit_tiles(n - 1, UR, S, start_pos, window, tile, b0, b1);
+    const int last = b1 - b0 > a1 - a0 ? b1 - b0 : a1 - a0;
+    // lengths grow to a window's size, and stay there
+    const bool flat = window > 0 && b0 > 0;
+    const double ramp = flat && window > start_pos ? (double)(window - start_pos) / S : 0.;
+    const double avg = flat ? last - ramp * 0.5 * (last - (a1 - a0)) : 0.5 * (a1 - a0 + b1 - b0);
+    return UnitLoad{(double)n * n_hg, (double)last, avg};
+}
+// What a workgroup of a prefill kernel costs (us): per key tile when it has
+// the chip nearly alone and when every CU runs one, and once per workgroup.
+struct PrefillCost {
+    double alone, full, fixed;
+};
+// Estimated time of `wgs` workgroups over `total` tiles, the longest of
+// `longest` (one workgroup per CU at a time).
+inline double prefill_us(const PrefillCost &c, double wgs, double longest, double total) {
+    const double fill = wgs < 256 ? wgs / 256 : 1., ts = c.alone + (c.full - c.alone) * fill;
+    const int rounds = (int)((wgs + 255) / 256);
+    // equal workgroups run in whole rounds; unequal ones fill each other's gaps
+    const double avg = total / wgs, even = longest * rounds, mixed = total / 256 + 0.5 * avg;
+    const double tiles = avg > 0.9 * longest ? even : (mixed > longest ? mixed : longest);
+    return tiles * ts + c.fixed * rounds;
+}
+// The number of parts with the least estimate, against `unsplit` us without a
+// split (0: one part on the same kernel); the merge streams the partial results
+// at 4 TB/s.  A split has to win by an eighth and by 1.5 us: over 146 random
+// shapes (2..4096 rows at 0..16384, all dtypes and head_dims) the calls that it
+// splits ran 1.1 to 13 times faster, and none of the others moved.
+inline SplitPlan choose_split(const PrefillCost &c, const UnitLoad &u, double unsplit, int S, int n_head,
+                              int D) {
+    static const int env = env_override("ULLM_HIP_PREFILL_PARTS");  // tuning: parts of the longest unit (1: never)
+    SplitPlan pl{(int)u.longest, 1, 0, 0};
+    if (!(unsplit > 0)) unsplit = prefill_us(c, u.n, u.longest, u.n * u.avg);
+    double best = unsplit * 0.875 < unsplit - 1.5 ? unsplit * 0.875 : unsplit - 1.5;
+    if (u.n > 1024 && env < 2) return pl;  // the chip is full many times over
+    for (int p : {2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 40, 48, 64}) {
+        if (env > 0 ? p != env : 2 * p > u.longest + 1) continue;
+        const int chunk = ((int)u.longest + p - 1) / p, parts = ((int)u.longest + chunk - 1) / chunk;
+        const size_t ml_off = (size_t)parts * S * n_head * D * 4;
+        if (parts < 2 || ml_off > (256u << 20)) continue;
+        double mean = u.avg > 0.9 * u.longest ? parts : u.avg / chunk + 0.5;
+        mean = mean > parts ? parts : (mean < 1 ? 1 : mean);
+        const double us = prefill_us(c, u.n * mean, chunk, u.n * u.avg) + 2.5 +
+                          (double)S * n_head * D * 4 * (2 * mean + 1) / 4e6;
+        if (us < best || env > 1) {
+            best = us;
+            pl = SplitPlan{chunk, parts, ml_off, ml_off + (size_t)parts * S * n_head * 8};
+        }
+    }
+    return pl;
+}
+inline KeySplit split_at(const SplitPlan &pl, int tile, void *ws) {
+    return KeySplit{pl.chunk, tile, (float *)ws, (float2 *)((char *)ws + pl.ml_off)};
+}
+
 // Head_dim-256 prefill on 16-row waves, two per SIMD (prefill16.hip);
 // pgs.tab == nullptr for a contiguous cache.
+// ws: scratch for a split of the key ranges over workgroups, used where the
+// plan asks for one and ws_bytes holds it (prefill16_ws_bytes).
 int launch_prefill16(int dtype, const void *q, const void *kc, const void *vc, int64_t kvs, int S,
                      int start_pos, int window, int n_head, int kv_mul, float qs, float *out,
-                     hipStream_t st, KvPages pgs);
+                     hipStream_t st, KvPages pgs, void *ws = nullptr, size_t ws_bytes = 0);
+// The split prefill16_kernel takes for these shapes, and the estimate (us) of
+// the call without one.
+SplitPlan prefill16_split(int dtype, int S, int start_pos, int window, int n_head, int kv_mul, int D);
+double prefill16_us(int dtype, int S, int start_pos, int window, int n_head, int kv_mul, int D);
 int launch_prefill16_128(int dtype, const void *q, const void *kc, const void *vc, int64_t kvs,
                          int S, int start_pos, int window, int n_head, int kv_mul, float qs,
-                         float *out, hipStream_t st, KvPages pgs);
+                         float *out, hipStream_t st, KvPages pgs, void *ws = nullptr,
+                         size_t ws_bytes = 0);
 
 }  // namespace ullm

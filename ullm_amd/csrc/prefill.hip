@@ -374,11 +374,14 @@ __global__ __launch_bounds__(512) void prefill2_kernel(
 // than 2^8 (in the exp2 domain): P = exp2(s - m) then stays <= 256, exact in
 // f16's range, and the O/l rescale runs a handful of times per block instead
 // of on every new maximum.
-template <class T, int D>
+//
+// SPLIT: a workgroup owns one block and one part of its key tiles (KeySplit,
+// np parts at most), its two sets half of the part each.
+template <class T, int D, bool SPLIT = false>
 __global__ __launch_bounds__(512) void prefill4_kernel(
     const uint16_t *__restrict__ q, const char *__restrict__ kc, const char *__restrict__ vc,
     int64_t kv_stride, int S, int start_pos, int n_head, int kv_mul, int lhw, int ng, int np,
-    float qscale, float *__restrict__ out, KvPages pgs) {
+    float qscale, float *__restrict__ out, KvPages pgs, KeySplit sp) {
     using C = PF2<D>;
     constexpr int BN = C::BN, RB = C::RB, SLOTS = C::SLOTS, RPI = C::RPI, NIW = C::NIW;
     constexpr int TILE = C::TILE, NKT = C::NKT, NKS = C::NKS, NDT = C::NDT;
@@ -399,14 +402,18 @@ __global__ __launch_bounds__(512) void prefill4_kernel(
     const int hw = 1 << lhw, rw = 4 >> lhw, BLK = 32 * rw;
     const int upk = kv_mul >> lhw;  // units per kv head
     const int n_units = (n_head / kv_mul) * upk;
-    const int total = n_units * np;
+    const int per_unit = SPLIT ? ng * np : np;
+    const int total = n_units * per_unit;
     const int per_xcd = (total + 7) / 8;
     const int tsk = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (tsk >= total) return;
-    const int unit = tsk / np, pair = tsk % np;
+    const int unit = tsk / per_unit, pair = tsk % per_unit;
     const int kvh = unit / upk;
     const int head0 = kvh * kv_mul + (unit % upk) * hw;
-    const int gA = pair, gB = ng - 1 - pair != pair ? ng - 1 - pair : -1;
+    // SPLIT: blocks longest first, a block's parts side by side
+    const int kpart = SPLIT ? pair % np : 0;
+    const int gA = SPLIT ? ng - 1 - pair / np : pair;
+    const int gB = !SPLIT && ng - 1 - pair != pair ? ng - 1 - pair : -1;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -419,7 +426,12 @@ __global__ __launch_bounds__(512) void prefill4_kernel(
 
     // ---- the two tile streams ----
     const int rowA = gA * BLK, rowB = gB >= 0 ? gB * BLK : rowA;  // rowB: merged block
-    const int TA = (start_pos + min(rowA + BLK, S) + BN - 1) / BN;
+    int TA = (start_pos + min(rowA + BLK, S) + BN - 1) / BN, tfirst = 0, parts = 1;
+    if constexpr (SPLIT) {
+        parts = part_tiles(sp, kpart, tfirst, TA);
+        if (kpart >= parts) return;
+        TA -= tfirst;
+    }
     const int TB = gB >= 0 ? (start_pos + min(rowB + BLK, S) + BN - 1) / BN : 0;
     const int n_tot = TA + TB;
     // Set 0 takes 34/64 of the tiles: set 1's waves are younger and lose
@@ -431,7 +443,7 @@ __global__ __launch_bounds__(512) void prefill4_kernel(
     // item i of stream s -> key tile, and whether it belongs to block A
     // (only set 0 has A items when the block has a partner).
     auto item_tile = [&](int s_, int i) {
-        if (gB < 0) return s_ ? n0 + i : i;
+        if (gB < 0) return tfirst + (s_ ? n0 + i : i);
         if (s_ == 0) return i;
         const int t = n0 + i;
         return t < TB ? t : t - TB;
@@ -781,7 +793,12 @@ __global__ __launch_bounds__(512) void prefill4_kernel(
         const float mu = M == -INFINITY ? 0.f : M;
         const float a0 = __builtin_amdgcn_exp2f(m_run - mu), a1 = __builtin_amdgcn_exp2f(m1 - mu);
         const float den = l0 * a0 + l1 * a1;
-        const float inv = den > 0.f ? 1.0f / den : 0.f;
+        float inv = den > 0.f ? 1.0f / den : 0.f;
+        if (SPLIT && parts > 1) {  // left for the merge
+            inv = 1.0f;
+            const int qrow = rowB + sub + c32;
+            if (h2 == 0 && qrow < S) sp.ml[((int64_t)kpart * S + qrow) * n_head + head] = float2{M, den};
+        }
         const float w0 = a0 * inv, w1 = a1 * inv;
         u32x4 o1[NDT][4];
 #pragma unroll
@@ -816,9 +833,12 @@ __global__ __launch_bounds__(512) void prefill4_kernel(
         for (int c = lane; c < cpr; c += 64) {
             const u32x4 v = lds_read_b128(stg + r * (hw * D * 4) + (c ^ (r & 15)) * 16);
             lds_wait_any();
-            if (qrow < S)
-                __builtin_nontemporal_store(__builtin_bit_cast(f32x4, v),
-                                            (f32x4 *)(out + (int64_t)qrow * q_dim + (int64_t)head0 * D) + c);
+            const int64_t at = (int64_t)qrow * q_dim + (int64_t)head0 * D;
+            if (qrow >= S) continue;
+            if (SPLIT && parts > 1)
+                *((f32x4 *)(sp.o + (int64_t)kpart * S * q_dim + at) + c) = __builtin_bit_cast(f32x4, v);
+            else
+                __builtin_nontemporal_store(__builtin_bit_cast(f32x4, v), (f32x4 *)(out + at) + c);
         }
     }
 }
@@ -1128,17 +1148,23 @@ __global__ __launch_bounds__(256, 1) void prefill_sk_kernel(
 
 // head_dim 256: prefill16_kernel (16-row waves, two per SIMD), or on request
 // prefill_sk_kernel (split-K inside one-wave-per-SIMD workgroups).
+// Caller's scratch of one call (none: p == nullptr).
+struct Scratch {
+    void *p;
+    size_t bytes;
+};
+
 template <class T, int D, bool V2 = (D <= 128)>
 struct PrefillLaunch {
     static void run(const void *q, const void *kc, const void *vc, int64_t kvs, int S, int sp,
                     int win, int nh, int kv_mul, float qs, float *out, hipStream_t st,
-                    KvPages pgs = KvPages{}) {
+                    KvPages pgs, Scratch ws) {
         // prefill16_kernel; ULLM_HIP_PREFILL256=1 selects prefill_sk_kernel
         // instead, for comparison.
         static const int pick = env_override("ULLM_HIP_PREFILL256");
         if (pick != 1) {
             launch_prefill16(__is_same(T, BF16) ? ULLM_DT_BF16 : ULLM_DT_F16, q, kc, vc, kvs, S, sp,
-                             win, nh, kv_mul, qs, out, st, pgs);
+                             win, nh, kv_mul, qs, out, st, pgs, ws.p, ws.bytes);
             return;
         }
         const int nb = (S + 31) / 32;
@@ -1153,13 +1179,63 @@ template <class T, int D>
 struct PrefillLaunch<T, D, true> {
     static void run(const void *q, const void *kc, const void *vc, int64_t kvs, int S, int sp,
                     int win, int nh, int kv_mul, float qs, float *out, hipStream_t st,
-                    KvPages pgs = KvPages{});
+                    KvPages pgs, Scratch ws);
 };
+
+// head_dim 128, 16-bit caches, short prompts: prefill16_kernel (16-row waves;
+// K/V tiles shared by the GQA group; two key streams when units are few) when
+// prefill4's causal pairs would cover half the CUs or fewer.  Measured
+// (us, prefill4 -> prefill16): 12/2 heads S=1024 26.2 -> 16.5, S=2048
+// 39.4 -> 29.6; 32/8 heads S=512 18.8 -> 12.0, S=1024 27.3 -> 23.7,
+// S=1536 (192 pairs) 39.7 -> 42.6, S=2048 (256) 51.8 -> 59.9.
+// ULLM_HIP_PREFILL128=16 / =4 forces either kernel (tuning override).
+static bool prefill16_takes_128(int S, int sp, int win, int nh, int kv_mul) {
+    static const int e128 = env_override("ULLM_HIP_PREFILL128");
+    const int hw = kv_mul % 4 == 0 ? 4 : (kv_mul % 2 == 0 ? 2 : 1), rows = 32 * (4 / hw);
+    const int64_t pairs = (int64_t)(nh / hw) * (((S + rows - 1) / rows + 1) / 2);
+    return e128 == 16 || (e128 != 4 && !(win > 0 && win < sp + S) && pairs <= 128);
+}
+
+// Split of a 16-bit cache's causal prefill at head_dim 64 or 128, on
+// prefill4_kernel, against the kernel the call runs on unsplit.  Per 64-key
+// tile: 32/8 heads x 128, bf16: 8 rows at 20000 in 4 parts 85 us for 78 tiles a
+// workgroup; 512 rows at 7680 in 2 parts (256 workgroups) 82 us before the merge
+// for 64 tiles; x 64, f16: 1000 rows at 3000, 128 pairs, 86 us for 110 tiles.
+// Measured (us, unsplit -> split): 512 rows at 7680 135 -> 95, 128 at 16000 240 ->
+// 57, 8 at 20000 (32/4 heads) 301 -> 27, 1000 at 16000 (12/2) 265 -> 165, 1000 at
+// 3000 x 64 86 -> 64; 512, 1024 and 2048 rows at 0 stay unsplit (14, 29, 53
+// against 22, 43, 99).
+static SplitPlan prefill4_split(int S, int sp, int nh, int kv_mul, int D) {
+    const int hw = kv_mul % 4 == 0 ? 4 : (kv_mul % 2 == 0 ? 2 : 1), rows = 32 * (4 / hw);
+    const PrefillCost c = D == 128 ? PrefillCost{.88, 1.2, 9.} : PrefillCost{.6, .72, 8.};
+    const UnitLoad u = unit_load(S, rows, nh / hw, sp, 0, 64);
+    double unsplit;
+    if (D == 128 && prefill16_takes_128(S, sp, 0, nh, kv_mul)) {
+        unsplit = prefill16_us(ULLM_DT_BF16, S, sp, 0, nh, kv_mul, D);
+    } else {
+        const double blocks = u.n / (nh / hw), pairs = (double)(((int)blocks + 1) / 2) * (nh / hw);
+        const double len = blocks > 1 ? 2 * u.avg : u.longest;
+        unsplit = prefill_us(c, pairs, len, pairs * len);
+    }
+    return choose_split(c, u, unsplit, S, nh, D);
+}
+
+// prefill_f32_kernel's split (a unit per workgroup, or less).  Per 32-key tile,
+// 32/8 heads x 64: 777 rows (200 units) 29.6 us for 25 tiles; 500 rows at 4000 in
+// 2 parts (256 workgroups) 82.9, in 4 60.7.  Measured (us, pairs of units per
+// workgroup -> a unit each -> this rule's split): 777 rows 33.9 -> 29.6 -> 27.1,
+// 500 at 4000 256 -> 140 -> 61, 61 at 700 52 -> 27 -> 13, 2048 rows 80 -> 71, 4096
+// rows 216 -> 211, 2000 rows with window 300 35 -> 28.
+static SplitPlan prefill_f32_split(int S, int sp, int win, int nh, int kv_mul, int D) {
+    int hw = 1;
+    while (hw < 4 && kv_mul % (hw * 2) == 0) hw *= 2;
+    return choose_split(PrefillCost{1.0, .9, 5.}, unit_load(S, 128 / hw, nh / hw, sp, win, 32), 0., S, nh, D);
+}
 
 template <class T, int D>
 void PrefillLaunch<T, D, true>::run(const void *q, const void *kc, const void *vc, int64_t kvs,
                                     int S, int sp, int win, int nh, int kv_mul, float qs,
-                                    float *out, hipStream_t st, KvPages pgs) {
+                                    float *out, hipStream_t st, KvPages pgs, Scratch ws) {
     // Units of HW heads (HW | kv_mul, at most 4) x groups of RW = 4/HW 32-row blocks.
     const int hw = kv_mul % 4 == 0 ? 4 : (kv_mul % 2 == 0 ? 2 : 1);
     const int rw = 4 / hw;
@@ -1171,24 +1247,28 @@ void PrefillLaunch<T, D, true>::run(const void *q, const void *kc, const void *v
     const int paired = !(win > 0 && win < sp + S);
     const int total = n_units * np;
     const int per_xcd = (total + 7) / 8;
-    // head_dim 128, short prompts: prefill16_kernel (16-row waves; K/V tiles
-    // shared by the GQA group; two key streams when units are few) when
-    // prefill4's causal pairs would cover half the CUs or fewer.  Measured
-    // (us, prefill4 -> prefill16): 12/2 heads S=1024 26.2 -> 16.5, S=2048
-    // 39.4 -> 29.6; 32/8 heads S=512 18.8 -> 12.0, S=1024 27.3 -> 23.7,
-    // S=1536 (192 pairs) 39.7 -> 42.6, S=2048 (256) 51.8 -> 59.9.
-    // ULLM_HIP_PREFILL128=16 / =4 forces either kernel (tuning override).
-    static const int e128 = env_override("ULLM_HIP_PREFILL128");
-    if (D == 128 && (e128 == 16 || (e128 != 4 && paired && total <= 128))) {
+    if (paired) {
+        const SplitPlan pl = prefill4_split(S, sp, nh, kv_mul, D);
+        if (pl.parts > 1 && ws.p && ws.bytes >= pl.bytes) {
+            const KeySplit ksp = split_at(pl, 64, ws.p);
+            const int lhw = hw == 4 ? 2 : (hw == 2 ? 1 : 0);
+            hipLaunchKernelGGL((prefill4_kernel<T, D, true>), dim3((n_units * ng * pl.parts + 7) / 8 * 8),
+                               dim3(512), 0, st, (const uint16_t *)q, (const char *)kc, (const char *)vc,
+                               kvs, S, sp, nh, kv_mul, lhw, ng, pl.parts, qs, out, pgs, ksp);
+            launch_prefill_merge(D, ksp, 32 * rw, S, sp, 0, nh, out, st);
+            return;
+        }
+    }
+    if (D == 128 && prefill16_takes_128(S, sp, win, nh, kv_mul)) {
         launch_prefill16_128(__is_same(T, BF16) ? ULLM_DT_BF16 : ULLM_DT_F16, q, kc, vc, kvs, S, sp,
-                             win, nh, kv_mul, qs, out, st, pgs);
+                             win, nh, kv_mul, qs, out, st, pgs, ws.p, ws.bytes);
         return;
     }
     if (D <= 128 && paired) {
         const int lhw = hw == 4 ? 2 : (hw == 2 ? 1 : 0);
         hipLaunchKernelGGL((prefill4_kernel<T, D>), dim3(per_xcd * 8), dim3(512), 0, st,
                            (const uint16_t *)q, (const char *)kc, (const char *)vc, kvs, S, sp,
-                           nh, kv_mul, lhw, ng, np, qs, out, pgs);
+                           nh, kv_mul, lhw, ng, np, qs, out, pgs, KeySplit{});
         return;
     }
     hipLaunchKernelGGL((prefill2_kernel<T, D>), dim3(per_xcd * 8), dim3(512), 0, st,
@@ -1199,8 +1279,8 @@ void PrefillLaunch<T, D, true>::run(const void *q, const void *kc, const void *v
 template <class T, int D>
 static int launch_prefill(const void *q, const void *kc, const void *vc, int64_t kvs, int S,
                           int sp, int win, int nh, int kv_mul, float qs, float *out,
-                          hipStream_t st) {
-    PrefillLaunch<T, D>::run(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st);
+                          hipStream_t st, KvPages pgs, Scratch ws) {
+    PrefillLaunch<T, D>::run(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st, pgs, ws);
     return check_hip(hipGetLastError(), "prefill launch");
 }
 
@@ -1223,10 +1303,11 @@ static int launch_prefill(const void *q, const void *kc, const void *vc, int64_t
 // query heads of one kv head (hw = the largest power of two dividing kv_mul,
 // at most 4) times 4/hw consecutive 32-row blocks: one "unit" of
 // UR = 128/hw rows; wave w takes head hw0 + w % hw and rows (w / hw) * 32 ..
-// +31 of the unit.  Units are taken in causal pairs, A = p and B = NU-1-p,
-// so every workgroup attends about the same number of keys.  The workgroup
-// walks the key tiles of A, then those of B, and each tile is loaded and
-// converted once for all 4 waves:
+// +31 of the unit.  A unit, or one part of its key tiles (KeySplit, max_parts
+// at most), is one workgroup; up to two fit a CU.  (Causal pairs of units per
+// workgroup, which balance the keys, were slower at every size: 777 rows of
+// 32/8 heads x 64 33.9 against 29.6 us, 4096 rows 216 against 211, 61 rows at 700
+// 52 against 27.)  Each tile is loaded and converted once for all 4 waves:
 //  * all 256 threads load the tile's f32 K and V rows (16-byte chunks, two
 //    full rows per wave instruction) into registers, NRAW tiles ahead;
 //  * they convert them into an LDS stage, a chunk at a time between the
@@ -1236,16 +1317,15 @@ static int launch_prefill(const void *q, const void *kc, const void *vc, int64_t
 //    banks), V as f16 rows in the kv_swz layout the transposing reads expect;
 //  * three stages: a stage is rewritten two tiles after it was read, so one
 //    barrier per tile orders every rewrite after all reads of it.
-// Each wave keeps (m, l, O) of its 32 rows over the whole key range, so it
-// writes its rows of A (normalised) when A's tiles end and starts B afresh;
-// no partials are merged.  A 32-row block of one head per workgroup with the
-// 4 waves splitting its keys (each wave streaming and converting its own
-// tiles) took 1.6x as long at the cfg3 shape.
+// Each wave keeps (m, l, O) of its 32 rows over the whole key range.  A 32-row
+// block of one head per workgroup with the 4 waves splitting its keys (each
+// wave streaming and converting its own tiles) took 1.6x as long at 2048 rows
+// of 32/8 heads x 128.
 template <int D, int NRAW = 2>
 __global__ __launch_bounds__(256, 1) void prefill_f32_kernel(
     const float *__restrict__ q, const float *__restrict__ kc, const float *__restrict__ vc,
     int64_t kv_stride, int S, int start_pos, int window, int n_head, int kv_mul, int hw,
-    int n_units, int n_pairs, float qscale, float *__restrict__ out, KvPages pgs) {
+    int n_units, int max_parts, float qscale, float *__restrict__ out, KvPages pgs, KeySplit sp) {
     constexpr int BN = 32, RB = D * 2, KP = D * 2 + 16;  // keys per tile; f16/bf16 row bytes; K pitch
     constexpr int NKS = D / 16, NDT = D / 32;
     constexpr int FPR = D / 4;              // 16-byte f32 chunks per cache row
@@ -1256,41 +1336,30 @@ __global__ __launch_bounds__(256, 1) void prefill_f32_kernel(
     constexpr float kLazy = 8.0f;
     static_assert(D == 64 || D == 128, "f32 prefill serves head_dim 64 and 128");
     auto swz = [](int r) { return kv_swz<D>(r); };
-    constexpr int QB = 2 * NKS * 64 * 16;   // one wave's unit-B Q operands (hi, lo)
     __shared__ __attribute__((aligned(1024))) char lds[NSTG * STAGE];
-    __shared__ __attribute__((aligned(16))) char qb_lds[4 * QB];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 31, h2 = lane >> 5;
-    // Task: (head group, pair), pairs of one head group on one XCD's L2.
+    // Task: (head group, unit, part), a head group's on one XCD's L2.
     const int n_hg = n_head / hw;
-    const int total = n_hg * n_pairs;
+    const int per_hg = n_units * max_parts;
+    const int total = n_hg * per_hg;
     const int per_xcd = (total + 7) / 8;
     const int tsk = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (tsk >= total) return;
-    const int hg = tsk / n_pairs, pr = tsk % n_pairs;
+    const int hg = tsk / per_hg, pr = tsk % per_hg;
+    const int kpart = pr % max_parts, u = n_units - 1 - pr / max_parts;  // longest first
     const int rbw = 4 / hw, UR = 32 * rbw;
     const int head = hg * hw + wave % hw, kvh = head / kv_mul;
     const int roff = (wave / hw) * 32;  // this wave's rows within a unit
     const int64_t q_dim = (int64_t)n_head * D;
     const int kv_len = start_pos + S;
-    const int ua = pr, ub = n_units - 1 - pr;  // ub == ua: the middle unit alone
-
-    // Key tiles [first, end) of a unit: from the window start of its first
-    // row to the causal end of its last row.
-    auto tiles = [&](int u, int &t0, int &t1) {
-        const int r0 = u * UR;
-        const int hi = start_pos + min(r0 + UR, S);
-        int lo = 0;
-        if (window > 0) lo = max(0, start_pos + r0 + 1 - window);
-        t0 = lo / BN;
-        t1 = (hi + BN - 1) / BN;
-    };
-    int a0, a1, b0 = 0, b1 = 0;
-    tiles(ua, a0, a1);
-    if (ub != ua) tiles(ub, b0, b1);
-    const int na = a1 - a0, nsteps = na + (b1 - b0);
+    int a0, a1;
+    unit_tiles(u, UR, S, start_pos, window, BN, a0, a1);
+    const int parts = part_tiles(sp, kpart, a0, a1);
+    if (kpart >= parts) return;
+    const int nsteps = a1 - a0;
 
     const int rbg = (int)(kv_stride * 4);
     const int range = (kv_len - 1) * rbg + D * 4;
@@ -1300,7 +1369,7 @@ __global__ __launch_bounds__(256, 1) void prefill_f32_kernel(
         __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(vc + (int64_t)kvh * D), 0, range, kRsrcWord3);
     // Step j's tile; steps past the end address past the buffer (zeros,
     // no memory access), so every step issues the same requests.
-    auto tile_of = [&](int j) { return j < na ? a0 + j : b0 + (j - na); };
+    auto tile_of = [&](int j) { return a0 + j; };
     auto step_off = [&](int j) {
         return __builtin_amdgcn_readfirstlane(j < nsteps ? tile_of(j) * BN * rbg : range);
     };
@@ -1360,10 +1429,8 @@ __global__ __launch_bounds__(256, 1) void prefill_f32_kernel(
             va_addr[dt][h] = 2 * KARR + R * RB + (((e0 >> 3) ^ swz(R)) * 16) + (e0 & 7) * 2;
         }
 
-    // Per-unit state of this wave: Q as hi/lo B operands (unit B's are
-    // prepared at the start and parked in LDS, lane-major), row, (m, l, O).
+    // This wave's Q as hi/lo B operands, row, (m, l, O).
     u32x4 qh[NKS], ql[NKS];
-    const uint32_t qbw = lds_addr(qb_lds) + wave * QB + lane * 16;
     auto load_q = [&](int u, u32x4(&h)[NKS], u32x4(&l)[NKS]) {
         const int row = u * UR + roff + c;
         const bool ok = row < S;
@@ -1395,6 +1462,19 @@ __global__ __launch_bounds__(256, 1) void prefill_f32_kernel(
     auto end_unit = [&]() {
         const float l_tot = l_part + xor32(l_part);
         const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
+        if (parts > 1) {  // left for the merge
+            if (qrow >= S) return;
+            const int64_t prow = (int64_t)kpart * S + qrow;
+            float *op = sp.o + prow * q_dim + (int64_t)head * D + h2 * 4;
+#pragma unroll
+            for (int dt = 0; dt < NDT; dt++)
+#pragma unroll
+                for (int g = 0; g < 4; g++)
+                    *(f32x4 *)(op + dt * 32 + g * 8) = f32x4{oacc[dt][g * 4], oacc[dt][g * 4 + 1],
+                                                             oacc[dt][g * 4 + 2], oacc[dt][g * 4 + 3]};
+            if (h2 == 0) sp.ml[prow * n_head + head] = float2{m_run, l_tot};
+            return;
+        }
         if (qrow < S) {
             float *op = out + (int64_t)qrow * q_dim + (int64_t)head * D + h2 * 4;
 #pragma unroll
@@ -1508,16 +1588,8 @@ __global__ __launch_bounds__(256, 1) void prefill_f32_kernel(
     static_assert(NRAW == 2, "the step loop is unrolled for two raw register sets");
     issue(kraw[0], vraw[0], 0);
     issue(kraw[1], vraw[1], 1);
-    if (ub != ua) {
-        load_q(ub, qh, ql);
-#pragma unroll
-        for (int s = 0; s < NKS; s++) {
-            lds_write_b128(qbw + (2 * s) * 1024, qh[s]);
-            lds_write_b128(qbw + (2 * s + 1) * 1024, ql[s]);
-        }
-    }
-    load_q(ua, qh, ql);
-    begin_unit(ua);
+    load_q(u, qh, ql);
+    begin_unit(u);
     convert(kraw[0], vraw[0], 0);
     issue(kraw[0], vraw[0], 2);
     lds_wait_any();
@@ -1530,18 +1602,6 @@ __global__ __launch_bounds__(256, 1) void prefill_f32_kernel(
     auto step = [&](auto rs, int j, bool live) {
         constexpr int R = decltype(rs)::value;  // raw set of tile j+1
         const int nstg = stg == NSTG - 1 ? 0 : stg + 1;
-        if (live && j == na) {
-            end_unit();
-            begin_unit(ub);
-#pragma unroll
-            for (int s = 0; s < NKS; s++) {
-                qh[s] = lds_read_b128(qbw + (2 * s) * 1024);
-                ql[s] = lds_read_b128(qbw + (2 * s + 1) * 1024);
-            }
-            lds_wait_any();
-#pragma unroll
-            for (int s = 0; s < NKS; s++) { tie(qh[s]); tie(ql[s]); }
-        }
         if (live) compute(j, stg, [&](int i) { convert1(kraw[R], vraw[R], nstg, i); });
         else convert(kraw[R], vraw[R], nstg);
         issue(kraw[R], vraw[R], j + 3);
@@ -1566,39 +1626,66 @@ __global__ __launch_bounds__(256, 1) void prefill_f32_kernel(
 template <int D>
 static int launch_prefill_f32(const void *q, const void *kc, const void *vc, int64_t kvs, int S,
                               int sp, int win, int nh, int kv_mul, float qs, float *out,
-                              hipStream_t st, KvPages pgs = KvPages{}) {
+                              hipStream_t st, KvPages pgs, Scratch ws) {
     int hw = 1;
     while (hw < 4 && kv_mul % (hw * 2) == 0) hw *= 2;
     const int n_units = (S + 128 / hw - 1) / (128 / hw);
-    const int n_pairs = (n_units + 1) / 2;
-    const int total = nh / hw * n_pairs;
-    const int per_xcd = (total + 7) / 8;
+    SplitPlan pl = prefill_f32_split(S, sp, win, nh, kv_mul, D);
+    if (!ws.p || ws.bytes < pl.bytes) pl = SplitPlan{INT_MAX / 2, 1, 0, 0};
+    const KeySplit ksp = split_at(pl, 32, ws.p);
+    const int per_xcd = (nh / hw * n_units * pl.parts + 7) / 8;
     hipLaunchKernelGGL((prefill_f32_kernel<D>), dim3(per_xcd * 8), dim3(256), 0, st,
                        (const float *)q, (const float *)kc, (const float *)vc, kvs, S, sp, win,
-                       nh, kv_mul, hw, n_units, n_pairs, qs, out, pgs);
+                       nh, kv_mul, hw, n_units, pl.parts, qs, out, pgs, ksp);
+    if (pl.parts > 1) return launch_prefill_merge(D, ksp, 128 / hw, S, sp, win, nh, out, st);
     return check_hip(hipGetLastError(), "prefill (f32) launch");
 }
 
 template <class T>
 static int dispatch_prefill(int D, const void *q, const void *kc, const void *vc, int64_t kvs,
                             int S, int sp, int win, int nh, int kv_mul, float qs, float *out,
-                            hipStream_t st) {
+                            hipStream_t st, KvPages pgs, Scratch ws) {
     switch (D) {
-        case 64: return launch_prefill<T, 64>(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st);
-        case 128: return launch_prefill<T, 128>(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st);
-        case 256: return launch_prefill<T, 256>(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st);
+        case 64: return launch_prefill<T, 64>(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st, pgs, ws);
+        case 128: return launch_prefill<T, 128>(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st, pgs, ws);
+        case 256: return launch_prefill<T, 256>(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st, pgs, ws);
         default: return set_error(ULLM_HIP_E_UNSUPPORTED, "prefill: head_dim %d not in {64,128,256}", D);
     }
+}
+
+// One prefill call, arguments checked; pgs.tab == nullptr: the contiguous cache.
+static int run_prefill(int dtype, const void *q, const void *kc, const void *vc, int64_t kvs, int S,
+                       int sp, int win, int nh, int kv_mul, int D, float qs, float *out,
+                       hipStream_t st, KvPages pgs, Scratch ws) {
+    if (dtype == ULLM_DT_F32) {
+        // head_dim 128: prefill16_kernel's f32 mode (faster at every measured
+        // prompt, 128..4096 rows); ULLM_HIP_PREFILL_F32=4 keeps
+        // prefill_f32_kernel for a contiguous cache.
+        static const int ef = env_override("ULLM_HIP_PREFILL_F32");
+        if (D == 256)
+            return launch_prefill16(ULLM_DT_F32, q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st,
+                                    pgs, ws.p, ws.bytes);
+        if (D == 128 && (ef != 4 || pgs.tab))
+            return launch_prefill16_128(ULLM_DT_F32, q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st,
+                                        pgs, ws.p, ws.bytes);
+        if (D == 64)
+            return launch_prefill_f32<64>(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st, pgs, ws);
+        return launch_prefill_f32<128>(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st, pgs, ws);
+    }
+    if (dtype == ULLM_DT_BF16)
+        return dispatch_prefill<BF16>(D, q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st, pgs, ws);
+    return dispatch_prefill<F16>(D, q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st, pgs, ws);
 }
 
 }  // namespace ullm
 
 using namespace ullm;
 
-extern "C" int ullm_hip_attn_prefill(const void *q, const void *k_cache, const void *v_cache,
-                                     int dtype, int64_t kv_stride, int S, int start_pos,
-                                     int window, int n_head, int n_kv_head, int head_dim,
-                                     float scale, float *out, void *stream) {
+extern "C" int ullm_hip_attn_prefill_ws(const void *q, const void *k_cache, const void *v_cache,
+                                        int dtype, int64_t kv_stride, int S, int start_pos,
+                                        int window, int n_head, int n_kv_head, int head_dim,
+                                        float scale, float *out, void *workspace,
+                                        size_t workspace_bytes, void *stream) {
     if (!dtype_ok(dtype))
         return set_error(ULLM_HIP_E_UNSUPPORTED, "prefill: dtype %d", dtype);
     if (n_head < 1 || n_kv_head < 1 || n_head % n_kv_head || S < 0 || start_pos < 0)
@@ -1617,34 +1704,26 @@ extern "C" int ullm_hip_attn_prefill(const void *q, const void *k_cache, const v
         return set_error(ULLM_HIP_E_INVALID, "prefill: null tensor pointer");
     if (((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)out) & 15)
         return set_error(ULLM_HIP_E_INVALID, "prefill: tensors must be 16-byte aligned");
-    const float qs = scale * kLog2e;
-    const int kv_mul = n_head / n_kv_head;
-    hipStream_t st = (hipStream_t)stream;
-    if (dtype == ULLM_DT_F32) {
-        // head_dim 128: prefill16_kernel's f32 mode (faster at every measured
-        // prompt, 128..4096 rows); ULLM_HIP_PREFILL_F32=4 keeps prefill_f32_kernel.
-        static const int ef = env_override("ULLM_HIP_PREFILL_F32");
-        if (head_dim == 256)
-            return launch_prefill16(ULLM_DT_F32, q, k_cache, v_cache, kv_stride, S, start_pos, window,
-                                    n_head, kv_mul, qs, out, st, KvPages{});
-        if (head_dim == 128 && ef != 4)
-            return launch_prefill16_128(ULLM_DT_F32, q, k_cache, v_cache, kv_stride, S, start_pos, window,
-                                        n_head, kv_mul, qs, out, st, KvPages{});
-        if (head_dim == 64)
-            return launch_prefill_f32<64>(q, k_cache, v_cache, kv_stride, S, start_pos, window, n_head, kv_mul, qs, out, st);
-        return launch_prefill_f32<128>(q, k_cache, v_cache, kv_stride, S, start_pos, window, n_head, kv_mul, qs, out, st);
-    }
-    if (dtype == ULLM_DT_BF16)
-        return dispatch_prefill<BF16>(head_dim, q, k_cache, v_cache, kv_stride, S, start_pos, window, n_head, kv_mul, qs, out, st);
-    return dispatch_prefill<F16>(head_dim, q, k_cache, v_cache, kv_stride, S, start_pos, window, n_head, kv_mul, qs, out, st);
+    return run_prefill(dtype, q, k_cache, v_cache, kv_stride, S, start_pos, window, n_head,
+                       n_head / n_kv_head, head_dim, scale * kLog2e, out, (hipStream_t)stream, KvPages{},
+                       Scratch{workspace, workspace_bytes});
 }
 
-extern "C" int ullm_hip_attn_prefill_paged(const void *q, const void *k_pages, const void *v_pages,
-                                           int dtype, int64_t kv_stride, int page_size,
-                                           int n_pages, const int32_t *block_table,
-                                           int table_len, int S, int start_pos, int window,
-                                           int n_head, int n_kv_head, int head_dim, float scale,
-                                           float *out, void *stream) {
+extern "C" int ullm_hip_attn_prefill(const void *q, const void *k_cache, const void *v_cache,
+                                     int dtype, int64_t kv_stride, int S, int start_pos,
+                                     int window, int n_head, int n_kv_head, int head_dim,
+                                     float scale, float *out, void *stream) {
+    return ullm_hip_attn_prefill_ws(q, k_cache, v_cache, dtype, kv_stride, S, start_pos, window, n_head,
+                                    n_kv_head, head_dim, scale, out, nullptr, 0, stream);
+}
+
+extern "C" int ullm_hip_attn_prefill_paged_ws(const void *q, const void *k_pages, const void *v_pages,
+                                              int dtype, int64_t kv_stride, int page_size,
+                                              int n_pages, const int32_t *block_table,
+                                              int table_len, int S, int start_pos, int window,
+                                              int n_head, int n_kv_head, int head_dim, float scale,
+                                              float *out, void *workspace, size_t workspace_bytes,
+                                              void *stream) {
     if (!dtype_ok(dtype))
         return set_error(ULLM_HIP_E_UNSUPPORTED, "prefill_paged: dtype %d", dtype);
     if (head_dim != 64 && head_dim != 128 && head_dim != 256)
@@ -1673,28 +1752,33 @@ extern "C" int ullm_hip_attn_prefill_paged(const void *q, const void *k_pages, c
     if (((uintptr_t)q | (uintptr_t)k_pages | (uintptr_t)v_pages | (uintptr_t)out) & 15)
         return set_error(ULLM_HIP_E_INVALID, "prefill_paged: tensors must be 16-byte aligned");
     const KvPages pgs{block_table, table_len, __builtin_ctz(page_size), n_pages};
-    const float qs = scale * kLog2e;
-    const int kv_mul = n_head / n_kv_head;
-    hipStream_t st = (hipStream_t)stream;
-    if (dtype == ULLM_DT_F32) {  // f32 pages: prefill16_kernel's f32 mode, prefill_f32_kernel at 64
-        if (head_dim == 64)
-            return launch_prefill_f32<64>(q, k_pages, v_pages, kv_stride, S, start_pos, window, n_head,
-                                          kv_mul, qs, out, st, pgs);
-        if (head_dim == 256)
-            return launch_prefill16(ULLM_DT_F32, q, k_pages, v_pages, kv_stride, S, start_pos, window,
-                                    n_head, kv_mul, qs, out, st, pgs);
-        return launch_prefill16_128(ULLM_DT_F32, q, k_pages, v_pages, kv_stride, S, start_pos, window,
-                                    n_head, kv_mul, qs, out, st, pgs);
-    }
-    if (dtype == ULLM_DT_BF16) {
-        if (head_dim == 64) PrefillLaunch<BF16, 64>::run(q, k_pages, v_pages, kv_stride, S, start_pos, window, n_head, kv_mul, qs, out, st, pgs);
-        else if (head_dim == 128) PrefillLaunch<BF16, 128>::run(q, k_pages, v_pages, kv_stride, S, start_pos, window, n_head, kv_mul, qs, out, st, pgs);
-        else PrefillLaunch<BF16, 256>::run(q, k_pages, v_pages, kv_stride, S, start_pos, window, n_head, kv_mul, qs, out, st, pgs);
-    } else {
-        if (head_dim == 64) PrefillLaunch<F16, 64>::run(q, k_pages, v_pages, kv_stride, S, start_pos, window, n_head, kv_mul, qs, out, st, pgs);
-        else if (head_dim == 128) PrefillLaunch<F16, 128>::run(q, k_pages, v_pages, kv_stride, S, start_pos, window, n_head, kv_mul, qs, out, st, pgs);
-        else PrefillLaunch<F16, 256>::run(q, k_pages, v_pages, kv_stride, S, start_pos, window, n_head, kv_mul, qs, out, st, pgs);
-    }
-    return check_hip(hipGetLastError(), "prefill_paged launch");
+    return run_prefill(dtype, q, k_pages, v_pages, kv_stride, S, start_pos, window, n_head,
+                       n_head / n_kv_head, head_dim, scale * kLog2e, out, (hipStream_t)stream, pgs,
+                       Scratch{workspace, workspace_bytes});
 }
 
+extern "C" int ullm_hip_attn_prefill_paged(const void *q, const void *k_pages, const void *v_pages,
+                                           int dtype, int64_t kv_stride, int page_size,
+                                           int n_pages, const int32_t *block_table,
+                                           int table_len, int S, int start_pos, int window,
+                                           int n_head, int n_kv_head, int head_dim, float scale,
+                                           float *out, void *stream) {
+    return ullm_hip_attn_prefill_paged_ws(q, k_pages, v_pages, dtype, kv_stride, page_size, n_pages,
+                                          block_table, table_len, S, start_pos, window, n_head, n_kv_head,
+                                          head_dim, scale, out, nullptr, 0, stream);
+}
+
+extern "C" size_t ullm_hip_prefill_workspace_bytes(int dtype, int S, int start_pos, int window,
+                                                   int n_head, int n_kv_head, int head_dim) {
+    if (!dtype_ok(dtype) || S < 1 || start_pos < 0 || n_head < 1 || n_kv_head < 1 || n_head % n_kv_head ||
+        (int64_t)start_pos + S > 0x7fffffff) return 0;
+    const int kv_mul = n_head / n_kv_head;
+    SplitPlan pl{0, 1, 0, 0};
+    if (head_dim == 256 || (head_dim == 128 && dtype == ULLM_DT_F32))
+        pl = prefill16_split(dtype, S, start_pos, window, n_head, kv_mul, head_dim);
+    else if (head_dim == 64 && dtype == ULLM_DT_F32)
+        pl = prefill_f32_split(S, start_pos, window, n_head, kv_mul, 64);
+    else if ((head_dim == 64 || head_dim == 128) && !(window > 0 && window < start_pos + S))
+        pl = prefill4_split(S, start_pos, n_head, kv_mul, head_dim);
+    return pl.bytes;
+}

@@ -77,12 +77,12 @@ constexpr int p16_stages() {
     return st > 4 ? 4 : st;
 }
 
-template <class T, int KS, int DS, int D = 256, int OCC = 1,
+template <class T, int KS, int DS, int D = 256, int OCC = 1, bool SPLIT = false,
           int NSTG = p16_stages<KS, DS, D, OCC, T::bytes>()>
 __global__ __launch_bounds__(512, OCC) void prefill16_kernel(
     const uint16_t *__restrict__ q, const char *__restrict__ kc, const char *__restrict__ vc,
     int64_t kv_stride, int S, int start_pos, int window, int n_head, int kv_mul, int hw,
-    int n_hg, int n_units, float qscale, float *__restrict__ out, KvPages pgs) {
+    int n_hg, int n_units, float qscale, float *__restrict__ out, KvPages pgs, KeySplit sp) {
     // DS = 2: the workgroup computes the full Q.K and softmax of its rows but
     // P.V and the output for one half of the 256 value columns only; its V
     // tiles hold that half (256-byte rows).
@@ -125,7 +125,9 @@ __global__ __launch_bounds__(512, OCC) void prefill16_kernel(
 
     const int dh = DS == 1 ? 0 : (int)(blockIdx.x % DS);  // value half
     const int bx = (int)(blockIdx.x / DS);
-    const int hg = bx % n_hg, u = n_units - 1 - bx / n_hg;
+    const int hg = bx % n_hg, item = bx / n_hg;
+    const int part = SPLIT ? item / n_units : 0;
+    const int u = n_units - 1 - (SPLIT ? item - part * n_units : item);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ks = wave / NWS, ws = wave % NWS;  // key stream, wave within the stream
@@ -138,15 +140,12 @@ __global__ __launch_bounds__(512, OCC) void prefill16_kernel(
     const int64_t q_dim = (int64_t)n_head * D;
     const int kv_len = start_pos + S;
 
-    // Key tiles [t0, t1) of the unit: the window start of its first row to
-    // the causal end of its last; stream ks takes [t0 + ks*nsteps, ..).
-    int t0, t1;
-    {
-        const int hi = start_pos + min(u * UR + UR, S);
-        int lo = 0;
-        if (window > 0) lo = max(start_pos + u * UR + 1 - window, 0);
-        t0 = lo / BN;
-        t1 = (hi + BN - 1) / BN;
+    // This workgroup's key tiles [t0, t1); stream ks takes [t0 + ks*nsteps, ..).
+    int t0, t1, parts = 1;
+    unit_tiles(u, UR, S, start_pos, window, BN, t0, t1);
+    if constexpr (SPLIT) {
+        parts = part_tiles(sp, part, t0, t1);
+        if (part >= parts) return;
     }
     const int nsteps = (t1 - t0 + KS - 1) / KS;
     const int tbase = t0 + ks * nsteps;  // this stream's first tile
@@ -501,6 +500,16 @@ __global__ __launch_bounds__(512, OCC) void prefill16_kernel(
             oacc[dt] = oacc[dt] * a0 + __builtin_bit_cast(f32x4, o1[dt]) * a1;
         }
     }
+    if constexpr (SPLIT) {
+        if (parts > 1) {  // workgroup-uniform
+            if (qrow >= S) return;
+            float *op = sp.o + ((int64_t)part * S + qrow) * q_dim + (int64_t)head * D + dh * (D / DS) + 4 * g;
+#pragma unroll
+            for (int dt = 0; dt < NDT; dt++) *(f32x4 *)(op + dt * 16) = oacc[dt];
+            if (g == 0 && dh == 0) sp.ml[((int64_t)part * S + qrow) * n_head + head] = float2{m_run, l_tot};
+            return;
+        }
+    }
     if (qrow < S) {
         const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
         float *op = out + (int64_t)qrow * q_dim + (int64_t)head * D + dh * (D / DS) + 4 * g;
@@ -510,15 +519,63 @@ __global__ __launch_bounds__(512, OCC) void prefill16_kernel(
     }
 }
 
+// Rows of split units: out = sum_p 2^(m_p - M) O_p / sum_p 2^(m_p - M) l_p over
+// the unit's parts (the parts of one row are in flight together).  Four
+// columns per thread; streams the parts once.
+template <int D>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(KeySplit sp, int UR, int S, int start_pos,
+                                                              int window, int n_head,
+                                                              float *__restrict__ out) {
+    const int row = blockIdx.x, col = (blockIdx.y * 256 + threadIdx.x) * 4;
+    int t0, t1;
+    unit_tiles(row / UR, UR, S, start_pos, window, sp.tile, t0, t1);
+    const int parts = (t1 - t0 + sp.chunk - 1) / sp.chunk;
+    if (parts < 2 || col >= n_head * D) return;
+    const float2 *ml = sp.ml + (int64_t)row * n_head + col / D;
+    const float *o = sp.o + (int64_t)row * n_head * D + col;
+    const int64_t mls = (int64_t)S * n_head, os = mls * D;
+    float M = -INFINITY, L = 0.f;
+    f32x4 acc = f32x4{};
+    constexpr int B = 8;  // parts loaded together
+    for (int p0 = 0; p0 < parts; p0 += B) {
+        float2 v[B];
+        f32x4 x[B];
+#pragma unroll
+        for (int i = 0; i < B; i++) {
+            const bool in = p0 + i < parts;
+            v[i] = in ? ml[(p0 + i) * mls] : float2{-INFINITY, 0.f};
+            x[i] = in ? *(const f32x4 *)(o + (p0 + i) * os) : f32x4{};
+        }
+        float m = M;
+#pragma unroll
+        for (int i = 0; i < B; i++) m = fmaxf(m, v[i].x);
+        const float mu = m == -INFINITY ? 0.f : m;
+        const float c = __builtin_amdgcn_exp2f(M - mu);
+        L *= c;
+        acc *= c;
+#pragma unroll
+        for (int i = 0; i < B; i++) {
+            const float a = __builtin_amdgcn_exp2f(v[i].x - mu);
+            L += v[i].y * a;
+            acc += x[i] * a;
+        }
+        M = m;
+    }
+    *(f32x4 *)(out + (int64_t)row * n_head * D + col) = acc * (L > 0.f ? 1.0f / L : 0.f);
+}
+
 static int p16_hw(int kv_mul, int nws) {
     int hw = 1;
     while (hw < nws && hw < 4 && kv_mul % (hw * 2) == 0) hw *= 2;
     return hw;
 }
 
-// Key streams and value-column split for a prompt.  Two key streams when
-// whole units would leave CUs idle, or fill the chip exactly with causal
-// (window-free) chains, whose longest unit then sets the time; the value
+// Key streams and value-column split for a prompt.  Two key streams up to one
+// causal (window-free) unit per CU, the longest setting the time; with a
+// binding window, where all units are alike, up to half that, so that the
+// twice as many workgroups still run in one round (8/4 heads x 256, f16, window
+// 1024, KS1 / KS2: 2000 rows 44.2 / 38.5, 2500 rows (160 units) 45.5 / 49.3, 4001
+// rows 53.0 / 77.9; causal 4001 rows 135 / 126); the value
 // split on top when the workgroups still fit one per CU.  Measured at 8/4
 // heads, f16 (us; KS/DS): S=1024 KS2/DS2 23.9, KS2/DS1 27.1, KS1/DS2 34.5;
 // S=2048 KS2/DS1 51.5, KS2/DS2 53.2; S=4096 causal KS2/DS1 122-130, KS1/DS1
@@ -531,7 +588,7 @@ static void prefill16_plan(int S, int start_pos, int window, int n_head, int kv_
     const int hw = p16_hw(kv_mul, 8);
     const int64_t grid1 = (int64_t)((S + 128 / hw - 1) / (128 / hw)) * (n_head / hw);
     const bool binding = window > 0 && window < start_pos + S;
-    ks = grid1 < 256 || (grid1 == 256 && !binding) ? 2 : 1;
+    ks = grid1 <= (binding ? 128 : 256) ? 2 : 1;
     if (eks == 1 || eks == 2) ks = eks;
     const int hw2 = p16_hw(kv_mul, 8 / ks), ur = 16 * (8 / ks) / hw2;
     const int64_t grid = (int64_t)((S + ur - 1) / ur) * (n_head / hw2);
@@ -539,9 +596,73 @@ static void prefill16_plan(int S, int start_pos, int window, int n_head, int kv_
     if (eds == 1 || eds == 2) ds = eds;
 }
 
+int launch_prefill_merge(int D, KeySplit sp, int UR, int S, int start_pos, int window, int n_head,
+                         float *out, hipStream_t st) {
+    const dim3 g((unsigned)S, (unsigned)((n_head * D + 1023) / 1024)), b(256);
+    if (D == 64) hipLaunchKernelGGL((prefill_merge_kernel<64>), g, b, 0, st, sp, UR, S, start_pos, window, n_head, out);
+    else if (D == 128) hipLaunchKernelGGL((prefill_merge_kernel<128>), g, b, 0, st, sp, UR, S, start_pos, window, n_head, out);
+    else hipLaunchKernelGGL((prefill_merge_kernel<256>), g, b, 0, st, sp, UR, S, start_pos, window, n_head, out);
+    return check_hip(hipGetLastError(), "prefill merge launch");
+}
+
+double prefill16_us(int dtype, int S, int start_pos, int window, int n_head, int kv_mul, int D) {
+    int KS, DS;
+    prefill16_plan(S, start_pos, window, n_head, kv_mul, KS, DS);
+    if (D == 128) DS = 1;
+    if (dtype == ULLM_DT_F32 && D == 256) KS = 1, DS = 2;
+    const int hw = p16_hw(kv_mul, 8 / KS), UR = 16 * (8 / KS) / hw;
+    const UnitLoad u = unit_load(S, UR, n_head / hw, start_pos, window, 32);
+    // Per 32-key step (us): one key stream; two streams take two tiles a step.
+    // 8/4 heads x 256, f16: 1500 rows KS1 53.5 us for 47 steps on 94 CUs, KS2
+    // 43.0 for 24; 4001 rows, window 1024, KS1 53.0 for 34 on 252 CUs.  32/8 x
+    // 128: 512 rows at 7680, bf16, KS2 135 for 128 steps; 512 rows at 4000, f32,
+    // KS2 147 for 71.
+    const bool f32 = dtype == ULLM_DT_F32;
+    const PrefillCost c = D == 256 ? (f32 ? PrefillCost{2.0, 2.1, 6.} : KS == 1 ? PrefillCost{1.03, 1.4, 6.}
+                                          : DS == 2 ? PrefillCost{.62, .68, 6.} : PrefillCost{.72, .85, 6.})
+                                   : (f32 ? (KS == 1 ? PrefillCost{1.2, 1.4, 6.} : PrefillCost{1.0, 1.0, 6.})
+                                          : (KS == 1 ? PrefillCost{.9, .95, 5.} : PrefillCost{.46, .5, 5.}));
+    return prefill_us(c, u.n * DS, u.longest, u.n * DS * u.avg);
+}
+
+SplitPlan prefill16_split(int dtype, int S, int start_pos, int window, int n_head, int kv_mul, int D) {
+    const int hw = p16_hw(kv_mul, 8);
+    UnitLoad u = unit_load(S, 128 / hw, n_head / hw, start_pos, window, 32);
+    // One key stream (f32 at head_dim 256: two workgroups per unit).
+    const PrefillCost c = dtype == ULLM_DT_F32 ? (D == 256 ? PrefillCost{2.0, 2.1, 6.} : PrefillCost{1.2, 1.4, 6.})
+                                               : (D == 256 ? PrefillCost{1.03, 1.1, 6.} : PrefillCost{.9, .95, 5.});
+    if (dtype == ULLM_DT_F32 && D == 256) u.n *= 2;
+    return choose_split(c, u, prefill16_us(dtype, S, start_pos, window, n_head, kv_mul, D), S, n_head, D);
+}
+
+template <int D>
+static int launch_prefill16_split(int dtype, const void *q, const void *kc, const void *vc, int64_t kvs,
+                                  int S, int start_pos, int window, int n_head, int kv_mul, float qs,
+                                  float *out, hipStream_t st, KvPages pgs, const SplitPlan &pl, void *ws) {
+    const int hw = p16_hw(kv_mul, 8), UR = 128 / hw;
+    const int n_units = (S + UR - 1) / UR, n_hg = n_head / hw;
+    const KeySplit sp = split_at(pl, 32, ws);
+    auto go = [&](auto kern, int ds) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)(n_units * n_hg * pl.parts * ds)), dim3(512), 0, st,
+                           (const uint16_t *)q, (const char *)kc, (const char *)vc, kvs, S, start_pos,
+                           window, n_head, kv_mul, hw, n_hg, n_units, qs, out, pgs, sp);
+    };
+    constexpr int FDS = D == 256 ? 2 : 1;  // f32 tiles at head_dim 256: value columns split (LDS)
+    if (dtype == ULLM_DT_F32) go(prefill16_kernel<F32, 1, FDS, D, 1, true>, FDS);
+    if constexpr (D == 256) {  // 16-bit caches at head_dim 128 split on prefill4_kernel
+        if (dtype == ULLM_DT_BF16) go(prefill16_kernel<BF16, 1, 1, D, 1, true>, 1);
+        if (dtype == ULLM_DT_F16) go(prefill16_kernel<F16, 1, 1, D, 1, true>, 1);
+    }
+    return launch_prefill_merge(D, sp, UR, S, start_pos, window, n_head, out, st);
+}
+
 int launch_prefill16(int dtype, const void *q, const void *kc, const void *vc, int64_t kvs, int S,
                      int start_pos, int window, int n_head, int kv_mul, float qs, float *out,
-                     hipStream_t st, KvPages pgs) {
+                     hipStream_t st, KvPages pgs, void *ws, size_t ws_bytes) {
+    const SplitPlan pl = prefill16_split(dtype, S, start_pos, window, n_head, kv_mul, 256);
+    if (pl.parts > 1 && ws && ws_bytes >= pl.bytes)
+        return launch_prefill16_split<256>(dtype, q, kc, vc, kvs, S, start_pos, window, n_head, kv_mul, qs,
+                                           out, st, pgs, pl, ws);
     int KS, DS;
     prefill16_plan(S, start_pos, window, n_head, kv_mul, KS, DS);
     const int hw = p16_hw(kv_mul, 8 / KS), UR = 16 * (8 / KS) / hw;
@@ -550,7 +671,7 @@ int launch_prefill16(int dtype, const void *q, const void *kc, const void *vc, i
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, grid, dim3(512), 0, st, (const uint16_t *)q, (const char *)kc,
                            (const char *)vc, kvs, S, start_pos, window, n_head, kv_mul, hw, n_hg,
-                           n_units, qs, out, pgs);
+                           n_units, qs, out, pgs, KeySplit{});
     };
     auto pick = [&](auto t) {
         using T = decltype(t);
@@ -567,7 +688,7 @@ int launch_prefill16(int dtype, const void *q, const void *kc, const void *vc, i
         const int nu1 = (S + UR1 - 1) / UR1, nhg1 = n_head / hw1;
         hipLaunchKernelGGL((prefill16_kernel<F32, 1, 2>), dim3((unsigned)(nu1 * nhg1 * 2)), dim3(512), 0, st,
                            (const uint16_t *)q, (const char *)kc, (const char *)vc, kvs, S, start_pos,
-                           window, n_head, kv_mul, hw1, nhg1, nu1, qs, out, pgs);
+                           window, n_head, kv_mul, hw1, nhg1, nu1, qs, out, pgs, KeySplit{});
     } else if (dtype == ULLM_DT_BF16) pick(BF16{});
     else pick(F16{});
     return check_hip(hipGetLastError(), "prefill (16-row waves) launch");
@@ -577,7 +698,12 @@ int launch_prefill16(int dtype, const void *q, const void *kc, const void *vc, i
 // f16 or f32 cache, contiguous or paged.
 int launch_prefill16_128(int dtype, const void *q, const void *kc, const void *vc, int64_t kvs,
                          int S, int start_pos, int window, int n_head, int kv_mul, float qs,
-                         float *out, hipStream_t st, KvPages pgs) {
+                         float *out, hipStream_t st, KvPages pgs, void *ws, size_t ws_bytes) {
+    const bool f32 = dtype == ULLM_DT_F32;
+    const SplitPlan pl = f32 ? prefill16_split(dtype, S, start_pos, window, n_head, kv_mul, 128) : SplitPlan{0, 1, 0, 0};
+    if (pl.parts > 1 && ws && ws_bytes >= pl.bytes)
+        return launch_prefill16_split<128>(dtype, q, kc, vc, kvs, S, start_pos, window, n_head, kv_mul, qs,
+                                           out, st, pgs, pl, ws);
     int KS, DS;  // head_dim 128: no value split (V rows of 256 bytes)
     prefill16_plan(S, start_pos, window, n_head, kv_mul, KS, DS);
     const int hw = p16_hw(kv_mul, 8 / KS), UR = 16 * (8 / KS) / hw;
@@ -586,7 +712,7 @@ int launch_prefill16_128(int dtype, const void *q, const void *kc, const void *v
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, grid, dim3(512), 0, st, (const uint16_t *)q, (const char *)kc,
                            (const char *)vc, kvs, S, start_pos, window, n_head, kv_mul, hw, n_hg,
-                           n_units, qs, out, pgs);
+                           n_units, qs, out, pgs, KeySplit{});
     };
     auto pick = [&](auto t) {
         using T = decltype(t);
