@@ -1,0 +1,71 @@
+"""The native front end of attention.py: errors, returned tensors, layer
+indices, and calls on a stream that is not torch's current one."""
+import pytest
+import torch
+
+from ullm_amd import _lib as L
+from ullm_amd import attention as A
+
+pytestmark = pytest.mark.gpu
+
+H, Hk, D, N = 8, 2, 64, 300
+
+
+def _cache(dev, dtype=torch.float16):
+    g = torch.Generator(device=dev).manual_seed(4)
+    k, v = (torch.randn(N, Hk * D, device=dev, generator=g).to(dtype) for _ in range(2))
+    return torch.randn(1, H, D, device=dev, generator=g), k, v, torch.tensor([N], dtype=torch.int32, device=dev)
+
+
+@pytest.mark.parametrize("change,code", [
+    (dict(q=lambda q: q.cpu()), L.E_INVALID), (dict(q=lambda q: q.half()), L.E_INVALID),
+    (dict(q=lambda q: q.transpose(1, 2)), L.E_INVALID), (dict(lens=lambda t: t.long()), L.E_INVALID),
+    (dict(k=lambda k: k.double()), L.E_UNSUPPORTED), (dict(ws=lambda _: torch.empty(8, dtype=torch.uint8, device="cuda")), L.E_WORKSPACE),
+])
+def test_errors_keep_their_codes(dev, change, code):
+    q, k, v, lens = _cache(dev)
+    a = dict(q=q, k=k, v=v, lens=lens, ws=None)
+    for n, f in change.items():
+        a[n] = f(a[n])
+    with pytest.raises(L.UllmHipError) as e:
+        A.attn_decode(a["q"], a["k"], a["v"], a["lens"], N, Hk, workspace=a["ws"])
+    assert e.value.code == code
+    with pytest.raises(TypeError):
+        A.attn_decode(q, None, v, lens, N, Hk)
+
+
+def test_given_out_is_returned_and_written(dev):
+    q, k, v, lens = _cache(dev)
+    out = torch.full((1, H, D), 7.0, device=dev)
+    assert A.attn_decode(q, k, v, lens, N, Hk, out=out) is out
+    assert torch.equal(out, A.attn_decode(q, k, v, lens, N, Hk))
+
+
+def test_other_stream_owns_its_scratch(dev):
+    """Scratch of calls queued on another stream is not handed out while they
+    wait there: the calls give what they give on the current stream."""
+    q, k, v, lens = _cache(dev)
+    qp = torch.randn(9, H * D, device=dev).half()
+    want = A.attn_decode(q, k, v, lens, N, Hk), A.attn_prefill(qp, k, v, H, Hk, D, start_pos=N - 9)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        torch.cuda._sleep(20_000_000)
+    outs = [torch.empty_like(w) for w in want]
+    A.attn_decode(q, k, v, lens, N, Hk, out=outs[0], stream=s)
+    A.attn_prefill(qp, k, v, H, Hk, D, start_pos=N - 9, out=outs[1], stream=s)
+    for _ in range(8):  # would take the scratch if it were free
+        torch.full((1 << 20,), 0xFF, dtype=torch.uint8, device=dev)
+        torch.full((256,), 0xFF, dtype=torch.uint8, device=dev)
+    s.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(outs, want))
+
+
+def test_layer_indices(dev):
+    ga = A.GpuAttention(A.AttnParams(3, H, Hk, D, 16, kv_dtype=torch.float32))
+    q, kk = torch.randn(H * D, device=dev), torch.randn(Hk * D, device=dev)
+    ga.forward(-1, q, kk, kk, 5)
+    assert bool(ga.key_cache[2, 5].any()) and not bool(ga.key_cache[:2].any())
+    for bad in (3, -4):
+        with pytest.raises(IndexError):
+            ga.forward(bad, q, kk, kk, 5)

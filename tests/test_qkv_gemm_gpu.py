@@ -25,9 +25,9 @@ def _raw(x, ws, H, Hk, D, bits, start=0):
     cs = torch.zeros(start + rows, D // 2, 2, device=x.device)
     cs[..., 0] = 1
     kc = torch.full((start + rows + 1, Hk * D), 7.0, device=x.device)
-    vc, q = kc.clone(), torch.empty(rows, H * D, device=x.device)
-    assert A._proj_gemm(x, *ws, kc, vc, cs, start, H, Hk, D, D, True, None, None, 1e-6, None, None,
-                        None, q, Hk * D, bits, None)
+    vc = kc.clone()
+    q = A._F.proj(x, *ws, kc, vc, start, bits, cs, H, Hk, D, D, True, None, None, 1e-6, None, None, None,
+                  None, None, None, None, None)
     for c in (kc, vc):  # rows outside start.. are untouched
         assert bool((c[:start] == 7).all()) and bool((c[start + rows:] == 7).all())
     return q, kc[start:start + rows], vc[start:start + rows]

@@ -1,8 +1,9 @@
 """Torch-tensor front end of the C ABI, and `GpuAttention`, the attention
 part of the reference's `GpuForward` (crates/ullm-metal/src/forward.rs).
 
-Every op here is a thin call into libullm_hip.so; torch supplies device
-memory and the current HIP stream and nothing else.  There is no CPU or
+Every op here is a thin call into libullm_hip.so, through the native front end
+_front.so (argument checks, outputs and scratch, the call; csrc/front/front.cpp);
+torch supplies device memory and the current HIP stream and nothing else.  There is no CPU or
 PyTorch fallback: without the library or a GPU the calls raise.
 """
 from __future__ import annotations
@@ -16,6 +17,24 @@ from typing import Optional
 import torch
 
 from . import _lib as L
+
+class _NoFront:
+    """Stands for the native front end where it does not load: every use raises."""
+
+    def __init__(self, why):
+        self._why = why
+
+    def __getattr__(self, name):
+        raise ImportError(f"ullm_amd/_front.so does not load ({self._why}): build it with "
+                          "`python -m ullm_amd.build` (there is no fallback)")
+
+
+try:
+    from . import _front as _F
+
+    _F.set_error(L.UllmHipError)
+except ImportError as e:
+    _F = _NoFront(e)
 
 _DT = {torch.float32: L.DT_F32, torch.float16: L.DT_F16, torch.bfloat16: L.DT_BF16}
 
@@ -62,26 +81,8 @@ def attn_decode(q, k_cache, v_cache, seq_lens, max_len, n_kv_head, *, window=0, 
     `kv_stride` elements per position (default n_kv_head*D) and `seq_stride`
     between sequences.  seq_lens: int32 [B] on the GPU (= pos + 1).
     """
-    B, H, D = q.shape
-    _need_cuda(q, k_cache, v_cache, seq_lens)
-    if q.dtype != torch.float32 or not q.is_contiguous():
-        raise L.UllmHipError(L.E_INVALID, "q must be contiguous f32 [B, n_head, head_dim]")
-    if seq_lens.dtype != torch.int32 or seq_lens.numel() != B:
-        raise L.UllmHipError(L.E_INVALID, "seq_lens must be int32 [B]")
-    if kv_stride is None:
-        kv_stride = n_kv_head * D
-    if scale is None:
-        scale = 1.0 / math.sqrt(D)
-    if out is None:
-        out = torch.empty(B, H, D, dtype=torch.float32, device=q.device)
-    if workspace is None:
-        workspace = new_decode_workspace(B, H, n_kv_head, D, max_len, window, q.device)
-    rc = L.lib().ullm_hip_attn_decode(
-        _ptr(q), _ptr(k_cache), _ptr(v_cache), _dt(k_cache), kv_stride, seq_stride,
-        _ptr(seq_lens), max_len, window, B, H, n_kv_head, D, float(scale), _ptr(out),
-        _ptr(workspace), workspace.numel(), _stream(stream))
-    L.check(rc)
-    return out
+    return _F.decode(q, k_cache, v_cache, seq_lens, max_len, n_kv_head, window, scale, kv_stride,
+                     seq_stride, out, workspace, stream)
 
 
 def attn_decode_paged(q, k_pages, v_pages, block_table, seq_lens, max_len, n_kv_head, *,
@@ -92,32 +93,8 @@ def attn_decode_paged(q, k_pages, v_pages, block_table, seq_lens, max_len, n_kv_
     f16/bf16.  block_table: int32 [B, table_stride] (page of position t of
     sequence b = block_table[b, t // page_size]).  seq_lens: int32 [B].
     """
-    B, H, D = q.shape
-    _need_cuda(q, k_pages, v_pages, block_table, seq_lens)
-    if q.dtype != torch.float32 or not q.is_contiguous():
-        raise L.UllmHipError(L.E_INVALID, "q must be contiguous f32 [B, n_head, head_dim]")
-    if k_pages.dim() != 3 or k_pages.shape != v_pages.shape or not k_pages.is_contiguous() \
-            or not v_pages.is_contiguous():
-        raise L.UllmHipError(L.E_INVALID, "k_pages/v_pages must be contiguous [n_pages, page_size, kv_stride]")
-    if block_table.dtype != torch.int32 or block_table.dim() != 2 or block_table.shape[0] != B \
-            or not block_table.is_contiguous():
-        raise L.UllmHipError(L.E_INVALID, "block_table must be contiguous int32 [B, table_stride]")
-    if seq_lens.dtype != torch.int32 or seq_lens.numel() != B:
-        raise L.UllmHipError(L.E_INVALID, "seq_lens must be int32 [B]")
-    n_pages, page_size, kv_stride = k_pages.shape
-    if scale is None:
-        scale = 1.0 / math.sqrt(D)
-    if out is None:
-        out = torch.empty(B, H, D, dtype=torch.float32, device=q.device)
-    if workspace is None:
-        n = int(L.lib().ullm_hip_paged_decode_workspace_bytes(B, H, n_kv_head, D, max_len, window))
-        workspace = torch.zeros(max(n, 256), dtype=torch.uint8, device=q.device)
-    rc = L.lib().ullm_hip_attn_decode_paged(
-        _ptr(q), _ptr(k_pages), _ptr(v_pages), _dt(k_pages), kv_stride, page_size, n_pages,
-        _ptr(block_table), block_table.shape[1], _ptr(seq_lens), max_len, window, B, H, n_kv_head,
-        D, float(scale), _ptr(out), _ptr(workspace), workspace.numel(), _stream(stream))
-    L.check(rc)
-    return out
+    return _F.decode_paged(q, k_pages, v_pages, block_table, seq_lens, max_len, n_kv_head, window,
+                           scale, out, workspace, stream)
 
 
 def qkv_append_paged(q, k, v, k_pages, v_pages, rope_cs, positions, block_table, *, n_head,
@@ -127,58 +104,9 @@ def qkv_append_paged(q, k, v, k_pages, v_pages, rope_cs, positions, block_table,
     """Append one token per sequence into a paged cache: row r of q/k/v [rows,
     *] f32 is sequence r's token at positions[r] (int32 [rows] on the GPU);
     its K/V rows land in block_table[r, pos // page_size].  Returns q_out."""
-    rows = q.shape[0]
-    _need_cuda(q, k, v, k_pages, v_pages, rope_cs, positions, block_table)
-    for t in (q, k, v):
-        if t.dtype != torch.float32 or not t.is_contiguous():
-            raise L.UllmHipError(L.E_INVALID, "q/k/v must be contiguous f32")
-    if k_pages.dim() != 3 or k_pages.shape != v_pages.shape:
-        raise L.UllmHipError(L.E_INVALID, "k_pages/v_pages must be [n_pages, page_size, kv_stride]")
-    if positions.dtype != torch.int32 or positions.numel() != rows:
-        raise L.UllmHipError(L.E_INVALID, "positions must be int32 [rows]")
-    if block_table.dtype != torch.int32 or block_table.dim() != 2 or block_table.shape[0] != rows \
-            or not block_table.is_contiguous():
-        raise L.UllmHipError(L.E_INVALID, "block_table must be contiguous int32 [rows, table_stride]")
-    n_pages, page_size, kv_stride = k_pages.shape
-    if rotary_dim is None:
-        rotary_dim = head_dim
-    if q_dtype is None:
-        q_dtype = torch.float32
-    if q_out is None:
-        q_out = torch.empty(rows, n_head * head_dim, dtype=q_dtype, device=q.device)
-    rc = L.lib().ullm_hip_qkv_append_paged(
-        _ptr(q), _ptr(k), _ptr(v), _ptr(q_bias), _ptr(k_bias), _ptr(v_bias), _ptr(q_norm),
-        _ptr(k_norm), float(eps), _ptr(rope_cs), rope_cs.shape[0], int(bool(neox)), rotary_dim,
-        rows, _ptr(positions), n_head, n_kv_head, head_dim, _ptr(q_out), _DT[q_out.dtype],
-        _ptr(k_pages), _ptr(v_pages), _dt(k_pages), kv_stride, page_size, n_pages,
-        _ptr(block_table), block_table.shape[1], _stream(stream))
-    L.check(rc)
-    return q_out
-
-
-# The scratch sizes depend on these numbers alone.
-@functools.lru_cache(maxsize=1024)
-def _prefill_bytes(dtype, S, start_pos, window, n_head, n_kv_head, head_dim):
-    return int(L.lib().ullm_hip_prefill_workspace_bytes(dtype, S, start_pos, window, n_head,
-                                                        n_kv_head, head_dim))
-
-
-@functools.lru_cache(maxsize=1024)
-def _gemm_bytes(rows, in_dim, w_dtype, x_bits, n_head, n_kv_head, head_dim):
-    return int(L.lib().ullm_hip_qkv_gemm_workspace_bytes(rows, in_dim, w_dtype, x_bits, n_head,
-                                                         n_kv_head, head_dim))
-
-
-def _prefill_scratch(q, S, start_pos, window, n_head, n_kv_head, head_dim, stream):
-    """Scratch for a prefill call that splits its key ranges: (tensor, bytes),
-    or (None, 0) where it does not."""
-    n = _prefill_bytes(_dt(q), S, start_pos, window, n_head, n_kv_head, head_dim)
-    if n == 0:
-        return None, 0
-    ws = torch.empty(n, dtype=torch.uint8, device=q.device)
-    if stream is not None:
-        ws.record_stream(stream)
-    return ws, n
+    return _F.append_paged(q, k, v, k_pages, v_pages, positions, block_table, rope_cs, n_head,
+                           n_kv_head, head_dim, rotary_dim, neox, q_norm, k_norm, eps, q_bias,
+                           k_bias, v_bias, q_out, q_dtype, stream)
 
 
 def attn_prefill_paged(q, k_pages, v_pages, block_table, n_head, n_kv_head, head_dim, *,
@@ -187,26 +115,8 @@ def attn_prefill_paged(q, k_pages, v_pages, block_table, n_head, n_kv_head, head
     keys live in pages: block_table int32 [table_len] (page of key t =
     block_table[t // page_size]).  q: [S, n_head*head_dim] f16/bf16, or f32
     with f32 pages (head_dim 64, 128 or 256)."""
-    S = q.shape[0]
-    _need_cuda(q, k_pages, v_pages, block_table)
-    if not q.is_contiguous() or q.numel() != S * n_head * head_dim:
-        raise L.UllmHipError(L.E_INVALID, "q must be contiguous [S, n_head*head_dim]")
-    if k_pages.dim() != 3 or k_pages.shape != v_pages.shape or q.dtype != k_pages.dtype:
-        raise L.UllmHipError(L.E_INVALID, "k_pages/v_pages must be [n_pages, page_size, kv_stride] of q's dtype")
-    if block_table.dtype != torch.int32 or block_table.dim() != 1:
-        raise L.UllmHipError(L.E_INVALID, "block_table must be int32 [table_len]")
-    n_pages, page_size, kv_stride = k_pages.shape
-    if scale is None:
-        scale = 1.0 / math.sqrt(head_dim)
-    if out is None:
-        out = torch.empty(S, n_head * head_dim, dtype=torch.float32, device=q.device)
-    ws, wsb = _prefill_scratch(q, S, start_pos, window, n_head, n_kv_head, head_dim, stream)
-    rc = L.lib().ullm_hip_attn_prefill_paged_ws(
-        _ptr(q), _ptr(k_pages), _ptr(v_pages), _dt(q), kv_stride, page_size, n_pages,
-        _ptr(block_table), block_table.numel(), S, start_pos, window, n_head, n_kv_head, head_dim,
-        float(scale), _ptr(out), _ptr(ws), wsb, _stream(stream))
-    L.check(rc)
-    return out
+    return _F.prefill_paged(q, k_pages, v_pages, block_table, n_head, n_kv_head, head_dim,
+                            start_pos, window, scale, out, stream)
 
 
 # Largest q the prefill entry points take in one call (below 2 GiB, and a
@@ -225,29 +135,8 @@ def attn_prefill(q, k_cache, v_cache, n_head, n_kv_head, head_dim, *, start_pos=
     cache already holds every position, so each chunk's rows see the same
     keys.
     """
-    S = q.shape[0]
-    _need_cuda(q, k_cache, v_cache)
-    if not q.is_contiguous() or q.numel() != S * n_head * head_dim:
-        raise L.UllmHipError(L.E_INVALID, "q must be contiguous [S, n_head*head_dim]")
-    if q.dtype != k_cache.dtype or q.dtype != v_cache.dtype:
-        raise L.UllmHipError(L.E_INVALID, "q and cache dtypes differ")
-    if kv_stride is None:
-        kv_stride = n_kv_head * head_dim
-    if scale is None:
-        scale = 1.0 / math.sqrt(head_dim)
-    if out is None:
-        out = torch.empty(S, n_head * head_dim, dtype=torch.float32, device=q.device)
-    row_bytes = n_head * head_dim * q.element_size()
-    rows = max(1, PREFILL_Q_MAX_BYTES // row_bytes)
-    for r0 in range(0, max(S, 1), rows):
-        n = min(rows, S - r0)
-        ws, wsb = _prefill_scratch(q, n, start_pos + r0, window, n_head, n_kv_head, head_dim, stream)
-        rc = L.lib().ullm_hip_attn_prefill_ws(
-            _ptr(q[r0:r0 + n]), _ptr(k_cache), _ptr(v_cache), _dt(q), kv_stride, n,
-            start_pos + r0, window, n_head, n_kv_head, head_dim, float(scale),
-            _ptr(out[r0:r0 + n]), _ptr(ws), wsb, _stream(stream))
-        L.check(rc)
-    return out
+    return _F.prefill(q, k_cache, v_cache, n_head, n_kv_head, head_dim, start_pos, window, scale,
+                      kv_stride, out, stream, PREFILL_Q_MAX_BYTES)
 
 
 def rope_table(n_pos: int, rotary_dim: int, theta: float, device="cuda") -> torch.Tensor:
@@ -267,41 +156,30 @@ def qkv_append(q, k, v, k_cache, v_cache, rope_cs, *, start_pos, n_head, n_kv_he
     q: [rows, n_head*D] f32, k/v: [rows, n_kv_head*D] f32.  K/V land in the
     cache at positions start_pos..; returns q_out ([rows, n_head*D], q_dtype).
     """
-    rows = q.shape[0]
-    _need_cuda(q, k, v, k_cache, v_cache, rope_cs)
-    for t in (q, k, v):
-        if t.dtype != torch.float32 or not t.is_contiguous():
-            raise L.UllmHipError(L.E_INVALID, "q/k/v must be contiguous f32")
-    if rotary_dim is None:
-        rotary_dim = head_dim
-    if q_dtype is None:
-        q_dtype = torch.float32
-    if q_out is None:
-        q_out = torch.empty(rows, n_head * head_dim, dtype=q_dtype, device=q.device)
-    if kv_stride is None:
-        kv_stride = n_kv_head * head_dim
-    rc = L.lib().ullm_hip_qkv_append(
-        _ptr(q), _ptr(k), _ptr(v), _ptr(q_bias), _ptr(k_bias), _ptr(v_bias), _ptr(q_norm),
-        _ptr(k_norm), float(eps), _ptr(rope_cs), rope_cs.shape[0], int(bool(neox)), rotary_dim,
-        rows, start_pos, n_head, n_kv_head, head_dim, _ptr(q_out), _DT[q_out.dtype],
-        _ptr(k_cache), _ptr(v_cache), _dt(k_cache), kv_stride, _stream(stream))
-    L.check(rc)
-    return q_out
+    return _F.append(q, k, v, k_cache, v_cache, start_pos, rope_cs, n_head, n_kv_head, head_dim,
+                     rotary_dim, neox, q_norm, k_norm, eps, q_bias, k_bias, v_bias, q_out, q_dtype,
+                     kv_stride, stream)
 
 
 _proj_ws = {}
 
 
+@functools.lru_cache(maxsize=256)
+def _proj_ws_bytes(rows, n_head, n_kv_head, head_dim):
+    return int(L.lib().ullm_hip_qkv_proj_workspace_bytes(rows, n_head, n_kv_head, head_dim))
+
+
 def proj_workspace(rows, n_head, n_kv_head, head_dim, device="cuda"):
     """The (zeroed once, reusable) workspace ullm_hip_qkv_proj_append needs for
     this shape, or None; cached per shape and device."""
-    n = int(L.lib().ullm_hip_qkv_proj_workspace_bytes(rows, n_head, n_kv_head, head_dim))
+    n = _proj_ws_bytes(rows, n_head, n_kv_head, head_dim)
     if n == 0:
         return None
-    key = (str(torch.device(device)), rows, n_head, n_kv_head, head_dim)
-    if key not in _proj_ws:
-        _proj_ws[key] = torch.zeros(n, dtype=torch.uint8, device=device)
-    return _proj_ws[key]
+    key = (str(device), rows, n_head, n_kv_head, head_dim)
+    ws = _proj_ws.get(key)
+    if ws is None:
+        ws = _proj_ws[key] = torch.zeros(n, dtype=torch.uint8, device=device)
+    return ws
 
 
 def _gemm_pays(rows, n, in_dim, head_dim, w_dtype):
@@ -317,28 +195,6 @@ def _gemm_pays(rows, n, in_dim, head_dim, w_dtype):
     return rows * n * in_dim >= (320_000_000 if w_dtype == torch.float32 else 160_000_000)
 
 
-def _proj_gemm(x, w_q, w_k, w_v, k_cache, v_cache, rope_cs, start_pos, n_head, n_kv_head, head_dim,
-               rotary_dim, neox, q_norm, k_norm, eps, q_bias, k_bias, v_bias, q_out, kv_stride,
-               x_bits, stream):
-    """ullm_hip_qkv_gemm_append with its scratch from the caching allocator;
-    False (nothing done) where an operand is too large for it."""
-    rows, in_dim = x.shape
-    lib = L.lib()
-    n = _gemm_bytes(rows, in_dim, _dt(w_q), x_bits, n_head, n_kv_head, head_dim)
-    if n == 0:
-        return False
-    ws = torch.empty(n, dtype=torch.uint8, device=x.device)
-    if stream is not None:
-        ws.record_stream(stream)
-    L.check(lib.ullm_hip_qkv_gemm_append(
-        _ptr(x), in_dim, _ptr(w_q), _ptr(w_k), _ptr(w_v), _dt(w_q), x_bits, _ptr(q_bias),
-        _ptr(k_bias), _ptr(v_bias), _ptr(q_norm), _ptr(k_norm), float(eps), _ptr(rope_cs),
-        rope_cs.shape[0], int(bool(neox)), rotary_dim, rows, start_pos, n_head, n_kv_head, head_dim,
-        _ptr(q_out), _DT[q_out.dtype], _ptr(k_cache), _ptr(v_cache), _dt(k_cache), kv_stride,
-        _ptr(ws), n, _stream(stream)))
-    return True
-
-
 def qkv_proj_append(x, w_q, w_k, w_v, k_cache, v_cache, rope_cs, *, start_pos, n_head,
                     n_kv_head, head_dim, rotary_dim=None, neox=True, q_norm=None, k_norm=None,
                     eps=1e-6, q_bias=None, k_bias=None, v_bias=None, q_out=None, q_dtype=None,
@@ -349,39 +205,17 @@ def qkv_proj_append(x, w_q, w_k, w_v, k_cache, v_cache, rope_cs, *, start_pos, n
     workspace defaults to a cached one per shape (one caller at a time, as for
     GpuForward)."""
     rows, in_dim = x.shape
-    _need_cuda(x, w_q, w_k, w_v, k_cache, v_cache, rope_cs)
-    if x.dtype != torch.float32 or not x.is_contiguous():
-        raise L.UllmHipError(L.E_INVALID, "x must be contiguous f32")
-    if not (w_q.dtype == w_k.dtype == w_v.dtype):
-        raise L.UllmHipError(L.E_INVALID, "w_q/w_k/w_v must share one dtype")
-    for w, n in ((w_q, n_head), (w_k, n_kv_head), (w_v, n_kv_head)):
-        if tuple(w.shape) != (n * head_dim, in_dim) or not w.is_contiguous():
-            raise L.UllmHipError(L.E_INVALID, f"weight shape {tuple(w.shape)} != ({n * head_dim}, {in_dim})")
-    if rotary_dim is None:
-        rotary_dim = head_dim
-    if q_dtype is None:
-        q_dtype = torch.float32
-    if q_out is None:
-        q_out = torch.empty(rows, n_head * head_dim, dtype=q_dtype, device=x.device)
-    if kv_stride is None:
-        kv_stride = n_kv_head * head_dim
     n = (n_head + 2 * n_kv_head) * head_dim
-    if rows <= 65535 and _gemm_pays(rows, n, in_dim, head_dim, w_q.dtype) and _proj_gemm(
-            x, w_q, w_k, w_v, k_cache, v_cache, rope_cs, start_pos, n_head, n_kv_head, head_dim,
-            rotary_dim, neox, q_norm, k_norm, eps, q_bias, k_bias, v_bias, q_out, kv_stride, 24,
-            stream):
-        return q_out
+    args = (x, w_q, w_k, w_v, k_cache, v_cache, start_pos)
+    prep = (rope_cs, n_head, n_kv_head, head_dim, rotary_dim, neox, q_norm, k_norm, eps, q_bias, k_bias,
+            v_bias, q_out, q_dtype, kv_stride)
+    if rows <= 65535 and _gemm_pays(rows, n, in_dim, head_dim, w_q.dtype):
+        q = _F.proj(*args, 24, *prep, None, stream)
+        if q is not None:
+            return q
     if workspace is None:
         workspace = proj_workspace(rows, n_head, n_kv_head, head_dim, x.device)
-    wsb = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    rc = L.lib().ullm_hip_qkv_proj_append(
-        _ptr(x), in_dim, _ptr(w_q), _ptr(w_k), _ptr(w_v), _dt(w_q), _ptr(q_bias), _ptr(k_bias),
-        _ptr(v_bias), _ptr(q_norm), _ptr(k_norm), float(eps), _ptr(rope_cs), rope_cs.shape[0],
-        int(bool(neox)), rotary_dim, rows, start_pos, n_head, n_kv_head, head_dim, _ptr(q_out),
-        _DT[q_out.dtype], _ptr(k_cache), _ptr(v_cache), _dt(k_cache), kv_stride, _ptr(workspace),
-        wsb, _stream(stream))
-    L.check(rc)
-    return q_out
+    return _F.proj(*args, 0, *prep, workspace, stream)
 
 
 def matmul(w, x, y=None, *, stream=None):
@@ -495,11 +329,9 @@ class GpuAttention:
                                    rotary_dim=self.rotary_dim, neox=p.rope_neox, q_norm=norms[0],
                                    k_norm=norms[1], eps=p.eps, q_bias=biases[0],
                                    k_bias=biases[1], v_bias=biases[2], q_dtype=p.kv_dtype)
-        qr = torch.empty(rows, p.n_head * D, dtype=p.kv_dtype, device=xbs.device)
-        ok = _proj_gemm(xbs, wq, wk, wv, kc, vc, self.rope_cs, start_pos, p.n_head, p.n_kv_head, D,
-                        self.rotary_dim, p.rope_neox, norms[0], norms[1], p.eps, *biases, qr,
-                        self.kv_dim, 16, None)
-        return qr if ok else None
+        return _F.proj(xbs, wq, wk, wv, kc, vc, start_pos, 16, self.rope_cs, p.n_head, p.n_kv_head, D,
+                       self.rotary_dim, p.rope_neox, norms[0], norms[1], p.eps, *biases, None,
+                       p.kv_dtype, None, None, None)
 
     def forward(self, layer: int, q, k, v, pos: int, q_norm=None, k_norm=None, q_bias=None,
                 k_bias=None, v_bias=None):
@@ -508,13 +340,18 @@ class GpuAttention:
         p = self.p
         if not 0 <= pos < p.n_ctx:
             raise L.UllmHipError(L.E_INVALID, f"pos {pos} outside the context")
-        qr = self._append(layer, q.view(1, -1), k.view(1, -1), v.view(1, -1), pos,
-                          torch.float32, (q_norm, k_norm), (q_bias, k_bias, v_bias))
-        out = attn_decode(qr.view(1, p.n_head, p.head_dim), self.key_cache[layer],
-                          self.val_cache[layer], self._lens[pos:pos + 1], pos + 1, p.n_kv_head,
-                          window=self._window(layer), scale=self.scale,
-                          workspace=self.workspace)
-        return out.view(-1)
+        return self._token(False, layer, pos, q_norm, k_norm, q_bias, k_bias, v_bias, q, k, v, None,
+                           None)
+
+    def _token(self, proj, layer, pos, q_norm, k_norm, q_bias, k_bias, v_bias, *ins):
+        """Append or projection (proj), then attention, of one token in one
+        native call; `ins`: q, k, v or the hidden state, the weights and the
+        projection's workspace."""
+        p = self.p
+        return _F.token(proj, layer, pos, self.key_cache, self.val_cache, self._lens, self.workspace,
+                        self._window(layer), self.scale, self.rope_cs, p.n_head, p.n_kv_head,
+                        p.head_dim, self.rotary_dim, p.rope_neox, q_norm, k_norm, p.eps, q_bias,
+                        k_bias, v_bias, *ins)
 
     def forward_batch(self, layer: int, q, k, v, start_pos: int = 0, q_norm=None, k_norm=None,
                       q_bias=None, k_bias=None, v_bias=None):
@@ -540,17 +377,8 @@ class GpuAttention:
         p = self.p
         if not 0 <= pos < p.n_ctx:
             raise L.UllmHipError(L.E_INVALID, f"pos {pos} outside the context")
-        qr = qkv_proj_append(xb.view(1, -1), wq, wk, wv, self.key_cache[layer],
-                             self.val_cache[layer], self.rope_cs, start_pos=pos,
-                             n_head=p.n_head, n_kv_head=p.n_kv_head, head_dim=p.head_dim,
-                             rotary_dim=self.rotary_dim, neox=p.rope_neox, q_norm=q_norm,
-                             k_norm=k_norm, eps=p.eps, q_bias=q_bias, k_bias=k_bias,
-                             v_bias=v_bias, q_dtype=torch.float32)
-        out = attn_decode(qr.view(1, p.n_head, p.head_dim), self.key_cache[layer],
-                          self.val_cache[layer], self._lens[pos:pos + 1], pos + 1, p.n_kv_head,
-                          window=self._window(layer), scale=self.scale,
-                          workspace=self.workspace)
-        return out.view(-1)
+        return self._token(True, layer, pos, q_norm, k_norm, q_bias, k_bias, v_bias, xb, wq, wk, wv,
+                           proj_workspace(1, p.n_head, p.n_kv_head, p.head_dim, xb.device))
 
     def forward_batch_proj(self, layer: int, xbs, wq, wk, wv, start_pos: int = 0, q_norm=None,
                            k_norm=None, q_bias=None, k_bias=None, v_bias=None):

@@ -15,6 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libullm_hip.so")
+FRONT = os.path.join(HERE, "_front.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 # -packed-fp32-ops off: hipcc must not form v_pk_{add,mul,fma}_f32 on its own.
@@ -40,8 +41,32 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _build_front() -> None:
+    """The native half of attention.py (csrc/front/front.cpp), host code only,
+    against torch's headers and the library just built."""
+    import sysconfig
+
+    import torch
+
+    t = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(HIPCC))
+    tmp = FRONT + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-isystem", f"{t}/include", "-isystem", f"{t}/include/torch/csrc/api/include",
+           "-isystem", f"{rocm}/include", "-isystem", sysconfig.get_paths()["include"],
+           os.path.join(CSRC, "front", "front.cpp"), "-o", tmp, f"-L{HERE}", "-l:libullm_hip.so",
+           f"-L{t}/lib", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
+           "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"front end failed:\n{r.stderr}")
+    os.replace(tmp, FRONT)
+
+
 def build(verbose: bool = True) -> str:
-    """Compile every kernel source for gfx950 and link libullm_hip.so."""
+    """Compile every kernel source for gfx950, link libullm_hip.so, and build
+    the front end on it."""
     os.makedirs(OBJ, exist_ok=True)
     srcs = _sources()
     jobs = min(len(srcs), int(os.environ.get("MAX_JOBS", "8")))
@@ -60,6 +85,7 @@ def build(verbose: bool = True) -> str:
     except OSError as e:
         raise RuntimeError(f"built library does not load: {e}") from None
     os.replace(tmp, LIB)
+    _build_front()
     if verbose:
         print(f"built {LIB} from {len(srcs)} sources", file=sys.stderr)
     return LIB
