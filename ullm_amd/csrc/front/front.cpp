@@ -13,6 +13,7 @@
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <ATen/ATen.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/hip/HIPStream.h>
 #include <cmath>
 
@@ -106,7 +107,8 @@ struct Stream {
     at::Tensor scratch(const at::Tensor &like, int64_t bytes) const {
         at::Tensor t = at::empty({bytes}, like.options().dtype(at::kByte));
         if (given)
-            t.record_stream(c10::hip::getStreamFromExternal((hipStream_t)s, like.device().index()).unwrap());
+            t.record_stream(
+                c10::hip::getStreamFromExternalMasqueradingAsCUDA((hipStream_t)s, like.device().index()).unwrap());
         return t;
     }
 };
