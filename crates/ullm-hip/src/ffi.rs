@@ -100,6 +100,18 @@ unsafe extern "C" {
         stream: *mut c_void) -> c_int;
     pub fn ullm_hip_prefill_workspace_bytes(dtype: c_int, s: c_int, start_pos: c_int,
         window: c_int, n_head: c_int, n_kv_head: c_int, head_dim: c_int) -> usize;
+    pub fn ullm_hip_decode_token(q: *const f32, k: *const f32, v: *const f32,
+        q_bias: *const f32, k_bias: *const f32, v_bias: *const f32, q_norm: *const f32,
+        k_norm: *const f32, eps: f32, rope_cs: *const f32, rope_n_pos: c_int, rope_neox: c_int,
+        pos: c_int, old_len: *const i32, window: c_int, n_head: c_int, n_kv_head: c_int,
+        head_dim: c_int, scale: f32, k_cache: *mut c_void, v_cache: *mut c_void,
+        kv_dtype: c_int, kv_stride: i64, out: *mut f32, workspace: *mut c_void,
+        workspace_bytes: usize, stream: *mut c_void) -> c_int;
+    pub fn ullm_hip_decode_token_workspace_bytes(kv_dtype: c_int, pos: c_int, window: c_int,
+        n_head: c_int, n_kv_head: c_int, head_dim: c_int, rotary_dim: c_int) -> usize;
+    pub fn ullm_hip_qkv_matvec(x: *const f32, in_dim: c_int, w_q: *const c_void,
+        w_k: *const c_void, w_v: *const c_void, w_dtype: c_int, n_head: c_int,
+        n_kv_head: c_int, head_dim: c_int, y: *mut f32, stream: *mut c_void) -> c_int;
     pub fn ullm_hip_matmul(w: *const c_void, w_dtype: c_int, x: *const f32, y: *mut f32,
         in_dim: c_int, out_dim: c_int, n_cols: c_int, stream: *mut c_void) -> c_int;
 }

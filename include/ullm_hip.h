@@ -225,6 +225,33 @@ int ullm_hip_qkv_gemm_append(const float *x, int in_dim, const void *w_q, const 
 size_t ullm_hip_qkv_gemm_workspace_bytes(int rows, int in_dim, int w_dtype, int x_bits, int n_head,
                                          int n_kv_head, int head_dim);
 
+/* One decoded token from its raw q, k and v rows: the bias, norm and RoPE and
+ * the cache store of ullm_hip_qkv_append (one row at position pos, full-width
+ * RoPE) and the attention of ullm_hip_attn_decode over positions 0..pos, in the
+ * two launches of the attention alone: the split kernels prepare q and attend
+ * the old keys, the merge adds the token's own key and stores its cache row.
+ * q/k/v: DEVICE f32 rows; rope_cs as for ullm_hip_qkv_append with rotary_dim =
+ * head_dim; old_len: DEVICE int32 holding pos.  Every pointer 16-byte aligned
+ * (biases and norms may be NULL).  head_dim 64 or 128, one sequence, and
+ * enough old keys to be split: ullm_hip_decode_token_workspace_bytes returns 0
+ * for what it does not take (ULLM_HIP_E_UNSUPPORTED, nothing launched). */
+int ullm_hip_decode_token(const float *q, const float *k, const float *v, const float *q_bias,
+                          const float *k_bias, const float *v_bias, const float *q_norm,
+                          const float *k_norm, float eps, const float *rope_cs, int rope_n_pos,
+                          int rope_neox, int pos, const int32_t *old_len, int window, int n_head,
+                          int n_kv_head, int head_dim, float scale, void *k_cache, void *v_cache,
+                          int kv_dtype, int64_t kv_stride, float *out, void *workspace,
+                          size_t workspace_bytes, void *stream);
+size_t ullm_hip_decode_token_workspace_bytes(int kv_dtype, int pos, int window, int n_head,
+                                             int n_kv_head, int head_dim, int rotary_dim);
+
+/* The raw projection of one token, y = [W_q x | W_k x | W_v x] (f32, f32 sums),
+ * for ullm_hip_decode_token.  Arguments as for ullm_hip_qkv_proj_append;
+ * y: DEVICE f32 [(n_head + 2*n_kv_head) * head_dim]. */
+int ullm_hip_qkv_matvec(const float *x, int in_dim, const void *w_q, const void *w_k,
+                        const void *w_v, int w_dtype, int n_head, int n_kv_head, int head_dim,
+                        float *y, void *stream);
+
 /* Batched projection for prefill: y[s*out_dim + o] = sum_i w[o*in_dim + i] *
  * x[s*in_dim + i] for s < n_cols, o < out_dim.  Replaces the reference's
  * batched matmul (crates/ullm-metal/src/forward.rs:675-726, kernel

@@ -303,3 +303,27 @@ def test_workspace_for_n_ctx_bounds_every_shorter_call(dt, shape, n_ctx, win, pa
     for n in range(1, n_ctx + 1):
         need = _needed_ws(dt, h, hk, d, n, win, paged)
         assert need <= bound, f"max_len {n}: needs {need} > {bound} sized for {n_ctx}"
+
+
+def test_decode_token_validation():
+    f, wsz = L.lib().ullm_hip_decode_token, L.lib().ullm_hip_decode_token_workspace_bytes
+
+    def call(**kw):
+        a = dict(q=64, k=64, v=64, qb=None, kb=None, vb=None, qn=None, kn=None, eps=1e-6, cs=64, npos=600, neox=1,
+                 pos=511, ol=64, win=0, h=8, hk=2, d=64, sc=0.1, kc=64, vc=64, dt=L.DT_F16, kvs=128, out=64,
+                 ws=None, wsb=0, st=None)
+        a.update(kw)
+        return f(*a.values())
+
+    for bad in (dict(dt=7), dict(d=256), dict(h=7), dict(pos=0), dict(pos=32), dict(win=1)):
+        assert call(**bad) == L.E_UNSUPPORTED, bad
+    for bad in (dict(kvs=64), dict(kvs=132), dict(npos=511), dict(q=None), dict(k=72), dict(qn=68)):
+        assert call(**bad) == L.E_INVALID, bad
+    assert call() == L.E_WORKSPACE
+    assert wsz(L.DT_F16, 511, 0, 8, 2, 64, 32) == 0  # partial rotary
+    n = wsz(L.DT_F16, 511, 0, 8, 2, 64, 64)
+    assert 0 < n <= L.lib().ullm_hip_decode_workspace_bytes(1, 8, 2, 64, 512, 0)
+    g = L.lib().ullm_hip_qkv_matvec
+    assert g(64, 12, 64, 64, 64, L.DT_F16, 8, 2, 64, 64, None) == L.E_INVALID  # in_dim % 8
+    assert g(64, 16, 64, 72, 64, L.DT_F16, 8, 2, 64, 64, None) == L.E_INVALID  # alignment
+    assert g(64, 16, 64, 64, 64, 5, 8, 2, 64, 64, None) == L.E_UNSUPPORTED

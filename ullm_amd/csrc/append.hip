@@ -11,8 +11,10 @@
 // pair (SplitEpi) and one RMS reduction serves 256/D heads.
 // This replaces the bias, rmsnorm_heads and rope_* Metal dispatches
 // (forward.rs:416-447, :799-853; shader.metal:828-941) with one launch.
+#include <climits>
 #include <cmath>
 #include "common.hpp"
+#include "head_epi.hpp"
 #include "mfma_util.hpp"
 #include "wave.hpp"
 // The split projection's cross-workgroup exchange (qkv_proj_kernel) relies
@@ -22,134 +24,11 @@
 #error "append.hip: the split projection exchange is written for gfx950"
 #endif
 
-
 namespace ullm {
-
-template <int N>
-struct VecF;
-template <> struct VecF<1> { typedef float t; };
-template <> struct VecF<2> { typedef float2 t; };
-template <> struct VecF<4> { typedef float4 t; };
-
-template <int E>
-__device__ __forceinline__ void load_e(const float *p, float (&x)[E]) {
-    if constexpr (E == 1) x[0] = p[0];
-    else if constexpr (E == 2) { const float2 v = *(const float2 *)p; x[0] = v.x; x[1] = v.y; }
-    else { const float4 v = *(const float4 *)p; x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w; }
-}
-
-// Store E consecutive elements converted to OUT_DT.
-template <int OUT_DT, int E>
-__device__ __forceinline__ void store_e(void *base, int64_t idx, const float (&x)[E]) {
-    if constexpr (OUT_DT == ULLM_DT_F32) {
-        float *p = (float *)base + idx;
-        if constexpr (E == 1) p[0] = x[0];
-        else if constexpr (E == 2) *(float2 *)p = float2{x[0], x[1]};
-        else *(float4 *)p = float4{x[0], x[1], x[2], x[3]};
-    } else {
-        // hardware round-to-nearest-even packs
-        auto pk = [](float a, float b) {
-            return OUT_DT == ULLM_DT_F16 ? pack_f16x2(a, b) : pack_bf16x2(a, b);
-        };
-        uint16_t *p = (uint16_t *)base + idx;
-        if constexpr (E == 1) p[0] = (uint16_t)pk(x[0], 0.f);
-        else if constexpr (E == 2) *(uint32_t *)p = pk(x[0], x[1]);
-        else *(uint2 *)p = uint2{pk(x[0], x[1]), pk(x[2], x[3])};
-    }
-}
 
 constexpr int kAppendWaves = 4;
 constexpr int kBatch = 3;  // groups per wave with loads in flight together
 constexpr int kAppendSplitBelow = 256;  // rows under which a row's groups spread over workgroups
-
-// Per-lane state of the head epilogue of one token row: the (cos, sin) of
-// this lane's elements at the row's position and the Q/K norm weights.  A
-// lane holds E = D/64 consecutive elements of a head vector.
-template <int D>
-struct HeadEpi {
-    static constexpr int E = D / 64;
-    int lane, e0, rotary_dim, half, neox;
-    float eps;
-    float rc[E], rs[E], wq[E], wk[E];
-    const float *q_norm, *k_norm;
-
-    __device__ __forceinline__ HeadEpi(const float *cs, int pos, int rotary_dim_, int neox_,
-                                       const float *qn, const float *kn, float eps_)
-        : lane((int)(threadIdx.x & 63)), e0((int)(threadIdx.x & 63) * E), rotary_dim(rotary_dim_),
-          half(rotary_dim_ / 2), neox(neox_), eps(eps_), q_norm(qn), k_norm(kn) {
-        const float *cp = cs + (int64_t)pos * half * 2;
-#pragma unroll
-        for (int i = 0; i < E; i++) {
-            const int e = e0 + i;
-            const int j = e < rotary_dim ? (neox ? (e < half ? e : e - half) : e >> 1) : 0;
-            rc[i] = cp[2 * j];
-            rs[i] = cp[2 * j + 1];
-            wq[i] = 1.f;
-            wk[i] = 1.f;
-        }
-        if (q_norm) load_e<E>(q_norm + e0, wq);
-        if (k_norm) load_e<E>(k_norm + e0, wk);
-    }
-
-    // Bias (already added by the caller), per-head RMSNorm (math.rs:82-86)
-    // and RoPE (math.rs:116-161) of one head vector of kind 0 (q), 1 (k) or
-    // 2 (v), in the reference's order.  lds_row: D floats private to the
-    // wave, used only for partial-rotary pairs.
-    __device__ __forceinline__ void norm_rope(float (&x)[E], int kind, float *lds_row) const {
-        const float *nw = kind == 0 ? q_norm : (kind == 1 ? k_norm : nullptr);
-        if (nw) {
-            float ss = 0.f;
-#pragma unroll
-            for (int i = 0; i < E; i++) ss += x[i] * x[i];
-            ss = wave_sum(ss);
-            // v_rsq_f32 (~1 ulp) for (sum/n + eps).sqrt().recip()
-            const float inv = __builtin_amdgcn_rsqf(ss / (float)D + eps);
-#pragma unroll
-            for (int i = 0; i < E; i++) x[i] = x[i] * inv * (kind == 0 ? wq[i] : wk[i]);
-        }
-        if (kind == 2) return;
-        float y[E];
-        if (rotary_dim == D) {
-            // Full-width RoPE: a NeoX partner (e +- D/2) sits in lane l ^ 32 at
-            // the same element index; an interleaved partner (e ^ 1) in the same
-            // lane, or in lane l ^ 1 when a lane holds one element.
-#pragma unroll
-            for (int i = 0; i < E; i++) {
-                float pa;
-                if (neox) pa = xor32(x[i]);
-                else if constexpr (E == 1) pa = dpp<kDppXor1>(x[i]);
-                else pa = x[i ^ 1];
-                const bool lo = neox ? lane < 32 : ((e0 + i) & 1) == 0;
-                // lo: a*c - b*s with a = own, b = partner; hi: a*s + b*c with a = partner
-                y[i] = lo ? x[i] * rc[i] - pa * rs[i] : pa * rs[i] + x[i] * rc[i];
-            }
-        } else {
-            // Partial rotary: the partner of each pair comes from the wave's
-            // LDS row (LDS operations of one wave complete in order).
-#pragma unroll
-            for (int i = 0; i < E; i++) lds_row[e0 + i] = x[i];
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int i = 0; i < E; i++) {
-                const int e = e0 + i;
-                y[i] = x[i];
-                if (e < rotary_dim) {
-                    if (neox) {
-                        const int j = e < half ? e : e - half;
-                        const float a = lds_row[j], c = lds_row[j + half];
-                        y[i] = e < half ? a * rc[i] - c * rs[i] : a * rs[i] + c * rc[i];
-                    } else {
-                        const float a = lds_row[e & ~1], c = lds_row[e | 1];
-                        y[i] = (e & 1) ? a * rs[i] + c * rc[i] : a * rc[i] - c * rs[i];
-                    }
-                }
-            }
-            __builtin_amdgcn_wave_barrier();  // the row may be rewritten next
-        }
-#pragma unroll
-        for (int i = 0; i < E; i++) x[i] = y[i];
-    }
-};
 
 // Store one finished head vector: q to q_out (row-major [rows][n_head*D]),
 // k / v into cache row crow (the position, or its paged slot).
@@ -699,6 +578,105 @@ extern "C" int ullm_hip_qkv_append_paged(const float *q_in, const float *k_in, c
 
 namespace ullm {
 
+// y = [W_q; W_k; W_v] x of one token, without an epilogue: the decode step's
+// projection, whose bias, norm, RoPE and cache store happen in the attention
+// kernels (decode_mfma.hip).  A workgroup's 8 waves take RPW rows each, every
+// lane accumulating 16-byte chunks of a row in f32 as qkv_proj_kernel does; no
+// head belongs to several workgroups, so nothing is exchanged, and RPW is
+// chosen so that the workgroups fill the CUs in whole rounds.
+// Bound by HBM: 31.5 MB at 2560 -> 6144, bf16.  Six layers with their attention
+// there, us: 1 row per wave 111.7, 2 114.4, 3 (256 workgroups) 108.9, 4 111.2.
+constexpr int kMvWaves = 8;
+template <int WDT, int RPW>
+__global__ __launch_bounds__(kMvWaves * 64) void qkv_matvec_kernel(
+    const float *__restrict__ x, int in_dim, const char *__restrict__ wq,
+    const char *__restrict__ wk, const char *__restrict__ wv, int n_q, int n_kv, int n,
+    float *__restrict__ y) {
+    constexpr int VEC = WVec<WDT>::n, WB = WDT == ULLM_DT_F32 ? 4 : 2, STEP = 64 * VEC;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r0 = (blockIdx.x * kMvWaves + wave) * RPW;  // wave-uniform
+    if (r0 >= n) return;
+    const char *w[RPW];
+#pragma unroll
+    for (int r = 0; r < RPW; r++) {
+        const int o = min(r0 + r, n - 1);
+        w[r] = o < n_q ? wq + (int64_t)o * in_dim * WB
+                       : (o < n_q + n_kv ? wk + (int64_t)(o - n_q) * in_dim * WB
+                                         : wv + (int64_t)(o - n_q - n_kv) * in_dim * WB);
+    }
+    float acc[RPW];
+#pragma unroll
+    for (int r = 0; r < RPW; r++) acc[r] = 0.f;
+    auto load = [&](int c, u32x4 (&wr)[RPW], float (&xv)[VEC]) {
+        const bool ok = c < in_dim;
+#pragma unroll
+        for (int r = 0; r < RPW; r++)
+            wr[r] = ok ? ld16_stream(w[r] + (int64_t)c * WB) : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int h = 0; h < VEC / 4; h++) {
+            const float4 t = ok ? *(const float4 *)(x + c + 4 * h) : float4{0.f, 0.f, 0.f, 0.f};
+            xv[4 * h] = t.x; xv[4 * h + 1] = t.y; xv[4 * h + 2] = t.z; xv[4 * h + 3] = t.w;
+        }
+    };
+    auto mac = [&](const u32x4 (&wr)[RPW], const float (&xv)[VEC]) {
+#pragma unroll
+        for (int r = 0; r < RPW; r++) {
+            float wf[VEC];
+            widen_w<WDT>(wr[r], wf);
+#pragma unroll
+            for (int i = 0; i < VEC; i++) acc[r] = __builtin_fmaf(wf[i], xv[i], acc[r]);
+        }
+    };
+    u32x4 wa[RPW], wb[RPW];
+    float xa[VEC], xb[VEC];
+    int c = lane * VEC;
+    load(c, wa, xa);
+    for (; c < in_dim; c += 2 * STEP) {
+        load(c + STEP, wb, xb);
+        mac(wa, xa);
+        if (c + STEP >= in_dim) break;
+        load(c + 2 * STEP, wa, xa);
+        mac(wb, xb);
+    }
+#pragma unroll
+    for (int r = 0; r < RPW; r++) {
+        const float t = wave_sum(acc[r]);
+        if (lane == 0 && r0 + r < n) y[r0 + r] = t;
+    }
+}
+
+int launch_qkv_matvec(const float *x, int in_dim, const void *wq, const void *wk, const void *wv,
+                      int w_dtype, int n_q, int n_kv, float *y, hipStream_t st) {
+    const int n = n_q + 2 * n_kv;
+    static const int env = env_override("ULLM_HIP_MATVEC_RPW");  // tuning
+    // Rows per wave: the fewest rounds of 256 workgroups, weighted by rows.
+    int best = 1, cost = INT_MAX;
+    for (int rpw = 1; rpw <= 4; rpw++) {
+        const int wgs = (n + kMvWaves * rpw - 1) / (kMvWaves * rpw), c = (wgs + 255) / 256 * rpw;
+        if (c <= cost) best = rpw, cost = c;
+    }
+    if (env >= 1 && env <= 4) best = env;
+    auto go = [&](auto wdt, auto rpw) {
+        constexpr int WDT = decltype(wdt)::value, R = decltype(rpw)::value;
+        hipLaunchKernelGGL((qkv_matvec_kernel<WDT, R>), dim3((n + kMvWaves * R - 1) / (kMvWaves * R)),
+                           dim3(kMvWaves * 64), 0, st, x, in_dim, (const char *)wq, (const char *)wk,
+                           (const char *)wv, n_q, n_kv, n, y);
+    };
+    auto pick = [&](auto wdt) {
+        switch (best) {
+            case 1: go(wdt, Int<1>{}); break;
+            case 2: go(wdt, Int<2>{}); break;
+            case 3: go(wdt, Int<3>{}); break;
+            default: go(wdt, Int<4>{}); break;
+        }
+    };
+    if (w_dtype == ULLM_DT_F32) pick(Int<ULLM_DT_F32>{});
+    else if (w_dtype == ULLM_DT_F16) pick(Int<ULLM_DT_F16>{});
+    else pick(Int<ULLM_DT_BF16>{});
+    return check_hip(hipGetLastError(), "qkv_matvec launch");
+}
+
 // A head vector is split over kProjSplit workgroups when the grid would
 // otherwise leave most CUs idle (decode: a few dozen head vectors).
 constexpr int kProjSplit = 4;
@@ -823,4 +801,20 @@ extern "C" size_t ullm_hip_qkv_proj_workspace_bytes(int rows, int n_head, int n_
                                                     int head_dim) {
     if (rows < 1 || n_head < 1 || n_kv_head < 1 || head_dim < 1) return 0;
     return proj_ws_bytes(rows, n_head + 2 * n_kv_head, head_dim);
+}
+
+extern "C" int ullm_hip_qkv_matvec(const float *x, int in_dim, const void *w_q, const void *w_k,
+                                   const void *w_v, int w_dtype, int n_head, int n_kv_head, int head_dim,
+                                   float *y, void *stream) {
+    if (!dtype_ok(w_dtype)) return set_error(ULLM_HIP_E_UNSUPPORTED, "qkv_matvec: dtype %d", w_dtype);
+    if (n_head < 1 || n_kv_head < 1 || head_dim < 1 ||
+        ((int64_t)n_head + 2 * (int64_t)n_kv_head) * head_dim > 1 << 24)
+        return set_error(ULLM_HIP_E_INVALID, "qkv_matvec: bad heads");
+    if (in_dim < 8 || in_dim % 8)
+        return set_error(ULLM_HIP_E_INVALID, "qkv_matvec: in_dim %d must be a positive multiple of 8", in_dim);
+    if (!x || !w_q || !w_k || !w_v || !y) return set_error(ULLM_HIP_E_INVALID, "qkv_matvec: null tensor pointer");
+    if (((uintptr_t)x | (uintptr_t)w_q | (uintptr_t)w_k | (uintptr_t)w_v) & 15)
+        return set_error(ULLM_HIP_E_INVALID, "qkv_matvec: x and weights must be 16-byte aligned");
+    return launch_qkv_matvec(x, in_dim, w_q, w_k, w_v, w_dtype, n_head * head_dim, n_kv_head * head_dim, y,
+                             (hipStream_t)stream);
 }

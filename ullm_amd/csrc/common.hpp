@@ -121,6 +121,26 @@ int decode_mfma(int dtype, const float *q, const void *kc, const void *vc, int64
 bool decode_f32_block_plan(int batch, int n_head, int n_kv_head, int D, int max_len, int window,
                            size_t *bytes);
 
+// Raw Q/K/V rows of one token (append.hip): y = [q | k | v] f32.
+int launch_qkv_matvec(const float *x, int in_dim, const void *wq, const void *wk, const void *wv,
+                      int w_dtype, int n_q, int n_kv, float *y, hipStream_t st);
+// Bias, per-head norm and full-width RoPE of one token (its row of the
+// (cos, sin) table), for kernels that prepare q, k or v themselves.
+struct TokenPrep {
+    const float *q, *k, *v;     // raw rows
+    const float *qb, *kb, *vb;  // biases or nullptr
+    const float *qn, *kn;       // norm weights or nullptr
+    const float *cs;            // [head_dim/2][2]
+    float eps;
+    int neox;
+};
+// One decoded token on the MFMA kernels with the append fused in; false: not
+// one of its shapes (nothing launched, *rc untouched).
+size_t decode_token_bytes(int dtype, int pos, int win, int nh, int nkv, int D);
+bool decode_token_mfma(int dtype, const TokenPrep &t, void *kc, void *vc, int64_t kvs, const int32_t *old_len,
+                       int pos, int win, int nh, int nkv, int D, float qs, float *out, void *ws,
+                       size_t ws_bytes, hipStream_t st, int *rc);
+
 // f32-cache split-KV decode over a paged cache (decode.hip).
 size_t decode_f32_workspace(int batch, int n_head, int n_kv_head, int D, int max_len, int window);
 int decode_f32_paged(const float *q, const void *kp, const void *vp, int64_t kvs,

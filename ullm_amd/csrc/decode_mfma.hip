@@ -30,6 +30,7 @@
 #include <cstdlib>
 #include <type_traits>
 #include "common.hpp"
+#include "head_epi.hpp"
 #include "mfma_util.hpp"
 #include "wave.hpp"
 
@@ -37,6 +38,85 @@ namespace ullm {
 
 constexpr int kMW = 4;          // waves per workgroup
 constexpr int kTok = 32;        // keys per wave iteration (two 16-key tiles)
+// Bias, norm and RoPE of the q operand in the split kernels' registers: lane
+// (head n16, kg) holds d = 32 s + 8 kg + 4 h + i in qa[s][h][i], so a head is
+// four lanes (rows_sum), and both members of every RoPE pair (d and d + D/2, or
+// d and d + 1) are in one lane.  load() goes out with q, before the K/V stream.
+template <int D>
+struct QPrep {
+    static constexpr int NS = D / 32;
+    f32x4 w[NS][2], b[NS][2], cs[NS][2];
+    __device__ __forceinline__ void load(const TokenPrep &t, int head, int kg) {
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int d = s * 32 + kg * 8 + h * 4;
+                if (t.qb) b[s][h] = *(const f32x4 *)(t.qb + head * D + d);
+                if (t.qn) w[s][h] = *(const f32x4 *)(t.qn + d);
+                // NeoX: (c, s) of pairs d..d+3 (d < D/2) in cs[2s + h]'s two
+                // halves; interleaved: of the pairs (d, d+1), (d+2, d+3)
+                if (!t.neox) cs[s][h] = *(const f32x4 *)(t.cs + d);
+            }
+        if (t.neox) {
+#pragma unroll
+            for (int s = 0; s < NS / 2; s++)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+#pragma unroll
+                    for (int g = 0; g < 2; g++)
+                        cs[2 * s + h][g] = *(const f32x4 *)(t.cs + 2 * (s * 32 + kg * 8 + h * 4) + 4 * g);
+        }
+    }
+    __device__ __forceinline__ void apply(const TokenPrep &t, f32x4 (&x)[NS][2]) const {
+        if (t.qb)
+#pragma unroll
+            for (int s = 0; s < NS; s++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) x[s][h] += b[s][h];
+        if (t.qn) {
+            float ss = 0.f;
+#pragma unroll
+            for (int s = 0; s < NS; s++)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) ss += x[s][h][i] * x[s][h][i];
+            ss = rows_sum(ss);
+            const float inv = __builtin_amdgcn_rsqf(ss / (float)D + t.eps);
+#pragma unroll
+            for (int s = 0; s < NS; s++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) x[s][h] = x[s][h] * inv * w[s][h];
+        }
+        if (t.neox) {
+#pragma unroll
+            for (int s = 0; s < NS / 2; s++)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const float c = cs[2 * s + h][i >> 1][2 * (i & 1)], sn = cs[2 * s + h][i >> 1][2 * (i & 1) + 1];
+                        const float a = x[s][h][i], e = x[s + NS / 2][h][i];
+                        x[s][h][i] = a * c - e * sn;
+                        x[s + NS / 2][h][i] = a * sn + e * c;
+                    }
+        } else {
+#pragma unroll
+            for (int s = 0; s < NS; s++)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+#pragma unroll
+                    for (int i = 0; i < 4; i += 2) {
+                        const float c = cs[s][h][i], sn = cs[s][h][i + 1];
+                        const float a = x[s][h][i], e = x[s][h][i + 1];
+                        x[s][h][i] = a * c - e * sn;
+                        x[s][h][i + 1] = a * sn + e * c;
+                    }
+        }
+    }
+};
+
 constexpr int kMaxUnitHeads = 16;
 constexpr int kMfmaTargetWG = 256;  // one 4-wave workgroup per CU (LDS-bound)
 
@@ -387,13 +467,14 @@ namespace ullm {
 // there: their V rows are zeroed in LDS (P is 0 for them, but 0 * NaN is
 // NaN).
 
-template <class T, int D, int MW, bool PG = false>
+// TP: q is raw and prepared here (one sequence; see decode_token_mfma).
+template <class T, int D, int MW, bool PG = false, bool TP = false>
 __global__ __launch_bounds__(MW * 64, 1) void decode_dma_kernel(
     const float *__restrict__ q, const char *__restrict__ kc, const char *__restrict__ vc,
     int64_t kv_stride, int64_t seq_stride, const int32_t *__restrict__ seq_lens, int window,
     int fetch_len, int n_head, int kv_mul, int gt, int n_units, int chunk, int splits, float qscale,
     float *__restrict__ out, float *__restrict__ ws_ml, float *__restrict__ ws_acc,
-    const int32_t *__restrict__ ptab, int ptab_stride, int page_shift, int n_pages) {
+    const int32_t *__restrict__ ptab, int ptab_stride, int page_shift, int n_pages, TokenPrep tp) {
     constexpr int NS = D / 32;          // QK k-steps (32 d each)
     constexpr int NDT = D / 16;         // 16-wide d tiles of O^T
     // An f32 cache (the reference's) arrives as f32 tiles; both contractions
@@ -507,6 +588,8 @@ __global__ __launch_bounds__(MW * 64, 1) void decode_dma_kernel(
             qa[s][1] = *(const f32x4 *)(qp + (s * 4 + kg) * 8 + 4);
         }
     }
+    QPrep<D> qprep;
+    if constexpr (TP) qprep.load(tp, head0 + (head_ok ? n16 : 0), kg);
     // Stages are issued only for keys in the fetched range (a wave with one
     // block issues one stage); a stage is waited for with the other stage
     // still counted only when that one was issued, else with vmcnt(0).
@@ -516,6 +599,7 @@ __global__ __launch_bounds__(MW * 64, 1) void decode_dma_kernel(
     if (tb0 + STEP < cf) issue(wb1, tb0 + STEP);
     if (fetch_len > 0) take_len();
     c1 = min(c0 + chunk, len);
+    if constexpr (TP) qprep.apply(tp, qa);
 
     u32x4 qh[NS], ql[NS];
 #pragma unroll
@@ -761,12 +845,12 @@ __global__ __launch_bounds__(MW * 64, 1) void decode_dma_kernel(
 // masks and partial layout as decode_dma_kernel (chunk = NB * KB).  KB = 16
 // (head_dim 256): a block is one 16-key tile, so a short context spreads
 // over twice the workgroups; the P^T operand's keys 16-31 are zero.
-template <class T, int D, int NB, int KB = kTok>
+template <class T, int D, int NB, int KB = kTok, bool TP = false>
 __global__ __launch_bounds__(64, 1) void decode_block_kernel(
     const float *__restrict__ q, const char *__restrict__ kc, const char *__restrict__ vc,
     int64_t kv_stride, int64_t seq_stride, const int32_t *__restrict__ seq_lens, int window,
     int fetch_len, int n_head, int kv_mul, int gt, int n_units, int chunk, int splits, float qscale,
-    float *__restrict__ out, float *__restrict__ ws_ml, float *__restrict__ ws_acc) {
+    float *__restrict__ out, float *__restrict__ ws_ml, float *__restrict__ ws_acc, TokenPrep tp) {
     constexpr int NS = D / 32;          // QK k-steps (32 d each)
     constexpr int NDT = D / 16;         // 16-wide d tiles of O^T
     // An f32 cache (the reference's) runs both contractions on bf16 MFMAs
@@ -828,6 +912,8 @@ __global__ __launch_bounds__(64, 1) void decode_block_kernel(
             qa[s][1] = *(const f32x4 *)(qp + (s * 4 + kg) * 8 + 4);
         }
     }
+    QPrep<D> qprep;
+    if constexpr (TP) qprep.load(tp, head0 + (head_ok ? n16 : 0), kg);
     const int nfb = min(max((cf - c0 + KB - 1) / KB, 0), NB);  // blocks fetched (uniform)
     {
         const int drow = lane / SLOTS, dslot = lane % SLOTS;
@@ -852,6 +938,7 @@ __global__ __launch_bounds__(64, 1) void decode_block_kernel(
     }
     if (fetch_len > 0) take_len();
     const int c1 = min(c0 + chunk, len);
+    if constexpr (TP) qprep.apply(tp, qa);
 
     u32x4 qh[NS], ql[NS];
 #pragma unroll
@@ -1062,10 +1149,37 @@ constexpr int kMaxSplits = 256;
 // cover the splits) or 256.
 constexpr int kMergeGroups = 4;
 // NML = (m, l) pairs per lane, ceil(splits / 64).
-template <int D, int NL, int NML, int MT>
+//
+// TOK: the split partials cover the keys before the token's own (old ones);
+// its q, k and v arrive raw.  Every wave prepares q and k of the workgroup's
+// head, the token's score joins the partials as one more (m, 1, v), and the
+// first head of each kv head stores the cache row.  k and v enter as the cache
+// holds them (rounded to its type).
+struct TokenStore {
+    TokenPrep t;
+    void *kc, *vc;  // the token's cache row
+    int dtype, kv_mul;
+    float qscale;
+};
+template <int E>
+__device__ __forceinline__ void round_to(int dtype, float (&x)[E]) {
+    if (dtype == ULLM_DT_F32) return;
+#pragma unroll
+    for (int i = 0; i < E; i++) {
+        const uint32_t w = dtype == ULLM_DT_F16 ? pack_f16x2(x[i], 0.f) : pack_bf16x2(x[i], 0.f);
+        x[i] = dtype == ULLM_DT_F16 ? f16_lo(w) : bf16_lo(w);
+    }
+}
+template <int E>
+__device__ __forceinline__ void store_as(int dtype, void *p, int64_t i, const float (&x)[E]) {
+    if (dtype == ULLM_DT_F32) store_e<ULLM_DT_F32, E>(p, i, x);
+    else if (dtype == ULLM_DT_F16) store_e<ULLM_DT_F16, E>(p, i, x);
+    else store_e<ULLM_DT_BF16, E>(p, i, x);
+}
+template <int D, int NL, int NML, int MT, bool TOK = false>
 __global__ __launch_bounds__(MT) void decode_merge_kernel(
     const float *__restrict__ ws_ml, const float *__restrict__ ws_acc, int splits, int gt,
-    int n_units, int n_head, float *__restrict__ out) {
+    int n_units, int n_head, float *__restrict__ out, TokenStore tk) {
     constexpr int kMergeThreads = MT;
     constexpr int NC = D / 4 / kMergeGroups, R = kMergeThreads / NC;
     static_assert(NML * 64 <= kMaxSplits, "merge reads at most kMaxSplits (m, l) pairs");
@@ -1093,10 +1207,46 @@ __global__ __launch_bounds__(MT) void decode_merge_kernel(
         ml[j] = mlu[(int64_t)min(sp, splits - 1) * gt];
         if (sp >= splits) ml[j] = float2{-INFINITY, 0.f};
     }
+    // The token's own score, and its v in this thread's columns.
+    float m_new = -INFINITY;
+    f32x4 v_new = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (TOK) {
+        constexpr int E = D / 64;
+        const int head = unit * gt + g, kvh = head / tk.kv_mul;
+        const HeadEpi<D> epi(tk.t.cs, 0, D, tk.t.neox, tk.t.qn, tk.t.kn, tk.t.eps);
+        float qv[E], kv[E];
+        load_e<E>(tk.t.q + head * D + epi.e0, qv);
+        load_e<E>(tk.t.k + kvh * D + epi.e0, kv);
+        float vr[4];
+        load_e<4>(tk.t.v + kvh * D + c4 * 4, vr);
+        if (tk.t.qb)
+#pragma unroll
+            for (int i = 0; i < E; i++) qv[i] += tk.t.qb[head * D + epi.e0 + i];
+        if (tk.t.kb)
+#pragma unroll
+            for (int i = 0; i < E; i++) kv[i] += tk.t.kb[kvh * D + epi.e0 + i];
+        if (tk.t.vb)
+#pragma unroll
+            for (int i = 0; i < 4; i++) vr[i] += tk.t.vb[kvh * D + c4 * 4 + i];
+        epi.norm_rope(qv, 0, nullptr);  // full-width RoPE: no LDS row
+        epi.norm_rope(kv, 1, nullptr);
+        round_to<E>(tk.dtype, kv);
+        round_to<4>(tk.dtype, vr);
+        float dot = 0.f;
+#pragma unroll
+        for (int i = 0; i < E; i++) dot += qv[i] * kv[i];
+        m_new = wave_sum(dot) * tk.qscale;
+        v_new = f32x4{vr[0], vr[1], vr[2], vr[3]};
+        if (head % tk.kv_mul == 0) {
+            if (cg == 0 && tid < 64) store_as<E>(tk.dtype, tk.kc, (int64_t)kvh * D + epi.e0, kv);
+            if (tid < NC) store_as<4>(tk.dtype, tk.vc, (int64_t)kvh * D + c4 * 4, vr);
+        }
+    }
     float mx = -INFINITY;
 #pragma unroll
     for (int j = 0; j < NML; j++) mx = fmaxf(mx, ml[j].x);
     mx = wave_max(mx);
+    if constexpr (TOK) mx = fmaxf(mx, m_new);
     const float mu = mx == -INFINITY ? 0.f : mx;
     f32x4 a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1114,6 +1264,11 @@ __global__ __launch_bounds__(MT) void decode_merge_kernel(
 #pragma unroll
         for (int j = 0; j < NML; j++) den += ml[j].y * __builtin_amdgcn_exp2f(ml[j].x - mu);
         den = wave_sum(den);
+        if constexpr (TOK) {
+            const float w = __builtin_amdgcn_exp2f(m_new - mu);
+            den += w;
+            a += v_new * w;
+        }
         const float inv = den > 0.f ? 1.0f / den : 0.f;
         if (lane < NC)
             *(f32x4 *)(out + ((int64_t)b * n_head + unit * gt + g) * D + c4 * 4) = a * inv;
@@ -1126,11 +1281,14 @@ __global__ __launch_bounds__(MT) void decode_merge_kernel(
 #pragma unroll
         for (int j = 0; j < NML; j++) den += ml[j].y * __builtin_amdgcn_exp2f(ml[j].x - mu);
         den = wave_sum(den);
+        const float w_new = TOK ? __builtin_amdgcn_exp2f(m_new - mu) : 0.f;
+        if constexpr (TOK) den += w_new;
         const float inv = den > 0.f ? 1.0f / den : 0.f;
         for (int c = lane; c < NC; c += 64) {
             f32x4 t = red[0][c];
 #pragma unroll
             for (int w = 1; w < kMergeThreads / 64; w++) t += red[w][c];
+            if constexpr (TOK) t += v_new * w_new;  // c == col: NC <= 64
             *(f32x4 *)(out + ((int64_t)b * n_head + unit * gt + g) * D + (cg * NC + c) * 4) =
                 t * inv;
         }
@@ -1251,11 +1409,11 @@ struct MainLaunch {
     template <class... A>
     static void run(int mw, dim3 g, hipStream_t st, A... a) {
         const int32_t *nt = nullptr;
-        if (mw == 1) hipLaunchKernelGGL((decode_dma_kernel<T, D, 1>), g, dim3(64), 0, st, a..., nt, 0, 0, 0);
+        if (mw == 1) hipLaunchKernelGGL((decode_dma_kernel<T, D, 1>), g, dim3(64), 0, st, a..., nt, 0, 0, 0, TokenPrep{});
         else if (mw == 2 || (__is_same(T, F32) && D == 128))  // f32 at head_dim 128: at most 2 waves
-            hipLaunchKernelGGL((decode_dma_kernel<T, D, 2>), g, dim3(128), 0, st, a..., nt, 0, 0, 0);
+            hipLaunchKernelGGL((decode_dma_kernel<T, D, 2>), g, dim3(128), 0, st, a..., nt, 0, 0, 0, TokenPrep{});
         else if constexpr (!(__is_same(T, F32) && D == 128))
-            hipLaunchKernelGGL((decode_dma_kernel<T, D, kMW>), g, dim3(kMW * 64), 0, st, a..., nt, 0, 0, 0);
+            hipLaunchKernelGGL((decode_dma_kernel<T, D, kMW>), g, dim3(kMW * 64), 0, st, a..., nt, 0, 0, 0, TokenPrep{});
     }
 };
 template <class T, int D>
@@ -1271,22 +1429,28 @@ struct MainLaunch<T, D, false> {
 };
 
 template <int D>
-static void launch_merge(const MfmaPlan &p, int batch, int nh, float *out, char *ws, hipStream_t st) {
+static void launch_merge(const MfmaPlan &p, int batch, int nh, float *out, char *ws, hipStream_t st,
+                         const TokenStore *tok = nullptr) {
     constexpr int NC = D / 4 / kMergeGroups;
     const dim3 g(p.gt * kMergeGroups, p.n_units, batch);
     const float *ml = (const float *)(ws + p.off_ml), *ac = (const float *)(ws + p.off_acc);
     // (m, l) loads per lane: as many as the splits need, not kMaxSplits / 64.
     auto go = [&](auto nlc, auto mtc) {
         constexpr int NL = decltype(nlc)::value, MT = decltype(mtc)::value;
-        if (p.splits <= 64)
-            hipLaunchKernelGGL((decode_merge_kernel<D, NL, 1, MT>), g, dim3(MT), 0, st, ml, ac,
-                               p.splits, p.gt, p.n_units, nh, out);
-        else if (p.splits <= 128)
-            hipLaunchKernelGGL((decode_merge_kernel<D, NL, 2, MT>), g, dim3(MT), 0, st, ml, ac,
-                               p.splits, p.gt, p.n_units, nh, out);
-        else
-            hipLaunchKernelGGL((decode_merge_kernel<D, NL, kMaxSplits / 64, MT>), g, dim3(MT), 0,
-                               st, ml, ac, p.splits, p.gt, p.n_units, nh, out);
+        auto kern = [&](auto nmlc) {
+            constexpr int NML = decltype(nmlc)::value;
+            if (tok) {
+                if constexpr (D <= 128)
+                    hipLaunchKernelGGL((decode_merge_kernel<D, NL, NML, MT, true>), g, dim3(MT), 0, st, ml, ac,
+                                       p.splits, p.gt, p.n_units, nh, out, *tok);
+            } else {
+                hipLaunchKernelGGL((decode_merge_kernel<D, NL, NML, MT>), g, dim3(MT), 0, st, ml, ac,
+                                   p.splits, p.gt, p.n_units, nh, out, TokenStore{});
+            }
+        };
+        if (p.splits <= 64) kern(Int<1>{});
+        else if (p.splits <= 128) kern(Int<2>{});
+        else kern(Int<kMaxSplits / 64>{});
     };
     // One wave (no LDS step) when 4 split rows per lane cover the splits;
     // with more, four waves keep the rows per lane, hence the serial loads,
@@ -1331,7 +1495,7 @@ static void launch_mfma(const MfmaPlan &p, const float *q, const void *kc, const
             hipLaunchKernelGGL((decode_block_kernel<T, D, 1, 16>), dim3(p.splits, p.n_units, batch),
                                dim3(64), 0, st, q, (const char *)kc, (const char *)vc, kvs, ss, lens,
                                win, fetch_len, nh, kv_mul, p.gt, p.n_units, p.chunk, p.splits, qs,
-                               out, (float *)(ws + p.off_ml), (float *)(ws + p.off_acc));
+                               out, (float *)(ws + p.off_ml), (float *)(ws + p.off_acc), TokenPrep{});
             launch_merge<D>(p, batch, nh, out, ws, st);
             return;
         }
@@ -1341,7 +1505,7 @@ static void launch_mfma(const MfmaPlan &p, const float *q, const void *kc, const
                 hipLaunchKernelGGL(kern, dim3(p.splits, p.n_units, batch), dim3(64), 0, st, q,
                                    (const char *)kc, (const char *)vc, kvs, ss, lens, win,
                                    fetch_len, nh, kv_mul, p.gt, p.n_units, p.chunk, p.splits, qs,
-                                   out, (float *)(ws + p.off_ml), (float *)(ws + p.off_acc));
+                                   out, (float *)(ws + p.off_ml), (float *)(ws + p.off_acc), TokenPrep{});
             };
             if (p.chunk == 2 * kTok) go(decode_block_kernel<T, D, 2>);
             else go(decode_block_kernel<T, D, 1>);
@@ -1405,6 +1569,78 @@ int decode_mfma(int dtype, const float *q, const void *kc, const void *vc, int64
     return check_hip(hipGetLastError(), "decode (mfma) launch");
 }
 
+// One decoded token of one sequence whose q, k and v are raw: the split kernels
+// prepare q and attend the old keys (positions before pos), and the merge adds
+// the token's own key and stores its cache row.  The append in a launch of its
+// own costs a launch and a round trip through memory on a latency-bound chain.
+// Measured (us of GPU per layer, three launches -> two): f32, 512 keys, 32/8 x 64
+// 9.26 -> 6.76; with the projection (bf16 2560 -> 6144, 3001 keys, 32/8 x 128, its
+// matvec without the head exchange) 19.4 -> 18.1.
+template <class T, int D>
+static void launch_token(const MfmaPlan &p, const TokenStore &tk, const char *kc, const char *vc, int64_t kvs,
+                         const int32_t *old_len, int max_len, int win, int nh, int kv_mul, float qs,
+                         float *out, char *ws, hipStream_t st) {
+    const int fetch_len = win <= 0 || max_len <= win ? max_len : 0;
+    const dim3 g(p.splits, p.n_units, 1);
+    float *ml = (float *)(ws + p.off_ml), *ac = (float *)(ws + p.off_acc);
+    auto block = [&](auto kern) {
+        hipLaunchKernelGGL(kern, g, dim3(64), 0, st, tk.t.q, kc, vc, kvs, (int64_t)0, old_len, win, fetch_len, nh,
+                           kv_mul, p.gt, p.n_units, p.chunk, p.splits, qs, out, ml, ac, tk.t);
+    };
+    auto dma = [&](auto mwc) {
+        constexpr int MW = decltype(mwc)::value;
+        hipLaunchKernelGGL((decode_dma_kernel<T, D, MW, false, true>), g, dim3(MW * 64), 0, st, tk.t.q, kc, vc, kvs,
+                           (int64_t)0, old_len, win, fetch_len, nh, kv_mul, p.gt, p.n_units, p.chunk, p.splits, qs,
+                           out, ml, ac, (const int32_t *)nullptr, 0, 0, 0, tk.t);
+    };
+    if (p.mw == 1 && p.chunk == kTok) block(decode_block_kernel<T, D, 1, kTok, true>);
+    else if (p.mw == 1 && p.chunk == 2 * kTok) block(decode_block_kernel<T, D, 2, kTok, true>);
+    else if (p.mw == 1) dma(Int<1>{});
+    else dma(Int<2>{});
+    launch_merge<D>(p, 1, nh, out, ws, st, &tk);
+}
+
+// The plan of the old keys in sight (positions before pos, less the one the
+// token takes of a window), and whether it is one of the fused shapes.
+static bool token_plan(int dtype, int pos, int win, int nh, int nkv, int D, MfmaPlan &p) {
+    if ((D != 64 && D != 128) || pos < 1 || win == 1) return false;
+    p = plan_mfma(1, nh, nkv, D, pos, win > 0 ? win - 1 : 0, false, dtype_bytes(dtype));
+    // One split writes the output itself, and four-wave workgroups are its form.
+    return p.splits >= 2 && p.mw <= 2;
+}
+
+size_t decode_token_bytes(int dtype, int pos, int win, int nh, int nkv, int D) {
+    MfmaPlan p;
+    return token_plan(dtype, pos, win, nh, nkv, D, p) ? p.bytes : 0;
+}
+
+bool decode_token_mfma(int dtype, const TokenPrep &t, void *kc, void *vc, int64_t kvs, const int32_t *old_len,
+                       int pos, int win, int nh, int nkv, int D, float qs, float *out, void *ws,
+                       size_t ws_bytes, hipStream_t st, int *rc) {
+    MfmaPlan p;
+    if (!token_plan(dtype, pos, win, nh, nkv, D, p) || !ws || ws_bytes < p.bytes) return false;
+    const int owin = win > 0 ? win - 1 : 0;
+    const int kv_mul = nh / nkv;
+    const int64_t row = (int64_t)pos * kvs * dtype_bytes(dtype);
+    const TokenStore tk{t, (char *)kc + row, (char *)vc + row, dtype, kv_mul, qs};
+#define ULLM_TOKEN(TT, DD) \
+    launch_token<TT, DD>(p, tk, (const char *)kc, (const char *)vc, kvs, old_len, pos, owin, nh, kv_mul, qs, out, \
+                         (char *)ws, st)
+    if (dtype == ULLM_DT_F32) {
+        if (D == 64) ULLM_TOKEN(F32, 64);
+        else ULLM_TOKEN(F32, 128);
+    } else if (dtype == ULLM_DT_F16) {
+        if (D == 64) ULLM_TOKEN(F16, 64);
+        else ULLM_TOKEN(F16, 128);
+    } else {
+        if (D == 64) ULLM_TOKEN(BF16, 64);
+        else ULLM_TOKEN(BF16, 128);
+    }
+#undef ULLM_TOKEN
+    *rc = check_hip(hipGetLastError(), "decode (token) launch");
+    return true;
+}
+
 }  // namespace ullm
 
 // ---------------------------------------------------------------------------
@@ -1444,7 +1680,7 @@ static void launch_paged(const MfmaPlan &p, const float *q, const void *kp, cons
                                (const char *)kp, (const char *)vp, kvs, (int64_t)0, lens, win, 0,
                                nh, kv_mul, p.gt, p.n_units, p.chunk, p.splits, qs, out,
                                (float *)(ws + p.off_ml), (float *)(ws + p.off_acc), tab,
-                               tab_stride, shift, n_pages);
+                               tab_stride, shift, n_pages, TokenPrep{});
         };
         if (p.mw == 1) go(Int<1>{});
         else if (p.mw == 2) go(Int<2>{});
@@ -1457,6 +1693,49 @@ static void launch_paged(const MfmaPlan &p, const float *q, const void *kp, cons
 }  // namespace ullm
 
 using namespace ullm;
+
+extern "C" size_t ullm_hip_decode_token_workspace_bytes(int kv_dtype, int pos, int window, int n_head,
+                                                       int n_kv_head, int head_dim, int rotary_dim) {
+    if (!dtype_ok(kv_dtype) || pos < 0 || n_head < 1 || n_kv_head < 1 || n_head % n_kv_head ||
+        rotary_dim != head_dim)
+        return 0;
+    return decode_token_bytes(kv_dtype, pos, window, n_head, n_kv_head, head_dim);
+}
+
+extern "C" int ullm_hip_decode_token(const float *q, const float *k, const float *v, const float *q_bias,
+                                     const float *k_bias, const float *v_bias, const float *q_norm,
+                                     const float *k_norm, float eps, const float *rope_cs, int rope_n_pos,
+                                     int rope_neox, int pos, const int32_t *old_len, int window, int n_head,
+                                     int n_kv_head, int head_dim, float scale, void *k_cache, void *v_cache,
+                                     int kv_dtype, int64_t kv_stride, float *out, void *workspace,
+                                     size_t workspace_bytes, void *stream) {
+    const size_t need = ullm_hip_decode_token_workspace_bytes(kv_dtype, pos, window, n_head, n_kv_head,
+                                                              head_dim, head_dim);
+    if (need == 0)
+        return set_error(ULLM_HIP_E_UNSUPPORTED, "decode_token: dtype %d, pos %d, window %d, %d/%d heads x %d",
+                         kv_dtype, pos, window, n_head, n_kv_head, head_dim);
+    if (kv_stride < (int64_t)n_kv_head * head_dim || (kv_stride * dtype_bytes(kv_dtype)) % 16)
+        return set_error(ULLM_HIP_E_INVALID, "decode_token: kv_stride must be >= n_kv_head*head_dim and 16-byte aligned");
+    if (rope_n_pos <= pos)
+        return set_error(ULLM_HIP_E_INVALID, "decode_token: rope table has %d positions, need %d", rope_n_pos, pos + 1);
+    if (((int64_t)pos + 1) * kv_stride * dtype_bytes(kv_dtype) > 0x7fff0000LL)
+        return set_error(ULLM_HIP_E_INVALID, "decode_token: a layer's cache exceeds 2 GiB");
+    if (!q || !k || !v || !rope_cs || !old_len || !k_cache || !v_cache || !out)
+        return set_error(ULLM_HIP_E_INVALID, "decode_token: null tensor pointer");
+    const void *al[] = {q, k, v, q_bias, k_bias, v_bias, q_norm, k_norm, rope_cs, k_cache, v_cache, out};
+    for (const void *a : al)
+        if ((uintptr_t)a & 15) return set_error(ULLM_HIP_E_INVALID, "decode_token: tensors must be 16-byte aligned");
+    if (!workspace || workspace_bytes < need)
+        return set_error(ULLM_HIP_E_WORKSPACE, "decode_token: workspace of %zu bytes needed, %zu given", need,
+                         workspace_bytes);
+    const TokenPrep t{q, k, v, q_bias, k_bias, v_bias, q_norm, k_norm, rope_cs + (int64_t)pos * head_dim,
+                      eps, rope_neox};
+    int rc = ULLM_HIP_OK;
+    if (!decode_token_mfma(kv_dtype, t, k_cache, v_cache, kv_stride, old_len, pos, window, n_head, n_kv_head,
+                           head_dim, scale * kLog2e, out, workspace, workspace_bytes, (hipStream_t)stream, &rc))
+        return set_error(ULLM_HIP_E_UNSUPPORTED, "decode_token: shape");
+    return rc;
+}
 
 extern "C" size_t ullm_hip_paged_decode_workspace_bytes(int batch, int n_head, int n_kv_head,
                                                         int head_dim, int max_len, int window) {

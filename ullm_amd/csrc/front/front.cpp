@@ -405,17 +405,45 @@ at::Tensor token(const Args &a) {
     const Layer l(kc, vc, layer);
     void *s = (void *)c10::hip::getCurrentHIPStream().stream();
     const int64_t row = (int64_t)p.H * p.D, kvs = (int64_t)p.hk * p.D;
-    const at::Tensor q = at::empty({1, row}, x.options().dtype(at::kFloat));
-    if (is_proj) {
-        const at::Tensor &w2 = a.t(R + 3);
-        need_cuda({&x, &w0, &w1, &w2, &kc, &vc, &p.cs});
-        proj_check(x, w0, w1, w2, x.numel(), p);
-        proj_call(x, w0, w1, w2, x.numel(), p, 1, pos, q, l.k, l.v, l.kd, kvs, a.ot(R + 4), s);
-    } else {
-        need_cuda({&x, &w0, &w1, &kc, &vc, &p.cs});
-        if (!f32_rows(x) || !f32_rows(w0) || !f32_rows(w1)) invalid("q/k/v must be contiguous f32");
-        append_call(x, w0, w1, p, 1, pos, q, l.k, l.v, l.kd, kvs, s);
+    const at::Tensor *w2 = is_proj ? &a.t(R + 3) : nullptr;
+    need_cuda({&x, &w0, &w1, w2, &kc, &vc, &p.cs});
+    if (is_proj) proj_check(x, w0, w1, *w2, x.numel(), p);
+    else if (!f32_rows(x) || !f32_rows(w0) || !f32_rows(w1)) invalid("q/k/v must be contiguous f32");
+    // Append and attention in the attention's two launches, where the shape and
+    // the alignment allow it; whatever is refused below is refused there too.
+    const auto odd = [](const void *q) { return ((uintptr_t)q & 15) != 0; };
+    const size_t need = ullm_hip_decode_token_workspace_bytes(l.kd, pos, win, p.H, p.hk, p.D, p.rd);
+    bool fuse = need && ws.numel() >= (int64_t)need && pos < p.cs.size(0) && kvs * (int64_t)kc.element_size() % 16 == 0 &&
+                ((int64_t)pos + 1) * kvs * (int64_t)kc.element_size() <= 0x7fff0000LL;
+    const void *used[] = {l.k, l.v, ptr(&p.cs), ptr(p.qb), ptr(p.kb), ptr(p.vb), ptr(p.qn), ptr(p.kn), ptr(&x),
+                          ptr(&w0), ptr(&w1), ptr(w2)};
+    for (const void *q : used)
+        fuse = fuse && !odd(q);
+    if (is_proj) fuse = fuse && x.numel() >= 8 && x.numel() % 8 == 0;
+    if (fuse) {
+        const float *q = fptr(&x), *k = fptr(&w0), *v = fptr(&w1);
+        at::Tensor y;
+        if (is_proj) {
+            y = at::empty({row + 2 * kvs}, x.options().dtype(at::kFloat));
+            const int wd = dt(w0);
+            call([&] {
+                return ullm_hip_qkv_matvec(fptr(&x), (int)x.numel(), w0.data_ptr(), w1.data_ptr(), w2->data_ptr(), wd,
+                                           p.H, p.hk, p.D, (float *)y.data_ptr(), s);
+            });
+            q = fptr(&y), k = q + row, v = k + kvs;
+        }
+        const at::Tensor out = at::empty({row}, x.options().dtype(at::kFloat));
+        call([&] {
+            return ullm_hip_decode_token(q, k, v, fptr(p.qb), fptr(p.kb), fptr(p.vb), fptr(p.qn), fptr(p.kn), p.eps,
+                                         fptr(&p.cs), (int)p.cs.size(0), p.neox, pos,
+                                         (const int32_t *)lens.data_ptr() + pos - 1, win, p.H, p.hk, p.D, scale, l.k,
+                                         l.v, l.kd, kvs, (float *)out.data_ptr(), ws.data_ptr(), ws.numel(), s);
+        });
+        return out;
     }
+    const at::Tensor q = at::empty({1, row}, x.options().dtype(at::kFloat));
+    if (is_proj) proj_call(x, w0, w1, *w2, x.numel(), p, 1, pos, q, l.k, l.v, l.kd, kvs, a.ot(R + 4), s);
+    else append_call(x, w0, w1, p, 1, pos, q, l.k, l.v, l.kd, kvs, s);
     const at::Tensor out = at::empty({row}, q.options());
     call([&] {
         return ullm_hip_attn_decode(fptr(&q), l.k, l.v, l.kd, kvs, 0, (const int32_t *)lens.data_ptr() + pos, pos + 1,
