@@ -30,10 +30,10 @@ def _f64(q, k, v, rows, head, kvh, D, start, window):
 @pytest.mark.parametrize("dt,S,start,window,H,Hk,D", [
     ("bf16", 1, 4095, 0, 32, 8, 128), ("f16", 33, 3001, 0, 12, 4, 128), ("bf16", 129, 2000, 0, 32, 4, 128),
     ("f16", 8, 20000, 0, 8, 1, 128), ("bf16", 65, 4030, 0, 16, 16, 64), ("f16", 31, 6017, 0, 32, 8, 64),
-    ("f32", 1, 4000, 0, 32, 8, 64), ("f32", 130, 3000, 0, 6, 2, 64), ("f32", 127, 208, 0, 32, 8, 64),
+    ("f32", 1, 4000, 0, 32, 8, 64), ("f32", 130, 3000, 0, 6, 2, 64), ("f32", 250, 300, 0, 6, 2, 64),
     ("f32", 40, 5000, 700, 32, 8, 64), ("f32", 17, 3333, 0, 32, 8, 128), ("f32", 100, 4000, 1500, 8, 8, 128),
     ("f16", 45, 5605, 0, 8, 4, 256), ("bf16", 5, 13493, 1024, 8, 4, 256), ("f32", 70, 2222, 0, 8, 4, 256),
-    ("f32", 898, 0, 0, 12, 2, 128), ("f32", 334, 0, 0, 16, 16, 64), ("f32", 217, 22, 1024, 8, 4, 256),
+    ("f32", 898, 0, 0, 12, 2, 128), ("f32", 217, 22, 1024, 8, 4, 256),
 ])
 @pytest.mark.parametrize("paged", [False, True])
 def test_split_matches_unsplit_and_f64(dev, dt, S, start, window, H, Hk, D, paged):
@@ -88,3 +88,24 @@ def test_small_workspace_runs_unsplit(dev):
             1 / math.sqrt(D), A._ptr(out), A._ptr(ws), 0 if ws is None else n - 1, A._stream()))
         outs.append(out)
     assert torch.equal(*outs)
+
+
+# The f32 head_dim-64 kernel unsplit: one set of waves (4 key tiles at most, or
+# short windows on a full chip) and two, with 5 and odd tile counts, units whose
+# second set has a tile less, and rows before the second set's keys.
+@pytest.mark.parametrize("S,start,window,H,Hk", [(1, 0, 0, 8, 2), (127, 0, 0, 8, 8), (129, 0, 0, 4, 1), (161, 3, 0, 32, 8),
+                                                 (777, 0, 0, 32, 8), (300, 0, 90, 6, 2), (2000, 0, 300, 32, 8)])
+def test_f32_sets(dev, S, start, window, H, Hk):
+    D = 64
+    print(f"[prefill-f32-sets] S{S} start{start} win{window} {H}/{Hk}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(S)
+    q = torch.randn(S, H * D, device=dev, generator=g)
+    k, v = (torch.randn(start + S, Hk * D, device=dev, generator=g) for _ in range(2))
+    out = torch.empty(S, H * D, device=dev)
+    L.check(L.lib().ullm_hip_attn_prefill(A._ptr(q), A._ptr(k), A._ptr(v), L.DT_F32, Hk * D, S, start, window, H,
+                                          Hk, D, 1 / math.sqrt(D), A._ptr(out), A._stream()))
+    rows = list(range(0, S, max(1, S // 150))) + [S - 1]
+    for h in (0, H - 1):
+        ref = _f64(q, k, v, rows, h, h // (H // Hk), D, start, window)
+        got = out[rows, h * D:(h + 1) * D].double()
+        assert float((got - ref).norm() / ref.norm()) <= 1e-3

@@ -1220,16 +1220,21 @@ static SplitPlan prefill4_split(int S, int sp, int nh, int kv_mul, int D) {
     return choose_split(c, u, unsplit, S, nh, D);
 }
 
-// prefill_f32_kernel's split (a unit per workgroup, or less).  Per 32-key tile,
-// 32/8 heads x 64: 777 rows (200 units) 29.6 us for 25 tiles; 500 rows at 4000 in
-// 2 parts (256 workgroups) 82.9, in 4 60.7.  Measured (us, pairs of units per
-// workgroup -> a unit each -> this rule's split): 777 rows 33.9 -> 29.6 -> 27.1,
-// 500 at 4000 256 -> 140 -> 61, 61 at 700 52 -> 27 -> 13, 2048 rows 80 -> 71, 4096
-// rows 216 -> 211, 2000 rows with window 300 35 -> 28.
+// prefill_f32_kernel's split (a unit per workgroup, or less) and sets.  Two sets
+// cost 0.6 us per 32-key tile (32/8 heads x 64: 777 rows, 25 tiles, 21.1 us; 500
+// rows at 4000, 141 tiles, 84), one set 1.0; with more workgroups than CUs two
+// one-set workgroups share one and start their next unit on their own, which
+// is better for short units: 2000 rows, window 300 (504 units of 13 tiles) 27.7
+// us against 32.5, 100 rows (4 tiles) 8.2 against 9.1.  Measured (us, causal
+// pairs of units on one set -> this rule): 777 rows 33.9 -> 21.1, 1000 41.5 -> 24.9,
+// 2048 80 -> 57, 4096 216 -> 195, 500 at 4000 256 -> 55, 61 at 700 52 -> 13.
+static bool prefill_f32_two_sets(double wgs, double longest) {
+    return longest > (wgs > 256 ? 16 : 4);
+}
 static SplitPlan prefill_f32_split(int S, int sp, int win, int nh, int kv_mul, int D) {
     int hw = 1;
     while (hw < 4 && kv_mul % (hw * 2) == 0) hw *= 2;
-    return choose_split(PrefillCost{1.0, .9, 5.}, unit_load(S, 128 / hw, nh / hw, sp, win, 32), 0., S, nh, D);
+    return choose_split(PrefillCost{.58, .66, 6.}, unit_load(S, 128 / hw, nh / hw, sp, win, 32), 0., S, nh, D);
 }
 
 template <class T, int D>
@@ -1304,7 +1309,9 @@ static int launch_prefill(const void *q, const void *kc, const void *vc, int64_t
 // at most 4) times 4/hw consecutive 32-row blocks: one "unit" of
 // UR = 128/hw rows; wave w takes head hw0 + w % hw and rows (w / hw) * 32 ..
 // +31 of the unit.  A unit, or one part of its key tiles (KeySplit, max_parts
-// at most), is one workgroup; up to two fit a CU.  (Causal pairs of units per
+// at most), is one workgroup of one set of 4 waves, or of two sets that take
+// half of its tiles each (every SIMD then has two waves, one converting or in
+// its softmax while the other multiplies) and merge through LDS.  (Causal pairs of units per
 // workgroup, which balance the keys, were slower at every size: 777 rows of
 // 32/8 heads x 64 33.9 against 29.6 us, 4096 rows 216 against 211, 61 rows at 700
 // 52 against 27.)  Each tile is loaded and converted once for all 4 waves:
@@ -1321,8 +1328,8 @@ static int launch_prefill(const void *q, const void *kc, const void *vc, int64_t
 // block of one head per workgroup with the 4 waves splitting its keys (each
 // wave streaming and converting its own tiles) took 1.6x as long at 2048 rows
 // of 32/8 heads x 128.
-template <int D, int NRAW = 2>
-__global__ __launch_bounds__(256, 1) void prefill_f32_kernel(
+template <int D, int SETS = 1, int NRAW = 2>
+__global__ __launch_bounds__(256 * SETS, 1) void prefill_f32_kernel(
     const float *__restrict__ q, const float *__restrict__ kc, const float *__restrict__ vc,
     int64_t kv_stride, int S, int start_pos, int window, int n_head, int kv_mul, int hw,
     int n_units, int max_parts, float qscale, float *__restrict__ out, KvPages pgs, KeySplit sp) {
@@ -1336,9 +1343,12 @@ __global__ __launch_bounds__(256, 1) void prefill_f32_kernel(
     constexpr float kLazy = 8.0f;
     static_assert(D == 64 || D == 128, "f32 prefill serves head_dim 64 and 128");
     auto swz = [](int r) { return kv_swz<D>(r); };
-    __shared__ __attribute__((aligned(1024))) char lds[NSTG * STAGE];
+    __shared__ __attribute__((aligned(1024))) char lds[SETS * NSTG * STAGE];
+    static_assert(SETS == 1 || 4 * 64 * NDT * 16 * 4 <= NSTG * STAGE, "the merge's staging");
+    __shared__ float2 hand_ml[4][32];
 
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int set = SETS == 2 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+    const int tid = threadIdx.x & 255, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 31, h2 = lane >> 5;
     // Task: (head group, unit, part), a head group's on one XCD's L2.
@@ -1359,7 +1369,9 @@ __global__ __launch_bounds__(256, 1) void prefill_f32_kernel(
     unit_tiles(u, UR, S, start_pos, window, BN, a0, a1);
     const int parts = part_tiles(sp, kpart, a0, a1);
     if (kpart >= parts) return;
-    const int nsteps = a1 - a0;
+    const int nmax = (a1 - a0 + SETS - 1) / SETS;  // steps of set 0, at least set 1's
+    const int nsteps = set ? a1 - a0 - nmax : nmax;
+    if (set) a0 += nmax;
 
     const int rbg = (int)(kv_stride * 4);
     const int range = (kv_len - 1) * rbg + D * 4;
@@ -1395,7 +1407,7 @@ __global__ __launch_bounds__(256, 1) void prefill_f32_kernel(
             vr[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(vq, off, 0, 0));
         }
     };
-    const uint32_t lds0 = lds_addr(lds);
+    const uint32_t lds0 = lds_addr(lds) + set * NSTG * STAGE;
     // Chunk i of the thread's share (one K and one V chunk).
     auto convert1 = [&](const u32x4(&kr)[NCH], const u32x4(&vr)[NCH], int stg, int i) {
         const uint32_t sb = lds0 + stg * STAGE;
@@ -1459,8 +1471,7 @@ __global__ __launch_bounds__(256, 1) void prefill_f32_kernel(
         l_part = 0.f;
     };
     // O^T in registers: lane (row c, h2) holds d = dt*32 + 8g + 4*h2 + 0..3.
-    auto end_unit = [&]() {
-        const float l_tot = l_part + xor32(l_part);
+    auto end_unit = [&](float l_tot) {
         const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
         if (parts > 1) {  // left for the merge
             if (qrow >= S) return;
@@ -1616,11 +1627,44 @@ __global__ __launch_bounds__(256, 1) void prefill_f32_kernel(
     // that skipped the second half's requests would make every wait at the
     // loop head drain all of them); only the compute of a step past the end
     // is skipped.
-    for (int j = 0; j < nsteps; j += 2) {
-        step(Int<1>{}, j, true);
+    for (int j = 0; j < nmax; j += 2) {
+        step(Int<1>{}, j, j < nsteps);
         step(Int<0>{}, j + 1, j + 1 < nsteps);
     }
-    end_unit();
+    float l_tot = l_part + xor32(l_part);
+    if constexpr (SETS == 1) return end_unit(l_tot);
+    // Merge the sets' partials of each row: set 1's through its idle stages.
+    const uint32_t po = lds_addr(lds) + NSTG * STAGE + (wave * 64 + lane) * 16;
+    if (set) {
+        if (h2 == 0) hand_ml[wave][c] = float2{m_run, l_tot};
+#pragma unroll
+        for (int i = 0; i < NDT * 4; i++)
+            lds_write_b128(po + i * 4 * 64 * 16,
+                           __builtin_bit_cast(u32x4, f32x4{oacc[i >> 2][(i & 3) * 4], oacc[i >> 2][(i & 3) * 4 + 1],
+                                                           oacc[i >> 2][(i & 3) * 4 + 2], oacc[i >> 2][(i & 3) * 4 + 3]}));
+    }
+    lds_wait_any();
+    __syncthreads();
+    if (set) return;
+    {
+        const float2 o = hand_ml[wave][c];
+        const float M = fmaxf(m_run, o.x), mu = M == -INFINITY ? 0.f : M;
+        const float e0 = __builtin_amdgcn_exp2f(m_run - mu), e1 = __builtin_amdgcn_exp2f(o.x - mu);
+        l_tot = l_tot * e0 + o.y * e1;
+        m_run = M;
+#pragma unroll
+        for (int i = 0; i < NDT * 4; i++) {
+            u32x4 r = lds_read_b128(po + i * 4 * 64 * 16);
+            lds_wait_any();
+            tie(r);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float x = oacc[i >> 2][(i & 3) * 4 + e];
+                oacc[i >> 2][(i & 3) * 4 + e] = x * e0 + __uint_as_float(r[e]) * e1;
+            }
+        }
+    }
+    end_unit(l_tot);
 }
 
 template <int D>
@@ -1634,9 +1678,14 @@ static int launch_prefill_f32(const void *q, const void *kc, const void *vc, int
     if (!ws.p || ws.bytes < pl.bytes) pl = SplitPlan{INT_MAX / 2, 1, 0, 0};
     const KeySplit ksp = split_at(pl, 32, ws.p);
     const int per_xcd = (nh / hw * n_units * pl.parts + 7) / 8;
-    hipLaunchKernelGGL((prefill_f32_kernel<D>), dim3(per_xcd * 8), dim3(256), 0, st,
-                       (const float *)q, (const float *)kc, (const float *)vc, kvs, S, sp, win,
-                       nh, kv_mul, hw, n_units, pl.parts, qs, out, pgs, ksp);
+    auto go = [&](auto kern, int threads) {
+        hipLaunchKernelGGL(kern, dim3(per_xcd * 8), dim3(threads), 0, st, (const float *)q, (const float *)kc,
+                           (const float *)vc, kvs, S, sp, win, nh, kv_mul, hw, n_units, pl.parts, qs, out, pgs, ksp);
+    };
+    const UnitLoad u = unit_load(S, 128 / hw, nh / hw, sp, win, 32);
+    if (D == 64 && prefill_f32_two_sets(u.n * pl.parts, std::min((double)pl.chunk, u.longest)))
+        go(prefill_f32_kernel<64, 2>, 512);  // (head_dim 128 would spill)
+    else go(prefill_f32_kernel<D>, 256);
     if (pl.parts > 1) return launch_prefill_merge(D, ksp, 128 / hw, S, sp, win, nh, out, st);
     return check_hip(hipGetLastError(), "prefill (f32) launch");
 }
