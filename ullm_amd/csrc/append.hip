@@ -448,7 +448,7 @@ static void launch_kv(int kvdt, dim3 g, dim3 b, hipStream_t st, const float *qi,
                       int rd, int rows, int sp, int nh, int nkv, void *qo, void *kc, void *vc,
                       int64_t kvs, PageMap pm, int gpw, AppendSrc as) {
     auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, g, b, 0, st, qi, ki, vi, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, pm, gpw, as);
+        launch_kernel(kern, g, b, 0, st, qi, ki, vi, qb, kb, vb, qn, kn, eps, cs, neox, rd, rows, sp, nh, nkv, qo, kc, vc, kvs, pm, gpw, as);
     };
     auto pick = [&](auto kvc) {
         constexpr int KVDT = decltype(kvc)::value;
@@ -688,7 +688,7 @@ int launch_qkv_matvec(const float *x, int in_dim, const void *wq, const void *wk
     if (env >= 1 && env <= 4) best = env;
     auto go = [&](auto wdt, auto rpw) {
         constexpr int WDT = decltype(wdt)::value, R = decltype(rpw)::value;
-        hipLaunchKernelGGL((qkv_matvec_kernel<WDT, R>), dim3((n + kMvWaves * R - 1) / (kMvWaves * R)),
+        launch_kernel((qkv_matvec_kernel<WDT, R>), dim3((n + kMvWaves * R - 1) / (kMvWaves * R)),
                            dim3(kMvWaves * 64), 0, st, x, in_dim, (const char *)wq, (const char *)wk,
                            (const char *)wv, n_q, n_kv, n, y);
     };
@@ -732,7 +732,7 @@ static void launch_proj(bool split, int rows, hipStream_t st, const ProjArgs &a)
     const int slots = a.nh + 2 * a.nkv;
     auto go = [&](auto nspc) {
         constexpr int NSP = decltype(nspc)::value;
-        hipLaunchKernelGGL((qkv_proj_kernel<D, WDT, QDT, KVDT, NSP>),
+        launch_kernel((qkv_proj_kernel<D, WDT, QDT, KVDT, NSP>),
                            dim3((unsigned)(slots * NSP), (unsigned)rows), dim3(proj_waves(NSP) * 64), 0, st,
                            a.x, a.in_dim, a.wq, a.wk, a.wv, a.qb, a.kb, a.vb, a.qn, a.kn, a.eps, a.cs,
                            a.neox, a.rd, a.sp, a.nh, a.nkv, a.qo, a.kc, a.vc, a.kvs, a.ws_y, a.ws_cnt);

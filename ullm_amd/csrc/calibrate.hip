@@ -35,7 +35,7 @@ extern "C" int ullm_hip_stream_read(const void *src, size_t bytes, int workgroup
     if (!src || !sink || bytes < 16 || workgroups < 1 || ((uintptr_t)src & 15))
         return set_error(ULLM_HIP_E_INVALID, "stream_read: bad arguments");
     const int64_t n16 = (int64_t)(bytes / 16);
-    hipLaunchKernelGGL(stream_read_kernel, dim3(workgroups), dim3(256), 0, (hipStream_t)stream,
+    launch_kernel(stream_read_kernel, dim3(workgroups), dim3(256), 0, (hipStream_t)stream,
                        (const u32x4 *)src, n16, sink);
     return check_hip(hipGetLastError(), "stream_read launch");
 }

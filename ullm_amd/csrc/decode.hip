@@ -318,7 +318,7 @@ static void launch_decode(const DecodePlan &p, const float *q, const void *kc, c
     dim3 grid(p.splits, p.n_groups, batch);
     const int kpl = (p.chunk + p.nlg - 1) / p.nlg;  // keys per lane group
 #define ULLM_SPLIT(TTK)                                                                        \
-    hipLaunchKernelGGL((decode_split_kernel<T, D, G, TTK>), grid, dim3(kDecodeWaves * 64), 0, st, \
+    launch_kernel((decode_split_kernel<T, D, G, TTK>), grid, dim3(kDecodeWaves * 64), 0, st, \
                        q, (const char *)kc, (const char *)vc, kv_stride, seq_stride, lens,      \
                        window, n_head, kv_mul, p.n_groups, p.chunk, p.splits, qscale, out,      \
                        (float *)(ws + p.off_ml), (float *)(ws + p.off_acc), kp)

@@ -1409,11 +1409,11 @@ struct MainLaunch {
     template <class... A>
     static void run(int mw, dim3 g, hipStream_t st, A... a) {
         const int32_t *nt = nullptr;
-        if (mw == 1) hipLaunchKernelGGL((decode_dma_kernel<T, D, 1>), g, dim3(64), 0, st, a..., nt, 0, 0, 0, TokenPrep{});
+        if (mw == 1) launch_kernel((decode_dma_kernel<T, D, 1>), g, dim3(64), 0, st, a..., nt, 0, 0, 0, TokenPrep{});
         else if (mw == 2 || (__is_same(T, F32) && D == 128))  // f32 at head_dim 128: at most 2 waves
-            hipLaunchKernelGGL((decode_dma_kernel<T, D, 2>), g, dim3(128), 0, st, a..., nt, 0, 0, 0, TokenPrep{});
+            launch_kernel((decode_dma_kernel<T, D, 2>), g, dim3(128), 0, st, a..., nt, 0, 0, 0, TokenPrep{});
         else if constexpr (!(__is_same(T, F32) && D == 128))
-            hipLaunchKernelGGL((decode_dma_kernel<T, D, kMW>), g, dim3(kMW * 64), 0, st, a..., nt, 0, 0, 0, TokenPrep{});
+            launch_kernel((decode_dma_kernel<T, D, kMW>), g, dim3(kMW * 64), 0, st, a..., nt, 0, 0, 0, TokenPrep{});
     }
 };
 template <class T, int D>
@@ -1422,9 +1422,9 @@ struct MainLaunch<T, D, false> {
     static void run(int mw, dim3 g, hipStream_t st, A... a) {
         const int32_t *nt = nullptr;
         if (mw == 1)
-            hipLaunchKernelGGL((decode_mfma_kernel<T, D, false, 1>), g, dim3(64), 0, st, a..., nt, 0, 0, 0);
+            launch_kernel((decode_mfma_kernel<T, D, false, 1>), g, dim3(64), 0, st, a..., nt, 0, 0, 0);
         else
-            hipLaunchKernelGGL((decode_mfma_kernel<T, D>), g, dim3(kMW * 64), 0, st, a..., nt, 0, 0, 0);
+            launch_kernel((decode_mfma_kernel<T, D>), g, dim3(kMW * 64), 0, st, a..., nt, 0, 0, 0);
     }
 };
 
@@ -1441,10 +1441,10 @@ static void launch_merge(const MfmaPlan &p, int batch, int nh, float *out, char 
             constexpr int NML = decltype(nmlc)::value;
             if (tok) {
                 if constexpr (D <= 128)
-                    hipLaunchKernelGGL((decode_merge_kernel<D, NL, NML, MT, true>), g, dim3(MT), 0, st, ml, ac,
+                    launch_kernel((decode_merge_kernel<D, NL, NML, MT, true>), g, dim3(MT), 0, st, ml, ac,
                                        p.splits, p.gt, p.n_units, nh, out, *tok);
             } else {
-                hipLaunchKernelGGL((decode_merge_kernel<D, NL, NML, MT>), g, dim3(MT), 0, st, ml, ac,
+                launch_kernel((decode_merge_kernel<D, NL, NML, MT>), g, dim3(MT), 0, st, ml, ac,
                                    p.splits, p.gt, p.n_units, nh, out, TokenStore{});
             }
         };
@@ -1492,7 +1492,7 @@ static void launch_mfma(const MfmaPlan &p, const float *q, const void *kc, const
     const int fetch_len = batch == 1 && (win <= 0 || max_len <= win) ? max_len : 0;
     if constexpr (D > 128) {
         if (p.kb == 16) {
-            hipLaunchKernelGGL((decode_block_kernel<T, D, 1, 16>), dim3(p.splits, p.n_units, batch),
+            launch_kernel((decode_block_kernel<T, D, 1, 16>), dim3(p.splits, p.n_units, batch),
                                dim3(64), 0, st, q, (const char *)kc, (const char *)vc, kvs, ss, lens,
                                win, fetch_len, nh, kv_mul, p.gt, p.n_units, p.chunk, p.splits, qs,
                                out, (float *)(ws + p.off_ml), (float *)(ws + p.off_acc), TokenPrep{});
@@ -1502,7 +1502,7 @@ static void launch_mfma(const MfmaPlan &p, const float *q, const void *kc, const
     } else {
         if (p.mw == 1 && (p.chunk == kTok || p.chunk == 2 * kTok) && p.splits > 1 && !kNoBlock) {
             auto go = [&](auto kern) {
-                hipLaunchKernelGGL(kern, dim3(p.splits, p.n_units, batch), dim3(64), 0, st, q,
+                launch_kernel(kern, dim3(p.splits, p.n_units, batch), dim3(64), 0, st, q,
                                    (const char *)kc, (const char *)vc, kvs, ss, lens, win,
                                    fetch_len, nh, kv_mul, p.gt, p.n_units, p.chunk, p.splits, qs,
                                    out, (float *)(ws + p.off_ml), (float *)(ws + p.off_acc), TokenPrep{});
@@ -1584,12 +1584,12 @@ static void launch_token(const MfmaPlan &p, const TokenStore &tk, const char *kc
     const dim3 g(p.splits, p.n_units, 1);
     float *ml = (float *)(ws + p.off_ml), *ac = (float *)(ws + p.off_acc);
     auto block = [&](auto kern) {
-        hipLaunchKernelGGL(kern, g, dim3(64), 0, st, tk.t.q, kc, vc, kvs, (int64_t)0, old_len, win, fetch_len, nh,
+        launch_kernel(kern, g, dim3(64), 0, st, tk.t.q, kc, vc, kvs, (int64_t)0, old_len, win, fetch_len, nh,
                            kv_mul, p.gt, p.n_units, p.chunk, p.splits, qs, out, ml, ac, tk.t);
     };
     auto dma = [&](auto mwc) {
         constexpr int MW = decltype(mwc)::value;
-        hipLaunchKernelGGL((decode_dma_kernel<T, D, MW, false, true>), g, dim3(MW * 64), 0, st, tk.t.q, kc, vc, kvs,
+        launch_kernel((decode_dma_kernel<T, D, MW, false, true>), g, dim3(MW * 64), 0, st, tk.t.q, kc, vc, kvs,
                            (int64_t)0, old_len, win, fetch_len, nh, kv_mul, p.gt, p.n_units, p.chunk, p.splits, qs,
                            out, ml, ac, (const int32_t *)nullptr, 0, 0, 0, tk.t);
     };
@@ -1662,13 +1662,13 @@ static void launch_paged(const MfmaPlan &p, const float *q, const void *kp, cons
     const dim3 g(p.splits, p.n_units, batch);
     if constexpr (D > 128) {  // register-staged kernel, 4 waves
         if (p.mw == 1)
-            hipLaunchKernelGGL((decode_mfma_kernel<T, D, true, 1>), g, dim3(64), 0, st, q,
+            launch_kernel((decode_mfma_kernel<T, D, true, 1>), g, dim3(64), 0, st, q,
                                (const char *)kp, (const char *)vp, kvs, (int64_t)0, lens, win, 0,
                                nh, kv_mul, p.gt, p.n_units, p.chunk, p.splits, qs, out,
                                (float *)(ws + p.off_ml), (float *)(ws + p.off_acc), tab,
                                tab_stride, shift, n_pages);
         else
-            hipLaunchKernelGGL((decode_mfma_kernel<T, D, true>), g, dim3(kMW * 64), 0, st, q,
+            launch_kernel((decode_mfma_kernel<T, D, true>), g, dim3(kMW * 64), 0, st, q,
                                (const char *)kp, (const char *)vp, kvs, (int64_t)0, lens, win, 0,
                                nh, kv_mul, p.gt, p.n_units, p.chunk, p.splits, qs, out,
                                (float *)(ws + p.off_ml), (float *)(ws + p.off_acc), tab,
@@ -1676,7 +1676,7 @@ static void launch_paged(const MfmaPlan &p, const float *q, const void *kp, cons
     } else {
         auto go = [&](auto mwc) {
             constexpr int MW = decltype(mwc)::value;
-            hipLaunchKernelGGL((decode_dma_kernel<T, D, MW, true>), g, dim3(MW * 64), 0, st, q,
+            launch_kernel((decode_dma_kernel<T, D, MW, true>), g, dim3(MW * 64), 0, st, q,
                                (const char *)kp, (const char *)vp, kvs, (int64_t)0, lens, win, 0,
                                nh, kv_mul, p.gt, p.n_units, p.chunk, p.splits, qs, out,
                                (float *)(ws + p.off_ml), (float *)(ws + p.off_acc), tab,

@@ -267,7 +267,7 @@ static void launch_mm(const char *w, const float *x, float *y, int in_dim, int o
     using C = MmCfg<SI, OI, WS, WO>;
     const int mt = (n + C::BS - 1) / C::BS, nt = (out_dim + C::BO - 1) / C::BO;
     const int per_xcd = (mt * nt + 7) / 8;
-    hipLaunchKernelGGL((matmul_bf16_kernel<SI, OI, WS, WO>), dim3(per_xcd * 8), dim3(C::NT), 0, st,
+    launch_kernel((matmul_bf16_kernel<SI, OI, WS, WO>), dim3(per_xcd * 8), dim3(C::NT), 0, st,
                        w, x, y, in_dim, out_dim, n, mt, nt);
 }
 

@@ -1170,7 +1170,7 @@ struct PrefillLaunch {
         const int nb = (S + 31) / 32;
         const int total = nh * nb;
         const int per_xcd = (total + 7) / 8;
-        hipLaunchKernelGGL((prefill_sk_kernel<T, D>), dim3(per_xcd * 8), dim3(256), 0, st,
+        launch_kernel((prefill_sk_kernel<T, D>), dim3(per_xcd * 8), dim3(256), 0, st,
                            (const uint16_t *)q, (const char *)kc, (const char *)vc, kvs, S, sp,
                            win, nh, kv_mul, nb, qs, out, pgs);
     }
@@ -1257,7 +1257,7 @@ void PrefillLaunch<T, D, true>::run(const void *q, const void *kc, const void *v
         if (pl.parts > 1 && ws.p && ws.bytes >= pl.bytes) {
             const KeySplit ksp = split_at(pl, 64, ws.p);
             const int lhw = hw == 4 ? 2 : (hw == 2 ? 1 : 0);
-            hipLaunchKernelGGL((prefill4_kernel<T, D, true>), dim3((n_units * ng * pl.parts + 7) / 8 * 8),
+            launch_kernel((prefill4_kernel<T, D, true>), dim3((n_units * ng * pl.parts + 7) / 8 * 8),
                                dim3(512), 0, st, (const uint16_t *)q, (const char *)kc, (const char *)vc,
                                kvs, S, sp, nh, kv_mul, lhw, ng, pl.parts, qs, out, pgs, ksp);
             launch_prefill_merge(D, ksp, 32 * rw, S, sp, 0, nh, out, st);
@@ -1271,12 +1271,12 @@ void PrefillLaunch<T, D, true>::run(const void *q, const void *kc, const void *v
     }
     if (D <= 128 && paired) {
         const int lhw = hw == 4 ? 2 : (hw == 2 ? 1 : 0);
-        hipLaunchKernelGGL((prefill4_kernel<T, D>), dim3(per_xcd * 8), dim3(512), 0, st,
+        launch_kernel((prefill4_kernel<T, D>), dim3(per_xcd * 8), dim3(512), 0, st,
                            (const uint16_t *)q, (const char *)kc, (const char *)vc, kvs, S, sp,
                            nh, kv_mul, lhw, ng, np, qs, out, pgs, KeySplit{});
         return;
     }
-    hipLaunchKernelGGL((prefill2_kernel<T, D>), dim3(per_xcd * 8), dim3(512), 0, st,
+    launch_kernel((prefill2_kernel<T, D>), dim3(per_xcd * 8), dim3(512), 0, st,
                        (const uint16_t *)q, (const char *)kc, (const char *)vc, kvs, S, sp, win,
                        nh, kv_mul, hw, rw, n_units, ng, np, paired, qs, out, pgs);
 }
@@ -1679,7 +1679,7 @@ static int launch_prefill_f32(const void *q, const void *kc, const void *vc, int
     const KeySplit ksp = split_at(pl, 32, ws.p);
     const int per_xcd = (nh / hw * n_units * pl.parts + 7) / 8;
     auto go = [&](auto kern, int threads) {
-        hipLaunchKernelGGL(kern, dim3(per_xcd * 8), dim3(threads), 0, st, (const float *)q, (const float *)kc,
+        launch_kernel(kern, dim3(per_xcd * 8), dim3(threads), 0, st, (const float *)q, (const float *)kc,
                            (const float *)vc, kvs, S, sp, win, nh, kv_mul, hw, n_units, pl.parts, qs, out, pgs, ksp);
     };
     const UnitLoad u = unit_load(S, 128 / hw, nh / hw, sp, win, 32);

@@ -599,9 +599,9 @@ static void prefill16_plan(int S, int start_pos, int window, int n_head, int kv_
 int launch_prefill_merge(int D, KeySplit sp, int UR, int S, int start_pos, int window, int n_head,
                          float *out, hipStream_t st) {
     const dim3 g((unsigned)S, (unsigned)((n_head * D + 1023) / 1024)), b(256);
-    if (D == 64) hipLaunchKernelGGL((prefill_merge_kernel<64>), g, b, 0, st, sp, UR, S, start_pos, window, n_head, out);
-    else if (D == 128) hipLaunchKernelGGL((prefill_merge_kernel<128>), g, b, 0, st, sp, UR, S, start_pos, window, n_head, out);
-    else hipLaunchKernelGGL((prefill_merge_kernel<256>), g, b, 0, st, sp, UR, S, start_pos, window, n_head, out);
+    if (D == 64) launch_kernel((prefill_merge_kernel<64>), g, b, 0, st, sp, UR, S, start_pos, window, n_head, out);
+    else if (D == 128) launch_kernel((prefill_merge_kernel<128>), g, b, 0, st, sp, UR, S, start_pos, window, n_head, out);
+    else launch_kernel((prefill_merge_kernel<256>), g, b, 0, st, sp, UR, S, start_pos, window, n_head, out);
     return check_hip(hipGetLastError(), "prefill merge launch");
 }
 
@@ -643,7 +643,7 @@ static int launch_prefill16_split(int dtype, const void *q, const void *kc, cons
     const int n_units = (S + UR - 1) / UR, n_hg = n_head / hw;
     const KeySplit sp = split_at(pl, 32, ws);
     auto go = [&](auto kern, int ds) {
-        hipLaunchKernelGGL(kern, dim3((unsigned)(n_units * n_hg * pl.parts * ds)), dim3(512), 0, st,
+        launch_kernel(kern, dim3((unsigned)(n_units * n_hg * pl.parts * ds)), dim3(512), 0, st,
                            (const uint16_t *)q, (const char *)kc, (const char *)vc, kvs, S, start_pos,
                            window, n_head, kv_mul, hw, n_hg, n_units, qs, out, pgs, sp);
     };
@@ -669,7 +669,7 @@ int launch_prefill16(int dtype, const void *q, const void *kc, const void *vc, i
     const int n_units = (S + UR - 1) / UR, n_hg = n_head / hw;
     const dim3 grid((unsigned)(n_units * n_hg * DS));
     auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, grid, dim3(512), 0, st, (const uint16_t *)q, (const char *)kc,
+        launch_kernel(kern, grid, dim3(512), 0, st, (const uint16_t *)q, (const char *)kc,
                            (const char *)vc, kvs, S, start_pos, window, n_head, kv_mul, hw, n_hg,
                            n_units, qs, out, pgs, KeySplit{});
     };
@@ -686,7 +686,7 @@ int launch_prefill16(int dtype, const void *q, const void *kc, const void *vc, i
     if (dtype == ULLM_DT_F32) {  // f32 cache: one key stream, value columns split
         const int hw1 = p16_hw(kv_mul, 8), UR1 = 16 * 8 / hw1;
         const int nu1 = (S + UR1 - 1) / UR1, nhg1 = n_head / hw1;
-        hipLaunchKernelGGL((prefill16_kernel<F32, 1, 2>), dim3((unsigned)(nu1 * nhg1 * 2)), dim3(512), 0, st,
+        launch_kernel((prefill16_kernel<F32, 1, 2>), dim3((unsigned)(nu1 * nhg1 * 2)), dim3(512), 0, st,
                            (const uint16_t *)q, (const char *)kc, (const char *)vc, kvs, S, start_pos,
                            window, n_head, kv_mul, hw1, nhg1, nu1, qs, out, pgs, KeySplit{});
     } else if (dtype == ULLM_DT_BF16) pick(BF16{});
@@ -710,7 +710,7 @@ int launch_prefill16_128(int dtype, const void *q, const void *kc, const void *v
     const int n_units = (S + UR - 1) / UR, n_hg = n_head / hw;
     const dim3 grid((unsigned)(n_units * n_hg));
     auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, grid, dim3(512), 0, st, (const uint16_t *)q, (const char *)kc,
+        launch_kernel(kern, grid, dim3(512), 0, st, (const uint16_t *)q, (const char *)kc,
                            (const char *)vc, kvs, S, start_pos, window, n_head, kv_mul, hw, n_hg,
                            n_units, qs, out, pgs, KeySplit{});
     };

@@ -468,7 +468,7 @@ static void launch_gemm(int tile, const GemmArgs &a, hipStream_t st) {
     const dim3 g((unsigned)per_xcd * 8), b(512);
     constexpr bool T3 = NP == 3;
 #define GEMM(SI, OI, WS, WO, KU, NST) \
-    hipLaunchKernelGGL((qkv_gemm_kernel<T, NW, NP, SI, OI, WS, WO, KU, NST, F>), g, b, 0, st, a)
+    launch_kernel((qkv_gemm_kernel<T, NW, NP, SI, OI, WS, WO, KU, NST, F>), g, b, 0, st, a)
     if constexpr (!F) {
         if (tile == kT128x384) { GEMM(2, 3, 2, 4, 1, 4); return; }
         if (tile == kT128x256) { GEMM(2, 2, 2, 4, 1, 4); return; }
@@ -556,14 +556,14 @@ extern "C" int ullm_hip_qkv_gemm_append(const float *x, int in_dim, const void *
                f16 ? inv : nullptr, y, n_q, n_kv, n, in_dim, ld, rows, pl.mt, pl.nt, pl.ks};
     const dim3 xg((unsigned)rows), b(256);
     if (f16)
-        hipLaunchKernelGGL((split_rows_kernel<F16, 2, true>), xg, b, 0, st, x, x, x, rows, rows, in_dim, ld, rows, xp, inv);
+        launch_kernel((split_rows_kernel<F16, 2, true>), xg, b, 0, st, x, x, x, rows, rows, in_dim, ld, rows, xp, inv);
     else if (pl.np == 2)
-        hipLaunchKernelGGL((split_rows_kernel<BF16, 2, false>), xg, b, 0, st, x, x, x, rows, rows, in_dim, ld, rows, xp, inv);
+        launch_kernel((split_rows_kernel<BF16, 2, false>), xg, b, 0, st, x, x, x, rows, rows, in_dim, ld, rows, xp, inv);
     else
-        hipLaunchKernelGGL((split_rows_kernel<BF16, 3, false>), xg, b, 0, st, x, x, x, rows, rows, in_dim, ld, rows, xp, inv);
+        launch_kernel((split_rows_kernel<BF16, 3, false>), xg, b, 0, st, x, x, x, rows, rows, in_dim, ld, rows, xp, inv);
     if (pl.nw == 3) {
         uint16_t *wp = (uint16_t *)(ws + pl.w_off);
-        hipLaunchKernelGGL((split_rows_kernel<BF16, 3, false>), dim3((unsigned)n), b, 0, st,
+        launch_kernel((split_rows_kernel<BF16, 3, false>), dim3((unsigned)n), b, 0, st,
                            (const float *)w_q, (const float *)w_k, (const float *)w_v, n_q, n_q + n_kv,
                            in_dim, ld, n, wp, inv);
         a.wq = (const char *)wp;
