@@ -98,6 +98,8 @@ unsafe extern "C" {
         window: c_int, n_head: c_int, n_kv_head: c_int, head_dim: c_int, scale: f32,
         out: *mut f32, workspace: *mut c_void, workspace_bytes: usize,
         stream: *mut c_void) -> c_int;
+    pub fn ullm_hip_prefill_plan(dtype: c_int, s: c_int, start_pos: c_int, window: c_int,
+        n_head: c_int, n_kv_head: c_int, head_dim: c_int, plan: *mut i32) -> c_int;
     pub fn ullm_hip_prefill_workspace_bytes(dtype: c_int, s: c_int, start_pos: c_int,
         window: c_int, n_head: c_int, n_kv_head: c_int, head_dim: c_int) -> usize;
     pub fn ullm_hip_decode_token(q: *const f32, k: *const f32, v: *const f32,

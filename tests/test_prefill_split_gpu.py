@@ -34,6 +34,10 @@ def _f64(q, k, v, rows, head, kvh, D, start, window):
     ("f32", 40, 5000, 700, 32, 8, 64), ("f32", 17, 3333, 0, 32, 8, 128), ("f32", 100, 4000, 1500, 8, 8, 128),
     ("f16", 45, 5605, 0, 8, 4, 256), ("bf16", 5, 13493, 1024, 8, 4, 256), ("f32", 70, 2222, 0, 8, 4, 256),
     ("f32", 898, 0, 0, 12, 2, 128), ("f32", 217, 22, 1024, 8, 4, 256),
+    # the longest unit a middle one: the first on the window's ramp, the last cut short
+    ("f32", 1217, 0, 1024, 8, 4, 256), ("f32", 641, 1000, 1024, 8, 4, 256), ("f16", 2113, 5, 2048, 8, 4, 256),
+    ("bf16", 1621, 3000, 4096, 8, 4, 256), ("f16", 257, 1000, 1024, 8, 8, 256), ("f32", 1178, 0, 1024, 8, 8, 64),
+    ("f32", 257, 1000, 1024, 32, 8, 64), ("f32", 257, 1000, 1024, 32, 8, 128),
 ])
 @pytest.mark.parametrize("paged", [False, True])
 def test_split_matches_unsplit_and_f64(dev, dt, S, start, window, H, Hk, D, paged):
@@ -67,7 +71,7 @@ def test_split_matches_unsplit_and_f64(dev, dt, S, start, window, H, Hk, D, page
             1 / math.sqrt(D), A._ptr(whole), A._stream()))
     # both hold P (and V of an f32 or bf16 cache) to f16's 2^-11
     assert float((split - whole).norm() / whole.norm()) <= 5e-4
-    rows = sorted({0, S // 2, S - 1})
+    rows = sorted({0, S // 2, max(0, S - 40), S - 1})
     for h in (0, H - 1):
         ref = _f64(q, k, v, rows, h, h // (H // Hk), D, start, window)
         got = split[rows, h * D:(h + 1) * D].double()

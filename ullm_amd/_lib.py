@@ -34,6 +34,7 @@ SIGNATURES = {
         _i, [_vp, _vp, _vp, _i, _i64, _i, _i, _i, _i, _i, _i, _f, _vp, _vp, _sz, _vp]
     ),
     "ullm_hip_prefill_workspace_bytes": (_sz, [_i, _i, _i, _i, _i, _i, _i]),
+    "ullm_hip_prefill_plan": (_i, [_i, _i, _i, _i, _i, _i, _i, _vp]),
     "ullm_hip_rope_table": (_i, [_vp, _i, _i, _f]),
     "ullm_hip_stream_read": (_i, [_vp, _sz, _i, _vp, _vp]),
     "ullm_hip_qkv_append": (

@@ -232,9 +232,10 @@ __device__ __forceinline__ void page_tile(const KvPages &pg, const char *kc, con
 // `chunk` tiles is cut into parts of equal tile counts, each a workgroup of its
 // own that leaves (m, l) and the unnormalised O of its rows, which
 // launch_prefill_merge adds up.  Part p's O is a whole [S][n_head*D] plane,
-// its (m, l) a [S][n_head] plane of pairs.
+// its (m, l) a [S][n_head] plane of pairs.  No unit has more than the `parts`
+// parts that are launched and have planes.
 struct KeySplit {
-    int chunk, tile;
+    int chunk, parts, tile;
     float *o;
     float2 *ml;
 };
@@ -247,9 +248,13 @@ __host__ __device__ __forceinline__ void unit_tiles(int u, int UR, int S, int st
     t0 = lo / tile;
     t1 = (hi + tile - 1) / tile;
 }
+// Parts of a unit of n tiles.
+__device__ __forceinline__ int unit_parts(const KeySplit &sp, int n) {
+    return min((n + sp.chunk - 1) / sp.chunk, sp.parts);
+}
 // The unit's parts, and part `part`'s share of [t0, t1).
 __device__ __forceinline__ int part_tiles(const KeySplit &sp, int part, int &t0, int &t1) {
-    const int parts = (t1 - t0 + sp.chunk - 1) / sp.chunk, per = (t1 - t0 + parts - 1) / parts;
+    const int parts = unit_parts(sp, t1 - t0), per = (t1 - t0 + parts - 1) / parts;
     t0 += part * per;
     t1 = min(t1, t0 + per);
     return parts;
@@ -267,17 +272,25 @@ struct SplitPlan {
 struct UnitLoad {
     double n, longest, avg;
 };
+// Unit lengths never fall from one whole unit to the next (they grow with the
+// causal end until the window's start leaves key 0; from there UR, a multiple
+// of `tile` wherever a window is given, moves both ends by whole tiles), so the
+// longest is the last unit or, when S cuts that one short, the one before it.
 inline UnitLoad unit_load(int S, int UR, int n_hg, int start_pos, int window, int tile) {
     const int n = (S + UR - 1) / UR;
-    int a0, a1, b0, b1;
-    unit_tiles(0, UR, S, start_pos, window, tile, a0, a1);
-    unit_tiles(n - 1, UR, S, start_pos, window, tile, b0, b1);
-    const int last = b1 - b0 > a1 - a0 ? b1 - b0 : a1 - a0;
+    auto len = [&](int u, int &t0) {
+        int t1;
+        unit_tiles(u, UR, S, start_pos, window, tile, t0, t1);
+        return t1 - t0;
+    };
+    int a0, b0, p0;
+    const int first = len(0, a0), last = len(n - 1, b0), prev = len(n > 1 ? n - 2 : 0, p0);
+    const int longest = last > prev ? last : prev;
     // lengths grow to a window's size, and stay there
     const bool flat = window > 0 && b0 > 0;
     const double ramp = flat && window > start_pos ? (double)(window - start_pos) / S : 0.;
-    const double avg = flat ? last - ramp * 0.5 * (last - (a1 - a0)) : 0.5 * (a1 - a0 + b1 - b0);
-    return UnitLoad{(double)n * n_hg, (double)last, avg};
+    const double avg = flat ? longest - ramp * 0.5 * (longest - first) : 0.5 * (first + last);
+    return UnitLoad{(double)n * n_hg, (double)longest, avg};
 }
 // What a workgroup of a prefill kernel costs (us): per key tile when it has
 // the chip nearly alone and when every CU runs one, and once per workgroup.
@@ -296,9 +309,9 @@ inline double prefill_us(const PrefillCost &c, double wgs, double longest, doubl
 }
 // The number of parts with the least estimate, against `unsplit` us without a
 // split (0: one part on the same kernel); the merge streams the partial results
-// at 4 TB/s.  A split has to win by an eighth and by 1.5 us: over 146 random
-// shapes (2..4096 rows at 0..16384, all dtypes and head_dims) the calls that it
-// splits ran 1.1 to 13 times faster, and none of the others moved.
+// at 4 TB/s.  A split has to win by an eighth and by 1.5 us: timed over 146
+// random shapes (2..4096 rows at 0..16384, all dtypes and head_dims) the calls
+// that it splits ran 1.1 to 13 times faster, and none of the others moved.
 inline SplitPlan choose_split(const PrefillCost &c, const UnitLoad &u, double unsplit, int S, int n_head,
                               int D) {
     static const int env = env_override("ULLM_HIP_PREFILL_PARTS");  // tuning: parts of the longest unit (1: never)
@@ -323,7 +336,7 @@ inline SplitPlan choose_split(const PrefillCost &c, const UnitLoad &u, double un
     return pl;
 }
 inline KeySplit split_at(const SplitPlan &pl, int tile, void *ws) {
-    return KeySplit{pl.chunk, tile, (float *)ws, (float2 *)((char *)ws + pl.ml_off)};
+    return KeySplit{pl.chunk, pl.parts, tile, (float *)ws, (float2 *)((char *)ws + pl.ml_off)};
 }
 
 // Head_dim-256 prefill on 16-row waves, two per SIMD (prefill16.hip);

@@ -1817,17 +1817,42 @@ extern "C" int ullm_hip_attn_prefill_paged(const void *q, const void *k_pages, c
                                           head_dim, scale, out, nullptr, 0, stream);
 }
 
+// The split of a call over units of `rows` query rows and tiles of `tile` keys.
+static bool plan_prefill(int dtype, int S, int start_pos, int window, int n_head, int n_kv_head, int head_dim,
+                         int &rows, int &tile, SplitPlan &pl) {
+    if (!dtype_ok(dtype) || S < 1 || start_pos < 0 || n_head < 1 || n_kv_head < 1 || n_head % n_kv_head ||
+        (int64_t)start_pos + S > 0x7fffffff || (head_dim != 64 && head_dim != 128 && head_dim != 256))
+        return false;
+    const int kv_mul = n_head / n_kv_head;
+    rows = kv_mul % 4 == 0 ? 32 : (kv_mul % 2 == 0 ? 64 : 128);
+    tile = 32;
+    if (head_dim == 256 || (head_dim == 128 && dtype == ULLM_DT_F32)) {
+        pl = prefill16_split(dtype, S, start_pos, window, n_head, kv_mul, head_dim);
+    } else if (dtype == ULLM_DT_F32) {
+        pl = prefill_f32_split(S, start_pos, window, n_head, kv_mul, 64);
+    } else {
+        tile = 64;
+        if (window > 0 && window < start_pos + S) pl = SplitPlan{INT_MAX / 2, 1, 0, 0};
+        else pl = prefill4_split(S, start_pos, n_head, kv_mul, head_dim);
+    }
+    return true;
+}
+
 extern "C" size_t ullm_hip_prefill_workspace_bytes(int dtype, int S, int start_pos, int window,
                                                    int n_head, int n_kv_head, int head_dim) {
-    if (!dtype_ok(dtype) || S < 1 || start_pos < 0 || n_head < 1 || n_kv_head < 1 || n_head % n_kv_head ||
-        (int64_t)start_pos + S > 0x7fffffff) return 0;
-    const int kv_mul = n_head / n_kv_head;
-    SplitPlan pl{0, 1, 0, 0};
-    if (head_dim == 256 || (head_dim == 128 && dtype == ULLM_DT_F32))
-        pl = prefill16_split(dtype, S, start_pos, window, n_head, kv_mul, head_dim);
-    else if (head_dim == 64 && dtype == ULLM_DT_F32)
-        pl = prefill_f32_split(S, start_pos, window, n_head, kv_mul, 64);
-    else if ((head_dim == 64 || head_dim == 128) && !(window > 0 && window < start_pos + S))
-        pl = prefill4_split(S, start_pos, n_head, kv_mul, head_dim);
-    return pl.bytes;
+    int rows, tile;
+    SplitPlan pl;
+    return plan_prefill(dtype, S, start_pos, window, n_head, n_kv_head, head_dim, rows, tile, pl) ? pl.bytes : 0;
+}
+
+extern "C" int ullm_hip_prefill_plan(int dtype, int S, int start_pos, int window, int n_head, int n_kv_head,
+                                     int head_dim, int32_t *plan) {
+    int rows, tile;
+    SplitPlan pl;
+    if (!plan) return set_error(ULLM_HIP_E_INVALID, "prefill_plan: null pointer");
+    if (!plan_prefill(dtype, S, start_pos, window, n_head, n_kv_head, head_dim, rows, tile, pl))
+        return set_error(ULLM_HIP_E_UNSUPPORTED, "prefill_plan: dtype %d, %d rows at %d, %d/%d heads x %d", dtype, S,
+                         start_pos, n_head, n_kv_head, head_dim);
+    plan[0] = rows, plan[1] = tile, plan[2] = pl.chunk, plan[3] = pl.parts;
+    return ULLM_HIP_OK;
 }

@@ -529,7 +529,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(KeySplit sp, int UR,
     const int row = blockIdx.x, col = (blockIdx.y * 256 + threadIdx.x) * 4;
     int t0, t1;
     unit_tiles(row / UR, UR, S, start_pos, window, sp.tile, t0, t1);
-    const int parts = (t1 - t0 + sp.chunk - 1) / sp.chunk;
+    const int parts = unit_parts(sp, t1 - t0);
     if (parts < 2 || col >= n_head * D) return;
     const float2 *ml = sp.ml + (int64_t)row * n_head + col / D;
     const float *o = sp.o + (int64_t)row * n_head * D + col;
