@@ -143,8 +143,8 @@ int ullm_hip_attn_prefill_ws(const void *q, const void *k_cache, const void *v_c
 size_t ullm_hip_prefill_workspace_bytes(int dtype, int S, int start_pos, int window, int n_head,
                                         int n_kv_head, int head_dim);
 /* The split itself (host only): plan[0] query rows of a unit, plan[1] keys of a
- * tile, plan[2] the most key tiles of one part, plan[3] the most parts of a
- * unit (1: unsplit).  Unit u attends the tiles of keys from max(0, start_pos +
+ * tile, plan[2] the most key tiles of one part (unbounded when unsplit), plan[3]
+ * the most parts of a unit (1: unsplit, whatever workspace is given).  Unit u attends the tiles of keys from max(0, start_pos +
  * u*plan[0] + 1 - window) (0 without a window) to start_pos + min((u+1)*plan[0], S). */
 int ullm_hip_prefill_plan(int dtype, int S, int start_pos, int window, int n_head, int n_kv_head,
                           int head_dim, int32_t plan[4]);

@@ -33,6 +33,7 @@ def check(dt, S, start, window, H, Hk, D):
     rows, tile, chunk, parts = plan(dt, S, start, window, H, Hk, D)
     longest = int(unit_tiles(rows, tile, S, start, window).max())
     assert -(-longest // chunk) <= parts, (dt, S, start, window, H, Hk, D, chunk, parts, longest)
+    assert parts > 1 or chunk >= 1 << 26  # unsplit: no unit of any length is cut (2^31 keys are 2^26 tiles)
     need = parts * S * H * (D * 4 + 8) if parts > 1 else 0  # O and (m, l) planes of every part
     assert L.lib().ullm_hip_prefill_workspace_bytes(dt, S, start, window, H, Hk, D) == need
     return parts

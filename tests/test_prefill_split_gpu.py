@@ -94,6 +94,33 @@ def test_small_workspace_runs_unsplit(dev):
     assert torch.equal(*outs)
 
 
+# Calls that are not split, with a window and a middle unit longer than the
+# first and the last: a workspace given all the same is left alone.
+@pytest.mark.parametrize("dt,S,start,window,H,Hk,D", [
+    ("f32", 321, 16, 300, 32, 8, 64), ("f32", 385, 0, 129, 6, 2, 64),
+    ("f32", 257, 0, 129, 6, 2, 128), ("f16", 257, 0, 129, 8, 8, 256), ("bf16", 300, 0, 100, 8, 2, 128),
+])
+def test_unsplit_call_leaves_workspace_alone(dev, dt, S, start, window, H, Hk, D):
+    print(f"[prefill-unsplit-ws] {dt} S{S} start{start} win{window} {H}/{Hk}x{D}", flush=True)
+    assert L.lib().ullm_hip_prefill_workspace_bytes(A._DT[DT[dt]], S, start, window, H, Hk, D) == 0
+    g = torch.Generator(device=dev).manual_seed(S)
+    q = torch.randn(S, H * D, device=dev, generator=g).to(DT[dt])
+    k, v = (torch.randn(start + S, Hk * D, device=dev, generator=g).to(DT[dt]) for _ in range(2))
+    ws = torch.full((8 << 20,), 0xA5, dtype=torch.uint8, device=dev)
+    outs = []
+    for w in (None, ws):
+        out = torch.full((S, H * D), 7.0, device=dev)
+        L.check(L.lib().ullm_hip_attn_prefill_ws(
+            A._ptr(q), A._ptr(k), A._ptr(v), A._DT[DT[dt]], Hk * D, S, start, window, H, Hk, D,
+            1 / math.sqrt(D), A._ptr(out), A._ptr(w), 0 if w is None else w.numel(), A._stream()))
+        outs.append(out)
+    assert torch.equal(*outs) and bool((ws == 0xA5).all())
+    rows = list(range(0, S, 16)) + [S - 1]
+    ref = _f64(q, k, v, rows, H - 1, Hk - 1, D, start, window)
+    got = outs[1][rows, (H - 1) * D:].double()
+    assert float((got - ref).norm() / ref.norm()) <= 1e-3
+
+
 # The f32 head_dim-64 kernel unsplit: one set of waves (4 key tiles at most, or
 # short windows on a full chip) and two, with 5 and odd tile counts, units whose
 # second set has a tile less, and rows before the second set's keys.

@@ -262,11 +262,13 @@ __device__ __forceinline__ int part_tiles(const KeySplit &sp, int part, int &t0,
 int launch_prefill_merge(int D, KeySplit sp, int UR, int S, int start_pos, int window, int n_head,
                          float *out, hipStream_t st);
 // Host: the split of a call.  chunk: tiles per part of the longest unit, which
-// has `parts` of them (1: unsplit); bytes: the scratch for O and (m, l).
+// has `parts` of them; bytes: the scratch for O and (m, l).  kUncut: one part
+// for a unit of any length, and no scratch.
 struct SplitPlan {
     int chunk, parts;
     size_t ml_off, bytes;
 };
+constexpr SplitPlan kUncut{0x3fffffff, 1, 0, 0};
 // The units of a call: n workgroups' worth of them when unsplit (row units
 // times head groups), the longest and the average one in key tiles.
 struct UnitLoad {
@@ -315,7 +317,7 @@ inline double prefill_us(const PrefillCost &c, double wgs, double longest, doubl
 inline SplitPlan choose_split(const PrefillCost &c, const UnitLoad &u, double unsplit, int S, int n_head,
                               int D) {
     static const int env = env_override("ULLM_HIP_PREFILL_PARTS");  // tuning: parts of the longest unit (1: never)
-    SplitPlan pl{(int)u.longest, 1, 0, 0};
+    SplitPlan pl = kUncut;
     if (!(unsplit > 0)) unsplit = prefill_us(c, u.n, u.longest, u.n * u.avg);
     double best = unsplit * 0.875 < unsplit - 1.5 ? unsplit * 0.875 : unsplit - 1.5;
     if (u.n > 1024 && env < 2) return pl;  // the chip is full many times over

@@ -1675,7 +1675,7 @@ static int launch_prefill_f32(const void *q, const void *kc, const void *vc, int
     while (hw < 4 && kv_mul % (hw * 2) == 0) hw *= 2;
     const int n_units = (S + 128 / hw - 1) / (128 / hw);
     SplitPlan pl = prefill_f32_split(S, sp, win, nh, kv_mul, D);
-    if (!ws.p || ws.bytes < pl.bytes) pl = SplitPlan{INT_MAX / 2, 1, 0, 0};
+    if (pl.parts < 2 || !ws.p || ws.bytes < pl.bytes) pl = kUncut;
     const KeySplit ksp = split_at(pl, 32, ws.p);
     const int per_xcd = (nh / hw * n_units * pl.parts + 7) / 8;
     auto go = [&](auto kern, int threads) {
@@ -1832,7 +1832,7 @@ static bool plan_prefill(int dtype, int S, int start_pos, int window, int n_head
         pl = prefill_f32_split(S, start_pos, window, n_head, kv_mul, 64);
     } else {
         tile = 64;
-        if (window > 0 && window < start_pos + S) pl = SplitPlan{INT_MAX / 2, 1, 0, 0};
+        if (window > 0 && window < start_pos + S) pl = kUncut;
         else pl = prefill4_split(S, start_pos, n_head, kv_mul, head_dim);
     }
     return true;

@@ -700,7 +700,7 @@ int launch_prefill16_128(int dtype, const void *q, const void *kc, const void *v
                          int S, int start_pos, int window, int n_head, int kv_mul, float qs,
                          float *out, hipStream_t st, KvPages pgs, void *ws, size_t ws_bytes) {
     const bool f32 = dtype == ULLM_DT_F32;
-    const SplitPlan pl = f32 ? prefill16_split(dtype, S, start_pos, window, n_head, kv_mul, 128) : SplitPlan{0, 1, 0, 0};
+    const SplitPlan pl = f32 ? prefill16_split(dtype, S, start_pos, window, n_head, kv_mul, 128) : kUncut;
     if (pl.parts > 1 && ws && ws_bytes >= pl.bytes)
         return launch_prefill16_split<128>(dtype, q, kc, vc, kvs, S, start_pos, window, n_head, kv_mul, qs,
                                            out, st, pgs, pl, ws);
