@@ -238,7 +238,8 @@ size_t ullm_hip_qkv_gemm_workspace_bytes(int rows, int in_dim, int w_dtype, int 
  * the old keys, the merge adds the token's own key and stores its cache row.
  * q/k/v: DEVICE f32 rows; rope_cs as for ullm_hip_qkv_append with rotary_dim =
  * head_dim; old_len: DEVICE int32 holding pos.  Every pointer 16-byte aligned
- * (biases and norms may be NULL).  head_dim 64 or 128, one sequence, and
+ * (biases and norms may be NULL); q, k and v overlap neither out nor the
+ * position's cache rows (ullm_hip_qkv_append takes k and v in place there).  head_dim 64 or 128, one sequence, and
  * enough old keys to be split: ullm_hip_decode_token_workspace_bytes returns 0
  * for what it does not take (ULLM_HIP_E_UNSUPPORTED, nothing launched). */
 int ullm_hip_decode_token(const float *q, const float *k, const float *v, const float *q_bias,

@@ -310,7 +310,7 @@ def test_decode_token_validation():
 
     def call(**kw):
         a = dict(q=64, k=64, v=64, qb=None, kb=None, vb=None, qn=None, kn=None, eps=1e-6, cs=64, npos=600, neox=1,
-                 pos=511, ol=64, win=0, h=8, hk=2, d=64, sc=0.1, kc=64, vc=64, dt=L.DT_F16, kvs=128, out=64,
+                 pos=511, ol=64, win=0, h=8, hk=2, d=64, sc=0.1, kc=64, vc=64, dt=L.DT_F16, kvs=128, out=1 << 16,
                  ws=None, wsb=0, st=None)
         a.update(kw)
         return f(*a.values())
@@ -320,6 +320,13 @@ def test_decode_token_validation():
     for bad in (dict(kvs=64), dict(kvs=132), dict(npos=511), dict(q=None), dict(k=72), dict(qn=68)):
         assert call(**bad) == L.E_INVALID, bad
     assert call() == L.E_WORKSPACE
+    # raw rows in the cache row they go to (row 511 of 128 f16 at kc), or in out
+    far = dict(q=1 << 24, k=1 << 25, v=1 << 26, kc=1 << 20, vc=1 << 21, out=1 << 22)
+    row = (1 << 20) + 511 * 256
+    assert call(**far) == L.E_WORKSPACE and call(**{**far, "k": row + 256}) == L.E_WORKSPACE
+    for bad in (dict(k=row), dict(v=row), dict(k=row + 240), dict(v=row - 496), dict(q=row + 16 + (1 << 20)),
+                dict(out=(1 << 25) + 496), dict(out=1 << 24)):
+        assert call(**{**far, **bad}) == L.E_INVALID, bad
     assert wsz(L.DT_F16, 511, 0, 8, 2, 64, 32) == 0  # partial rotary
     n = wsz(L.DT_F16, 511, 0, 8, 2, 64, 64)
     assert 0 < n <= L.lib().ullm_hip_decode_workspace_bytes(1, 8, 2, 64, 512, 0)

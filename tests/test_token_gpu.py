@@ -116,3 +116,26 @@ def test_graph_replays_match_eager(dev):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want), i
+
+
+# An engine may project k and v straight into the slot of an f32 cache (a view
+# as matmul's y): the append takes them in place, also with norms and biases.
+@pytest.mark.parametrize("pos,window,H,Hk,D,neox", [(511, 0, 32, 8, 64, True), (2999, 0, 32, 4, 128, False),
+                                                    (900, 256, 8, 4, 128, True)])
+@pytest.mark.parametrize("which", ["kv", "k", "v"])
+def test_rows_projected_into_the_cache(dev, pos, window, H, Hk, D, neox, which):
+    print(f"[token-in-place] pos{pos} win{window} {H}/{Hk}x{D} {which}", flush=True)
+    ga, g = _engine(dev, "f32", H, Hk, D, pos + 2, window, neox, pos)
+    kw = _prep(dev, g, H, Hk, D, True, True)
+    q, k, v = (torch.randn(n * D, device=dev, generator=g) for n in (H, Hk, Hk))
+    before = ga.key_cache.clone(), ga.val_cache.clone()
+    want = _separate(ga, q, k, v, pos, kw)
+    rows = ga.key_cache.clone(), ga.val_cache.clone()
+    for c, b, x, n in ((ga.key_cache, before[0], k, "k"), (ga.val_cache, before[1], v, "v")):
+        c.copy_(b)
+        if n in which:
+            c[0, pos] = x
+    got = ga.forward(0, q, ga.key_cache[0, pos] if "k" in which else k,
+                     ga.val_cache[0, pos] if "v" in which else v, pos, **kw)
+    assert torch.equal(got, want)
+    assert torch.equal(ga.key_cache, rows[0]) and torch.equal(ga.val_cache, rows[1])

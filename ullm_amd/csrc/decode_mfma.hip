@@ -1725,6 +1725,15 @@ extern "C" int ullm_hip_decode_token(const float *q, const float *k, const float
     const void *al[] = {q, k, v, q_bias, k_bias, v_bias, q_norm, k_norm, rope_cs, k_cache, v_cache, out};
     for (const void *a : al)
         if ((uintptr_t)a & 15) return set_error(ULLM_HIP_E_INVALID, "decode_token: tensors must be 16-byte aligned");
+    // Every head's workgroups read q, k and v while one of them stores the row.
+    const int64_t qb = (int64_t)n_head * head_dim * 4, kb = (int64_t)n_kv_head * head_dim * 4;
+    const int64_t at = (int64_t)pos * kv_stride * dtype_bytes(kv_dtype), rb = kb / 4 * dtype_bytes(kv_dtype);
+    const struct { const void *p; int64_t n; } in[] = {{q, qb}, {k, kb}, {v, kb}},
+        made[] = {{(char *)k_cache + at, rb}, {(char *)v_cache + at, rb}, {out, qb}};
+    for (const auto &a : in)
+        for (const auto &b : made)
+            if ((uintptr_t)a.p < (uintptr_t)b.p + b.n && (uintptr_t)b.p < (uintptr_t)a.p + a.n)
+                return set_error(ULLM_HIP_E_INVALID, "decode_token: q, k or v overlaps the cache row or out");
     if (!workspace || workspace_bytes < need)
         return set_error(ULLM_HIP_E_WORKSPACE, "decode_token: workspace of %zu bytes needed, %zu given", need,
                          workspace_bytes);

@@ -420,6 +420,15 @@ at::Tensor token(const Args &a) {
     for (const void *q : used)
         fuse = fuse && !odd(q);
     if (is_proj) fuse = fuse && x.numel() >= 8 && x.numel() % 8 == 0;
+    // Raw rows projected straight into the position's f32 cache rows: the append
+    // takes them in place, the fused launch stores there while others read.
+    const int64_t rb = kvs * (int64_t)kc.element_size();
+    const auto over = [&](const at::Tensor &t, const char *c) {
+        const uintptr_t p = (uintptr_t)t.data_ptr(), r = (uintptr_t)c + pos * rb;
+        return p < r + rb && r < p + t.nbytes();
+    };
+    if (!is_proj)
+        for (const at::Tensor *t : {&x, &w0, &w1}) fuse = fuse && !over(*t, l.k) && !over(*t, l.v);
     if (fuse) {
         const float *q = fptr(&x), *k = fptr(&w0), *v = fptr(&w1);
         at::Tensor y;
