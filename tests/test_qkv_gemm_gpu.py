@@ -106,3 +106,31 @@ def test_append_and_rule_match_matvec(dev, rows, D, wdt, neox, rd, kvdt, monkeyp
         assert float((a - b).norm() / b.norm()) <= (2e-6 if kvdt == "f32" else 5e-4)
         step = 2.0 ** -7 * b.abs() if kvdt == "bf16" else 0
         assert bool(((a - b).abs() <= 2e-5 + step).all())
+
+
+@pytest.mark.parametrize("rows", [2, 3, 5])
+def test_few_row_prompts_share_no_counters(dev, rows, monkeypatch):
+    """bf16 prompts of few rows: engines of one shape on two streams give what
+    each gives alone, and none uses the process-wide projection workspace."""
+    print(f"[few-rows] {rows}", flush=True)
+    H, Hk, D, E = 32, 8, 128, 2560
+
+    def no_cached(*a):
+        raise AssertionError("the shared workspace")
+
+    monkeypatch.setattr(A, "proj_workspace", no_cached)
+    runs = []
+    for i in range(2):
+        ga = A.GpuAttention(A.AttnParams(1, H, Hk, D, 64, kv_dtype=torch.bfloat16))
+        x, ws = _inputs(dev, rows, E, H, Hk, D, "bf16", 20 + i)
+        runs.append((ga, x, ws, ga.forward_batch_proj(0, x, *ws, 0)))
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in runs]
+    outs = [[], []]
+    for _ in range(20):
+        for i, (ga, x, ws, _) in enumerate(runs):
+            with torch.cuda.stream(streams[i]):
+                outs[i].append(ga.forward_batch_proj(0, x, *ws, 0))
+    torch.cuda.synchronize()
+    for (_, _, _, want), got in zip(runs, outs):
+        assert all(torch.equal(o, want) for o in got)

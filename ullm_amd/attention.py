@@ -324,11 +324,16 @@ class GpuAttention:
         rows = xbs.shape[0]
         kc, vc = self.key_cache[layer], self.val_cache[layer]
         if rows < 32 and not _gemm_pays(rows, n, xbs.shape[1], D, wq.dtype):
+            # Counters and partial rows of this call alone: prompts of several
+            # engines, on several streams or threads, share nothing here.
+            nb = _proj_ws_bytes(rows, p.n_head, p.n_kv_head, D)
+            ws = torch.zeros(nb, dtype=torch.uint8, device=xbs.device) if nb else None
             return qkv_proj_append(xbs, wq, wk, wv, kc, vc, self.rope_cs, start_pos=start_pos,
                                    n_head=p.n_head, n_kv_head=p.n_kv_head, head_dim=D,
                                    rotary_dim=self.rotary_dim, neox=p.rope_neox, q_norm=norms[0],
                                    k_norm=norms[1], eps=p.eps, q_bias=biases[0],
-                                   k_bias=biases[1], v_bias=biases[2], q_dtype=p.kv_dtype)
+                                   k_bias=biases[1], v_bias=biases[2], q_dtype=p.kv_dtype,
+                                   workspace=ws)
         return _F.proj(xbs, wq, wk, wv, kc, vc, start_pos, 16, self.rope_cs, p.n_head, p.n_kv_head, D,
                        self.rotary_dim, p.rope_neox, norms[0], norms[1], p.eps, *biases, None,
                        p.kv_dtype, None, None, None)
