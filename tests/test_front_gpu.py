@@ -9,12 +9,13 @@ from ullm_amd import attention as A
 pytestmark = pytest.mark.gpu
 
 H, Hk, D, N = 8, 2, 64, 300
+NL = 5000  # keys enough for a prefill of 9 rows to be split, with scratch
 
 
-def _cache(dev, dtype=torch.float16):
+def _cache(dev, dtype=torch.float16, n=N):
     g = torch.Generator(device=dev).manual_seed(4)
-    k, v = (torch.randn(N, Hk * D, device=dev, generator=g).to(dtype) for _ in range(2))
-    return torch.randn(1, H, D, device=dev, generator=g), k, v, torch.tensor([N], dtype=torch.int32, device=dev)
+    k, v = (torch.randn(n, Hk * D, device=dev, generator=g).to(dtype) for _ in range(2))
+    return torch.randn(1, H, D, device=dev, generator=g), k, v, torch.tensor([n], dtype=torch.int32, device=dev)
 
 
 @pytest.mark.parametrize("change,code", [
@@ -44,21 +45,43 @@ def test_given_out_is_returned_and_written(dev):
 def test_other_stream_owns_its_scratch(dev):
     """Scratch of calls queued on another stream is not handed out while they
     wait there: the calls give what they give on the current stream."""
-    q, k, v, lens = _cache(dev)
+    q, k, v, lens = _cache(dev, n=NL)
     qp = torch.randn(9, H * D, device=dev).half()
-    want = A.attn_decode(q, k, v, lens, N, Hk), A.attn_prefill(qp, k, v, H, Hk, D, start_pos=N - 9)
+    want = A.attn_decode(q, k, v, lens, NL, Hk), A.attn_prefill(qp, k, v, H, Hk, D, start_pos=NL - 9)
     s = torch.cuda.Stream()
     torch.cuda.synchronize()
     with torch.cuda.stream(s):
         torch.cuda._sleep(20_000_000)
     outs = [torch.empty_like(w) for w in want]
-    A.attn_decode(q, k, v, lens, N, Hk, out=outs[0], stream=s)
-    A.attn_prefill(qp, k, v, H, Hk, D, start_pos=N - 9, out=outs[1], stream=s)
+    A.attn_decode(q, k, v, lens, NL, Hk, out=outs[0], stream=s)
+    A.attn_prefill(qp, k, v, H, Hk, D, start_pos=NL - 9, out=outs[1], stream=s)
     for _ in range(8):  # would take the scratch if it were free
         torch.full((1 << 20,), 0xFF, dtype=torch.uint8, device=dev)
         torch.full((256,), 0xFF, dtype=torch.uint8, device=dev)
     s.synchronize()
     assert all(torch.equal(a, b) for a, b in zip(outs, want))
+
+
+def test_scratch_comes_from_the_given_streams_memory(dev, monkeypatch):
+    """A block that work queued on torch's current stream may still write is not
+    handed to a call on another stream: its scratch is that stream's own."""
+    q, k, v, lens = _cache(dev, n=NL)
+    qp = torch.randn(9, H * D, device=dev).half()
+    x, ws = torch.randn(64, 2048, device=dev), [torch.randn(n * D, 2048, device=dev).half() for n in (H, Hk, Hk)]
+    cs = A.rope_table(64, D, 1e4, device=dev)
+    monkeypatch.setattr(A, "_gemm_pays", lambda *a: True)
+    assert L.lib().ullm_hip_prefill_workspace_bytes(L.DT_F16, 9, NL - 9, 0, H, Hk, D) > 0
+    calls = [lambda s: A.attn_decode(q, k, v, lens, NL, Hk, out=torch.empty_like(q), stream=s),
+             lambda s: A.attn_prefill(qp, k, v, H, Hk, D, start_pos=NL - 9, out=torch.empty(9, H * D, device=dev), stream=s),
+             lambda s: A.qkv_proj_append(x, *ws, k, v, cs, start_pos=0, n_head=H, n_kv_head=Hk, head_dim=D, stream=s)]
+    for i, call in enumerate(calls):
+        s = torch.cuda.Stream()
+        torch.cuda.synchronize()
+        call(s)
+        torch.cuda.synchronize()
+        assert [b for b in torch.cuda.memory_snapshot() if b["stream"] == s.cuda_stream], \
+            f"call {i}: its scratch came from another stream's memory"
+        assert torch.cuda.current_stream().cuda_stream != s.cuda_stream
 
 
 def test_layer_indices(dev):

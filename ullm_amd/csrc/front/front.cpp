@@ -13,9 +13,9 @@
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <ATen/ATen.h>
-#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/hip/HIPStream.h>
 #include <cmath>
+#include <optional>
 
 #include "../../../include/ullm_hip.h"
 
@@ -103,13 +103,22 @@ struct Stream {
         Py_DECREF(v);
         if (!s && PyErr_Occurred()) throw PyRaised{};
     }
-    // Scratch of one call, kept from reuse until this stream is past it.
+    // Scratch of one call, from this stream's own memory: what held the block
+    // before and what takes it next are in order with the call, whichever
+    // stream is torch's current one.
     at::Tensor scratch(const at::Tensor &like, int64_t bytes) const {
-        at::Tensor t = at::empty({bytes}, like.options().dtype(at::kByte));
-        if (given)
-            t.record_stream(
-                c10::hip::getStreamFromExternalMasqueradingAsCUDA((hipStream_t)s, like.device().index()).unwrap());
-        return t;
+        const auto dev = like.device().index();
+        struct Current {
+            c10::hip::HIPStream was;
+            explicit Current(c10::DeviceIndex d) : was(c10::hip::getCurrentHIPStream(d)) {}
+            ~Current() { c10::hip::setCurrentHIPStream(was); }
+        };
+        std::optional<Current> back;
+        if (given) {
+            back.emplace(dev);
+            c10::hip::setCurrentHIPStream(c10::hip::getStreamFromExternal((hipStream_t)s, dev));
+        }
+        return at::empty({bytes}, like.options().dtype(at::kByte));
     }
 };
 
