@@ -84,6 +84,44 @@ def test_scratch_comes_from_the_given_streams_memory(dev, monkeypatch):
         assert torch.cuda.current_stream().cuda_stream != s.cuda_stream
 
 
+def test_calls_do_without_scratch_they_cannot_have(dev, monkeypatch):
+    """With memory for the outputs alone, the split prefill runs unsplit and the
+    projection of many rows row by row, as both did before they had scratch."""
+    S, start, E, rows = 64, 60000, 2048, 1500
+    k, v = (torch.randn(start + S, Hk * D, device=dev).half() for _ in range(2))
+    q, out = torch.randn(S, H * D, device=dev).half(), torch.empty(S, H * D, device=dev)
+    x, ws = torch.randn(rows, E, device=dev), [torch.randn(n * D, E, device=dev).half() / 45 for n in (H, Hk, Hk)]
+    cs = A.rope_table(rows, D, 1e4, device=dev)
+    kc, vc, qo = (torch.empty(rows, n * D, device=dev) for n in (Hk, Hk, H))
+    kw = dict(start_pos=0, n_head=H, n_kv_head=Hk, head_dim=D)
+    monkeypatch.setattr(A, "_gemm_pays", lambda *a: True)
+    lib = L.lib()
+    need = min(lib.ullm_hip_prefill_workspace_bytes(L.DT_F16, S, start, 0, H, Hk, D),
+               lib.ullm_hip_qkv_gemm_workspace_bytes(rows, E, L.DT_F16, 24, H, Hk, D))
+    assert need > 4 << 20  # more than a small-block segment of the allocator holds
+    whole = torch.empty_like(out)
+    L.check(lib.ullm_hip_attn_prefill(A._ptr(q), A._ptr(k), A._ptr(v), L.DT_F16, Hk * D, S, start, 0, H, Hk, D,
+                                      D ** -0.5, A._ptr(whole), A._stream()))
+    monkeypatch.setattr(A, "_gemm_pays", lambda *a: False)
+    want = A.qkv_proj_append(x, *ws, kc.clone(), vc.clone(), cs, **kw)
+    monkeypatch.setattr(A, "_gemm_pays", lambda *a: True)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / torch.cuda.mem_get_info()[1])
+    try:
+        pad = []
+        with pytest.raises(torch.OutOfMemoryError):  # the allocator's free blocks
+            while len(pad) < 1024:
+                pad.append(torch.empty(2 << 20, dtype=torch.uint8, device=dev))
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(need, dtype=torch.uint8, device=dev)
+        A.attn_prefill(q, k, v, H, Hk, D, start_pos=start, out=out)
+        A.qkv_proj_append(x, *ws, kc, vc, cs, q_out=qo, **kw)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(out, whole) and torch.equal(qo, want)
+
+
 def test_layer_indices(dev):
     ga = A.GpuAttention(A.AttnParams(3, H, Hk, D, 16, kv_dtype=torch.float32))
     q, kk = torch.randn(H * D, device=dev), torch.randn(Hk * D, device=dev)

@@ -120,6 +120,15 @@ struct Stream {
         }
         return at::empty({bytes}, like.options().dtype(at::kByte));
     }
+    // Scratch that a call can do without: undefined where memory has run out.
+    at::Tensor scratch_if_any(const at::Tensor &like, int64_t bytes) const {
+        if (bytes)
+            try {
+                return scratch(like, bytes);
+            } catch (const c10::OutOfMemoryError &) {
+            }
+        return at::Tensor();
+    }
 };
 
 template <class F>
@@ -294,7 +303,7 @@ void proj_call(const at::Tensor &x, const at::Tensor &wq, const at::Tensor &wk, 
 
 // One matvec per row (and the workspace of the caller), or one GEMM over the
 // rows with its own scratch: x_bits 0 or 16 / 24.  None where the GEMM does not
-// take the sizes.
+// take the sizes or has no memory for its scratch.
 PyObject *proj(const Args &a) {
     // x w_q w_k w_v k_cache v_cache start_pos x_bits <Prep> q_out q_dtype kv_stride ws stream
     const at::Tensor &x = a.t(0), &wq = a.t(1), &wk = a.t(2), &wv = a.t(3), &kc = a.t(4), &vc = a.t(5);
@@ -310,16 +319,17 @@ PyObject *proj(const Args &a) {
     const int64_t kvs = a.none(R + 2) ? (int64_t)p.hk * p.D : a.i64(R + 2);
     if (rows != (int)rows || in_dim != (int)in_dim) invalid("x: sizes of 2^31 or more");
     size_t need = 0;
+    at::Tensor ws;
     if (bits) {
         need = ullm_hip_qkv_gemm_workspace_bytes((int)rows, (int)in_dim, wd, bits, p.H, p.hk, p.D);
-        if (need == 0) Py_RETURN_NONE;
+        ws = st.scratch_if_any(x, need);
+        if (!ws.defined()) Py_RETURN_NONE;
     }
     const at::Tensor qo = out_or(a.ot(R), {rows, (int64_t)p.H * p.D}, x, dtype_arg(a, R + 1));
     if (!bits) {
         proj_call(x, wq, wk, wv, in_dim, p, (int)rows, start, qo, kc.data_ptr(), vc.data_ptr(), kd, kvs,
                   a.ot(R + 3), st.s);
     } else {
-        const at::Tensor ws = st.scratch(x, need);
         const int qd = dt(qo);
         call([&] {
             return ullm_hip_qkv_gemm_append(
@@ -349,13 +359,12 @@ at::Tensor prefill(const Args &a) {
     for (int64_t r0 = 0; r0 < std::max<int64_t>(S, 1); r0 += step) {
         const int n = (int)std::min(step, S - r0);
         const size_t need = ullm_hip_prefill_workspace_bytes(qd, n, start + (int)r0, win, H, hk, D);
-        at::Tensor ws;
-        if (need) ws = st.scratch(q, need);
+        const at::Tensor ws = st.scratch_if_any(q, need);
         call([&] {
             return ullm_hip_attn_prefill_ws((const char *)q.data_ptr() + r0 * row * q.element_size(), k.data_ptr(),
                                             v.data_ptr(), qd, kvs, n, start + (int)r0, win, H, hk, D, scale,
-                                            (float *)out.data_ptr() + r0 * row, need ? ws.data_ptr() : nullptr, need,
-                                            st.s);
+                                            (float *)out.data_ptr() + r0 * row, ws.defined() ? ws.data_ptr() : nullptr,
+                                            need, st.s);
         });
     }
     return out;
@@ -376,13 +385,12 @@ at::Tensor prefill_paged(const Args &a) {
     const at::Tensor out = out_or(a.ot(10), {S, row}, q);
     const int qd = dt(q);
     const size_t need = ullm_hip_prefill_workspace_bytes(qd, (int)S, start, win, H, hk, D);
-    at::Tensor ws;
-    if (need) ws = st.scratch(q, need);
+    const at::Tensor ws = st.scratch_if_any(q, need);
     call([&] {
         return ullm_hip_attn_prefill_paged_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), qd, k.size(2), (int)k.size(1),
                                               (int)k.size(0), (const int32_t *)tab.data_ptr(), (int)tab.numel(), (int)S,
                                               start, win, H, hk, D, scale, (float *)out.data_ptr(),
-                                              need ? ws.data_ptr() : nullptr, need, st.s);
+                                              ws.defined() ? ws.data_ptr() : nullptr, need, st.s);
     });
     return out;
 }
