@@ -334,3 +334,28 @@ def test_decode_token_validation():
     assert g(64, 12, 64, 64, 64, L.DT_F16, 8, 2, 64, 64, None) == L.E_INVALID  # in_dim % 8
     assert g(64, 16, 64, 72, 64, L.DT_F16, 8, 2, 64, 64, None) == L.E_INVALID  # alignment
     assert g(64, 16, 64, 64, 64, 5, 8, 2, 64, 64, None) == L.E_UNSUPPORTED
+
+
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("dt,d", [(L.DT_F16, 64), (L.DT_BF16, 128), (L.DT_F16, 256), (L.DT_F32, 64), (L.DT_F32, 128),
+                                  (L.DT_F32, 256)])
+def test_prefill_reports_failed_launches(dt, d, paged):
+    """A split prefill (two launches) and an unsplit one on a machine without a
+    GPU: the launches fail, and the call says so.  A workspace that is not
+    256-byte aligned is refused before that."""
+    if _gpu_visible():
+        pytest.skip("launches kernels on fake pointers when a GPU is visible; runs on CPU-only hosts")
+    lib, fake, S, start, h, hk = L.lib(), 0x10000, 8, 20000, 8, 2
+    need = lib.ullm_hip_prefill_workspace_bytes(dt, S, start, 0, h, hk, d)
+    assert need > 0
+
+    def call(ws):
+        if paged:
+            return lib.ullm_hip_attn_prefill_paged_ws(fake, fake, fake, dt, hk * d, 64, 400, fake, 400, S, start, 0, h,
+                                                      hk, d, 0.1, fake, ws, need if ws else 0, None)
+        return lib.ullm_hip_attn_prefill_ws(fake, fake, fake, dt, hk * d, S, start, 0, h, hk, d, 0.1, fake, ws,
+                                            need if ws else 0, None)
+
+    assert call(fake) == L.E_HIP
+    assert call(None) == L.E_HIP
+    assert call(fake + 16) == L.E_INVALID

@@ -1146,38 +1146,37 @@ __global__ __launch_bounds__(256, 1) void prefill_sk_kernel(
     }
 }
 
-// head_dim 256: prefill16_kernel (16-row waves, two per SIMD), or on request
-// prefill_sk_kernel (split-K inside one-wave-per-SIMD workgroups).
 // Caller's scratch of one call (none: p == nullptr).
 struct Scratch {
     void *p;
     size_t bytes;
 };
 
+// head_dim 256: prefill16_kernel (16-row waves, two per SIMD), or on request
+// prefill_sk_kernel (split-K inside one-wave-per-SIMD workgroups).
 template <class T, int D, bool V2 = (D <= 128)>
 struct PrefillLaunch {
-    static void run(const void *q, const void *kc, const void *vc, int64_t kvs, int S, int sp,
+    static int run(const void *q, const void *kc, const void *vc, int64_t kvs, int S, int sp,
                     int win, int nh, int kv_mul, float qs, float *out, hipStream_t st,
                     KvPages pgs, Scratch ws) {
         // prefill16_kernel; ULLM_HIP_PREFILL256=1 selects prefill_sk_kernel
         // instead, for comparison.
         static const int pick = env_override("ULLM_HIP_PREFILL256");
-        if (pick != 1) {
-            launch_prefill16(__is_same(T, BF16) ? ULLM_DT_BF16 : ULLM_DT_F16, q, kc, vc, kvs, S, sp,
-                             win, nh, kv_mul, qs, out, st, pgs, ws.p, ws.bytes);
-            return;
-        }
+        if (pick != 1)
+            return launch_prefill16(__is_same(T, BF16) ? ULLM_DT_BF16 : ULLM_DT_F16, q, kc, vc, kvs, S, sp,
+                                    win, nh, kv_mul, qs, out, st, pgs, ws.p, ws.bytes);
         const int nb = (S + 31) / 32;
         const int total = nh * nb;
         const int per_xcd = (total + 7) / 8;
         launch_kernel((prefill_sk_kernel<T, D>), dim3(per_xcd * 8), dim3(256), 0, st,
                            (const uint16_t *)q, (const char *)kc, (const char *)vc, kvs, S, sp,
                            win, nh, kv_mul, nb, qs, out, pgs);
+        return check_hip(hipGetLastError(), "prefill launch");
     }
 };
 template <class T, int D>
 struct PrefillLaunch<T, D, true> {
-    static void run(const void *q, const void *kc, const void *vc, int64_t kvs, int S, int sp,
+    static int run(const void *q, const void *kc, const void *vc, int64_t kvs, int S, int sp,
                     int win, int nh, int kv_mul, float qs, float *out, hipStream_t st,
                     KvPages pgs, Scratch ws);
 };
@@ -1238,9 +1237,9 @@ static SplitPlan prefill_f32_split(int S, int sp, int win, int nh, int kv_mul, i
 }
 
 template <class T, int D>
-void PrefillLaunch<T, D, true>::run(const void *q, const void *kc, const void *vc, int64_t kvs,
-                                    int S, int sp, int win, int nh, int kv_mul, float qs,
-                                    float *out, hipStream_t st, KvPages pgs, Scratch ws) {
+int PrefillLaunch<T, D, true>::run(const void *q, const void *kc, const void *vc, int64_t kvs,
+                                   int S, int sp, int win, int nh, int kv_mul, float qs,
+                                   float *out, hipStream_t st, KvPages pgs, Scratch ws) {
     // Units of HW heads (HW | kv_mul, at most 4) x groups of RW = 4/HW 32-row blocks.
     const int hw = kv_mul % 4 == 0 ? 4 : (kv_mul % 2 == 0 ? 2 : 1);
     const int rw = 4 / hw;
@@ -1260,32 +1259,22 @@ void PrefillLaunch<T, D, true>::run(const void *q, const void *kc, const void *v
             launch_kernel((prefill4_kernel<T, D, true>), dim3((n_units * ng * pl.parts + 7) / 8 * 8),
                                dim3(512), 0, st, (const uint16_t *)q, (const char *)kc, (const char *)vc,
                                kvs, S, sp, nh, kv_mul, lhw, ng, pl.parts, qs, out, pgs, ksp);
-            launch_prefill_merge(D, ksp, 32 * rw, S, sp, 0, nh, out, st);
-            return;
+            return launch_prefill_merge(D, ksp, 32 * rw, S, sp, 0, nh, out, st);
         }
     }
-    if (D == 128 && prefill16_takes_128(S, sp, win, nh, kv_mul)) {
-        launch_prefill16_128(__is_same(T, BF16) ? ULLM_DT_BF16 : ULLM_DT_F16, q, kc, vc, kvs, S, sp,
-                             win, nh, kv_mul, qs, out, st, pgs, ws.p, ws.bytes);
-        return;
-    }
+    if (D == 128 && prefill16_takes_128(S, sp, win, nh, kv_mul))
+        return launch_prefill16_128(__is_same(T, BF16) ? ULLM_DT_BF16 : ULLM_DT_F16, q, kc, vc, kvs, S, sp,
+                                    win, nh, kv_mul, qs, out, st, pgs, ws.p, ws.bytes);
     if (D <= 128 && paired) {
         const int lhw = hw == 4 ? 2 : (hw == 2 ? 1 : 0);
         launch_kernel((prefill4_kernel<T, D>), dim3(per_xcd * 8), dim3(512), 0, st,
                            (const uint16_t *)q, (const char *)kc, (const char *)vc, kvs, S, sp,
                            nh, kv_mul, lhw, ng, np, qs, out, pgs, KeySplit{});
-        return;
+        return check_hip(hipGetLastError(), "prefill launch");
     }
     launch_kernel((prefill2_kernel<T, D>), dim3(per_xcd * 8), dim3(512), 0, st,
                        (const uint16_t *)q, (const char *)kc, (const char *)vc, kvs, S, sp, win,
                        nh, kv_mul, hw, rw, n_units, ng, np, paired, qs, out, pgs);
-}
-
-template <class T, int D>
-static int launch_prefill(const void *q, const void *kc, const void *vc, int64_t kvs, int S,
-                          int sp, int win, int nh, int kv_mul, float qs, float *out,
-                          hipStream_t st, KvPages pgs, Scratch ws) {
-    PrefillLaunch<T, D>::run(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st, pgs, ws);
     return check_hip(hipGetLastError(), "prefill launch");
 }
 
@@ -1695,9 +1684,9 @@ static int dispatch_prefill(int D, const void *q, const void *kc, const void *vc
                             int S, int sp, int win, int nh, int kv_mul, float qs, float *out,
                             hipStream_t st, KvPages pgs, Scratch ws) {
     switch (D) {
-        case 64: return launch_prefill<T, 64>(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st, pgs, ws);
-        case 128: return launch_prefill<T, 128>(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st, pgs, ws);
-        case 256: return launch_prefill<T, 256>(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st, pgs, ws);
+        case 64: return PrefillLaunch<T, 64>::run(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st, pgs, ws);
+        case 128: return PrefillLaunch<T, 128>::run(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st, pgs, ws);
+        case 256: return PrefillLaunch<T, 256>::run(q, kc, vc, kvs, S, sp, win, nh, kv_mul, qs, out, st, pgs, ws);
         default: return set_error(ULLM_HIP_E_UNSUPPORTED, "prefill: head_dim %d not in {64,128,256}", D);
     }
 }
@@ -1753,6 +1742,8 @@ extern "C" int ullm_hip_attn_prefill_ws(const void *q, const void *k_cache, cons
         return set_error(ULLM_HIP_E_INVALID, "prefill: null tensor pointer");
     if (((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)out) & 15)
         return set_error(ULLM_HIP_E_INVALID, "prefill: tensors must be 16-byte aligned");
+    if ((uintptr_t)workspace & 255)
+        return set_error(ULLM_HIP_E_INVALID, "prefill: workspace must be 256-byte aligned");
     return run_prefill(dtype, q, k_cache, v_cache, kv_stride, S, start_pos, window, n_head,
                        n_head / n_kv_head, head_dim, scale * kLog2e, out, (hipStream_t)stream, KvPages{},
                        Scratch{workspace, workspace_bytes});
@@ -1800,6 +1791,8 @@ extern "C" int ullm_hip_attn_prefill_paged_ws(const void *q, const void *k_pages
         return set_error(ULLM_HIP_E_INVALID, "prefill_paged: null tensor pointer");
     if (((uintptr_t)q | (uintptr_t)k_pages | (uintptr_t)v_pages | (uintptr_t)out) & 15)
         return set_error(ULLM_HIP_E_INVALID, "prefill_paged: tensors must be 16-byte aligned");
+    if ((uintptr_t)workspace & 255)
+        return set_error(ULLM_HIP_E_INVALID, "prefill_paged: workspace must be 256-byte aligned");
     const KvPages pgs{block_table, table_len, __builtin_ctz(page_size), n_pages};
     return run_prefill(dtype, q, k_pages, v_pages, kv_stride, S, start_pos, window, n_head,
                        n_head / n_kv_head, head_dim, scale * kLog2e, out, (hipStream_t)stream, pgs,
