@@ -90,6 +90,21 @@ def p16_geometry(S, H, Hk, start_pos=0, window=0):
     grid1 = (S + 128 // hw1 - 1) // (128 // hw1) * (H // hw1)
     binding = 0 < window < start_pos + S
     ks = 2 if grid1 <= (128 if binding else 256) else 1
+    if binding and 128 < grid1 < 256:  # prefill16_two_streams
+        def tiles(u, rows):
+            lo, hi = max(0, start_pos + u * rows + 1 - window), start_pos + min(u * rows + rows, S)
+            return (hi + 31) // 32 - lo // 32
+
+        def longest(rows):
+            n = (S + rows - 1) // rows
+            return max(tiles(n - 1, rows), tiles(max(n - 2, 0), rows))
+        hw2 = hw_of(4)
+        ur2, n_hg = 64 // hw2, H // hw2
+        n = (S + ur2 - 1) // ur2
+        two = 10.7 + 0.94 * longest(ur2)
+        if n * n_hg > 256:
+            two = max(two, 1.57 * (10.7 + 0.94 * tiles(max(0, n - 1 - 256 // n_hg), ur2)))
+        ks = 2 if two <= 10.2 + 1.1 * longest(128 // hw1) else 1
     hw = hw_of(8 // ks)
     ur = 16 * (8 // ks) // hw
     ds = 2 if ks == 2 and (S + ur - 1) // ur * (H // hw) * 2 <= 256 else 1
@@ -114,7 +129,10 @@ P16_CASES = [
     ("bf16", 2500, 32, 8, 0, 0),
     ("f16", 1, 8, 4, 0, 0),
     ("bf16", 17, 16, 16, 5, 0),
-    ("f16", 2100, 16, 16, 0, 0)]
+    ("f16", 2100, 16, 16, 0, 0),
+    ("f16", 2100, 8, 4, 0, 512),     # 129 to 255 units with a window: two key streams,
+    ("bf16", 1030, 16, 8, 0, 768),
+    ("f16", 2100, 8, 4, 256, 512)]   # and one
 
 
 @pytest.mark.parametrize("dtype,S,H,Hk,start_pos,window", P16_CASES)
@@ -147,6 +165,15 @@ def test_head_dim_128_both_kernels(dev, dtype, S, H, Hk, start_pos):
 def test_head_dim_128_cases_cover_both_kernels():
     seen = {prefill128_kernel(S, H, Hk, sp) for (_, S, H, Hk, sp) in P128_CASES}
     assert {"prefill16", "prefill4"} <= seen, seen
+
+
+def test_windowed_key_streams():
+    """Prompts little longer than their window keep two key streams (their
+    second round of workgroups is short); later chunks run on one."""
+    for S, H, Hk, start, window, ks in ((2100, 8, 4, 0, 512, 2), (2100, 8, 4, 256, 512, 1), (1030, 16, 8, 0, 768, 2),
+                                        (2100, 8, 4, 4000, 1024, 1), (4001, 8, 4, 0, 1024, 1),
+                                        (2000, 8, 4, 0, 1024, 2)):
+        assert p16_geometry(S, H, Hk, start, window)[0] == ks, (S, H, Hk, start, window)
 
 
 def test_head_dim_256_geometries_covered():

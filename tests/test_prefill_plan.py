@@ -51,7 +51,7 @@ def test_no_unit_needs_more_parts_than_planned(dt, H, Hk, D, window):
 # A first unit still on the window's ramp and a last one cut short, so that a
 # middle unit is the longest; all of them are split.
 RAMPED = [(L.DT_F32, 1217, 0, 1024, 8, 4, 256), (L.DT_F32, 641, 1000, 1024, 8, 4, 256),
-          (L.DT_F32, 853, 300, 1024, 8, 4, 256), (L.DT_F16, 2113, 5, 2048, 8, 4, 256),
+          (L.DT_F32, 853, 300, 1024, 8, 4, 256), (L.DT_F16, 1025, 4000, 4096, 8, 4, 256),
           (L.DT_BF16, 1621, 3000, 4096, 8, 4, 256), (L.DT_F16, 257, 1000, 1024, 8, 8, 256),
           (L.DT_F32, 1178, 0, 1024, 8, 8, 64), (L.DT_F32, 257, 1000, 1024, 32, 8, 64),
           (L.DT_F32, 257, 1000, 1024, 32, 8, 128)]

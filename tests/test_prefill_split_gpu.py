@@ -35,7 +35,7 @@ def _f64(q, k, v, rows, head, kvh, D, start, window):
     ("f16", 45, 5605, 0, 8, 4, 256), ("bf16", 5, 13493, 1024, 8, 4, 256), ("f32", 70, 2222, 0, 8, 4, 256),
     ("f32", 898, 0, 0, 12, 2, 128), ("f32", 217, 22, 1024, 8, 4, 256),
     # the longest unit a middle one: the first on the window's ramp, the last cut short
-    ("f32", 1217, 0, 1024, 8, 4, 256), ("f32", 641, 1000, 1024, 8, 4, 256), ("f16", 2113, 5, 2048, 8, 4, 256),
+    ("f32", 1217, 0, 1024, 8, 4, 256), ("f32", 641, 1000, 1024, 8, 4, 256), ("f16", 1025, 4000, 4096, 8, 4, 256),
     ("bf16", 1621, 3000, 4096, 8, 4, 256), ("f16", 257, 1000, 1024, 8, 8, 256), ("f32", 1178, 0, 1024, 8, 8, 64),
     ("f32", 257, 1000, 1024, 32, 8, 64), ("f32", 257, 1000, 1024, 32, 8, 128),
 ])

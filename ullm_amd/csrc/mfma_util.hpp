@@ -278,6 +278,7 @@ struct UnitLoad {
 // causal end until the window's start leaves key 0; from there UR, a multiple
 // of `tile` wherever a window is given, moves both ends by whole tiles), so the
 // longest is the last unit or, when S cuts that one short, the one before it.
+// (Units of half a tile are only estimated with: to within a tile.)
 inline UnitLoad unit_load(int S, int UR, int n_hg, int start_pos, int window, int tile) {
     const int n = (S + UR - 1) / UR;
     auto len = [&](int u, int &t0) {

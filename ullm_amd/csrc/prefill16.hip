@@ -570,13 +570,33 @@ static int p16_hw(int kv_mul, int nws) {
     return hw;
 }
 
+// Whether two key streams beat one for a windowed prompt of 129 to 255 units,
+// whose two-stream workgroups (twice as many) need a second round on the CUs.
+// They run longest first, so the second round holds the units on the window's
+// ramp, and a short one starts when the first of those that it follows ends.
+// Estimate: us per workgroup and 32-key tile, fitted to 312 calls (f16 and bf16
+// at head_dim 256, f32 at 128, windows 128..2000 from 0 or from half a window;
+// one stream 0.72 to 1.67 times the rate of two).  No call runs on one stream
+// that is faster on two, and the choice is 1.3 % from the better one on
+// average.  8/4 heads x 256, f16, one / two, us: 2100 rows, window 512, from 0
+// 26.5 / 22.4; from 256 26.7 / 35.1; 4001 rows, window 1024, 53.0 / 77.9.
+static bool prefill16_two_streams(int S, int start_pos, int window, int n_head, int kv_mul) {
+    const int UR1 = 128 / p16_hw(kv_mul, 8), hw2 = p16_hw(kv_mul, 4), UR2 = 64 / hw2, n_hg = n_head / hw2;
+    const int n = (S + UR2 - 1) / UR2, first = n - 1 - 256 / n_hg;  // first unit of the second round
+    const double one = 10.2 + 1.1 * unit_load(S, UR1, 1, start_pos, window, 32).longest;
+    double two = 10.7 + 0.94 * unit_load(S, UR2, 1, start_pos, window, 32).longest;
+    if ((int64_t)n * n_hg > 256) {
+        int t0, t1;
+        unit_tiles(first > 0 ? first : 0, UR2, S, start_pos, window, 32, t0, t1);
+        two = std::max(two, 1.57 * (10.7 + 0.94 * (t1 - t0)));
+    }
+    return two <= one;
+}
+
 // Key streams and value-column split for a prompt.  Two key streams up to one
 // causal (window-free) unit per CU, the longest setting the time; with a
-// binding window, where all units are alike, up to half that, so that the
-// twice as many workgroups still run in one round (8/4 heads x 256, f16, window
-// 1024, KS1 / KS2: 2000 rows 44.2 / 38.5, 2500 rows (160 units) 45.5 / 49.3, 4001
-// rows 53.0 / 77.9; causal 4001 rows 135 / 126); the value
-// split on top when the workgroups still fit one per CU.  Measured at 8/4
+// binding window up to half that, or where prefill16_two_streams has it; the
+// value split on top when the workgroups still fit one per CU.  Measured at 8/4
 // heads, f16 (us; KS/DS): S=1024 KS2/DS2 23.9, KS2/DS1 27.1, KS1/DS2 34.5;
 // S=2048 KS2/DS1 51.5, KS2/DS2 53.2; S=4096 causal KS2/DS1 122-130, KS1/DS1
 // 134-137; S=4096 window 1024 KS1/DS1 57.9, KS2/DS1 76.6; 16/8 heads at
@@ -589,6 +609,8 @@ static void prefill16_plan(int S, int start_pos, int window, int n_head, int kv_
     const int64_t grid1 = (int64_t)((S + 128 / hw - 1) / (128 / hw)) * (n_head / hw);
     const bool binding = window > 0 && window < start_pos + S;
     ks = grid1 <= (binding ? 128 : 256) ? 2 : 1;
+    if (binding && grid1 > 128 && grid1 < 256)
+        ks = prefill16_two_streams(S, start_pos, window, n_head, kv_mul) ? 2 : 1;
     if (eks == 1 || eks == 2) ks = eks;
     const int hw2 = p16_hw(kv_mul, 8 / ks), ur = 16 * (8 / ks) / hw2;
     const int64_t grid = (int64_t)((S + ur - 1) / ur) * (n_head / hw2);
