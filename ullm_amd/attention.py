@@ -186,13 +186,23 @@ def _gemm_pays(rows, n, in_dim, head_dim, w_dtype):
     """Whether `rows` token rows of an [n, in_dim] projection run faster as
     ullm_hip_qkv_gemm_append (every weight read once, three launches) than as
     qkv_proj_append's matvec per row.  Measured (us, matvec / GEMM, 24 bits):
-    bf16 2560 -> 6144: 8 rows 20.8 / 24.5, 12 rows 29.3 / 24.7, 300 rows 509 /
-    48; f16 2048 -> 3072: 16 rows 15.8 / 20.1, 40 rows 36.4 / 21.5; f32 2560 ->
-    6144: 16 rows 49 / 62, 40 rows 126 / 58; head_dim 256 from 256 head vectors
-    on (16 rows of 16, 2560 -> 4096): 112..117 / 24 (16-bit), 105 / 49 (f32)."""
-    if head_dim == 256 and rows * (n // head_dim) >= 256:
+    16-bit weights: bf16 2560 -> 6144: 8 rows 20 / 20, 12 rows 29 / 20, 300 rows
+    509 / 48; f16 2048 -> 3072: 24 rows 22 / 17; bf16 8192 -> 10240: 2 rows 62 /
+    46; one row never gains (16384 -> 18432 122 / 152, f16 122 / 170).
+    f32 weights are split into planes on each call, which a few rows do not pay
+    for however large they are: 2560 -> 6144 16 rows 56 / 58, 24 rows 86 / 59;
+    4096 -> 6144 16 rows 86 / 96, 20 rows 109 / 97; 8192 -> 10240 8 rows 235 /
+    294, 12 rows 302 / 293; 16384 -> 18432 2 rows 365 / 1165, 12 rows 1529 / 1176.
+    head_dim 256 from 256 head vectors on, where the matvec is 4 to 9 times
+    slower (3584 -> 8192 6 / 8 rows: bf16 37 / 223 against 26, f32 62 / 203
+    against 91); f32 8192 -> 32768: 2 rows 508 / 912, 3 rows 940 / 919."""
+    f32 = w_dtype == torch.float32
+    if head_dim == 256 and rows * (n // head_dim) >= 256 and not (f32 and rows < 3):
         return True
-    return rows * n * in_dim >= (320_000_000 if w_dtype == torch.float32 else 160_000_000)
+    work = rows * n * in_dim
+    if f32:
+        return (rows >= 20 and work >= 320_000_000) or (rows >= 12 and work >= 800_000_000)
+    return rows > 1 and work >= 160_000_000
 
 
 def qkv_proj_append(x, w_q, w_k, w_v, k_cache, v_cache, rope_cs, *, start_pos, n_head,
