@@ -213,8 +213,8 @@ size_t ullm_hip_qkv_proj_workspace_bytes(int rows, int n_head, int n_kv_head, in
  * row) into the workspace, the append follows.  Same arguments and result as
  * ullm_hip_qkv_proj_append (any number of rows), plus
  * x_bits: significant bits of x that enter the products, 16 (as
- *         ullm_hip_matmul) or 24; with f16 weights x carries 22 bits (relative
- *         to no less than 2^-17 of its row's largest value) whatever x_bits is
+ *         ullm_hip_matmul) or 24; with f16 weights x carries 22 bits (of every
+ *         value down to 2^-29 of its row's largest) whatever x_bits is
  * workspace: DEVICE memory of ullm_hip_qkv_gemm_workspace_bytes, 256-byte
  *         aligned; needs no initialisation, one call at a time.
  * An operand of 2 GiB or more (rows or outputs times in_dim, 16-bit) is

@@ -26,8 +26,9 @@ def _raw(x, ws, H, Hk, D, bits, start=0):
     cs[..., 0] = 1
     kc = torch.full((start + rows + 1, Hk * D), 7.0, device=x.device)
     vc = kc.clone()
+    mv = None if bits else A.proj_workspace(rows, H, Hk, D, x.device)  # bits 0: the matvec per row
     q = A._F.proj(x, *ws, kc, vc, start, bits, cs, H, Hk, D, D, True, None, None, 1e-6, None, None, None,
-                  None, None, None, None, None)
+                  None, None, None, mv, None)
     for c in (kc, vc):  # rows outside start.. are untouched
         assert bool((c[:start] == 7).all()) and bool((c[start + rows:] == 7).all())
     return q, kc[start:start + rows], vc[start:start + rows]
@@ -48,15 +49,34 @@ def test_projection_vs_f64(dev, rows, in_dim, H, Hk, D, wdt, bits):
     x *= torch.exp2(torch.randint(-60, 61, (rows, 1), device=dev, dtype=torch.float32))
     x[0, 0] *= 2.0 ** 20
     # relative residual of the planes, plus the f32 additions (in_dim of them
-    # at most); f16 planes also lose 2^-39 of the row's largest |x|
+    # at most); f16 planes also lose 2^-51 of the row's largest |x|
     eps = (2.0 ** -16 if bits == 16 else 2.0 ** -21) + in_dim * 2.0 ** -24
     for y, w in zip(_raw(x, ws, H, Hk, D, bits, start=2), ws):
         w64 = w.double()
         ref = x.double() @ w64.t().contiguous()
         bound = eps * (x.double().abs() @ w64.abs().t().contiguous())
         if wdt == "f16":
-            bound += 2.0 ** -39 * x.double().abs().amax(1, keepdim=True) * w64.abs().sum(1)
+            bound += 2.0 ** -51 * x.double().abs().amax(1, keepdim=True) * w64.abs().sum(1)
         assert bool(((y.double() - ref).abs() <= bound + 1e-37).all())
+
+
+@pytest.mark.parametrize("wdt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("power,weight", [(0, 1), (5, 1), (10, 1), (20, 1), (10, 0), (15, 0), (20, 0)])
+def test_error_is_no_larger_than_the_matvecs(dev, wdt, power, weight):
+    """Against f64, also for rows with outliers, and where no weight takes the
+    outliers (what is small beside them then is all of the result)."""
+    rows, E, H, Hk, D = 64, 2048, 8, 4, 128
+    print(f"[qkv-gemm-outlier] {wdt} 2^{power} weight {weight}", flush=True)
+    x, ws = _inputs(dev, rows, E, H, Hk, D, wdt, 30 + power)
+    for col in (7, 1203):
+        x[:, col] *= 2.0 ** power
+        for w in ws:
+            w[:, col] *= weight
+    ref = x.double() @ torch.cat(ws).double().t().contiguous()
+    gemm, matvec = (float((torch.cat(_raw(x, ws, H, Hk, D, b), 1).double() - ref).norm() / ref.norm())
+                    for b in (24, 0))
+    print(f"gemm {gemm:.3g} matvec {matvec:.3g}", flush=True)
+    assert gemm <= matvec
 
 
 @pytest.mark.parametrize("wdt,bits", [("bf16", 16), ("bf16", 24), ("f16", 24), ("f32", 24)])

@@ -12,8 +12,10 @@
 //   bf16 weights: X = 2 bf16 planes (16 significant bits, what
 //     ullm_hip_matmul carries) or 3 (24 bits: every f32 exactly);
 //   f16 weights: X scaled by a power of two per row (its largest finite |x|
-//     in [2^14, 2^15)) into 2 f16 planes: 22 bits, and never less than 2^-39
-//     of the row's largest value; the scale is taken out of Y;
+//     in [2^14, 2^15)) into 2 f16 planes, the second times 2^12: 22 bits (at
+//     least: what f16 leaves of a value is rounded to f16 again), and never less
+//     than 2^-51 of the row's largest value; each plane has its own sum, and the
+//     scales are taken out of those and of Y;
 //   f32 weights: X and W as 3 bf16 planes each, the six products of weight
 //     2^-16 and above.
 //
@@ -33,6 +35,7 @@ constexpr int kGmK = 32;                // input dims of one row of a tile
 constexpr int kGmRB = kGmK * 2;         // its bytes
 constexpr int kGmPad = 128;             // X and W planes: dims padded to a multiple (zeros)
 constexpr int kGmOOB = 0x7ffffff0;      // buffer offset past every valid range: reads zero
+constexpr float kLowPlane = 0x1p-12f;   // scale of the second f16 plane
 
 struct GemmArgs {
     const char *wq, *wk, *wv;  // [n_q][in_dim] ...; NW > 1: wq = the planes [NW][n][ldx]
@@ -150,12 +153,13 @@ __global__ __launch_bounds__(512) void qkv_gemm_kernel(GemmArgs a) {
     }
 
     // FOLD: the matrix cores sum one step from zero, smallest products first,
-    // into acc[0] and acc[1] in turn.  The step before is added to `sum` in
+    // into acc[0] and acc[1] in turn (BYP: each plane of X into its own).  The step before is added to `sum` in
     // f32 in the shadow of the MFMAs, and every eight steps `sum` goes to
     // `top`, so that few additions round at the size of the whole result.
     // Relative error at in_dim 2048..2560 (f64 reference): 1.0e-7..1.1e-7,
     // against 1.2e-7..1.3e-7 of qkv_proj_kernel's f32 sums and 2.5e-7..5.6e-7
     // of one chain of MFMAs.
+    constexpr bool BYP = FOLD && __is_same(T, F16);
     constexpr int NA = FOLD ? 2 : 1;
     f32x16 acc[NA][OI][SI], sum[FOLD ? OI : 1][FOLD ? SI : 1], top[FOLD ? OI : 1][FOLD ? SI : 1];
 #pragma unroll
@@ -210,9 +214,40 @@ __global__ __launch_bounds__(512) void qkv_gemm_kernel(GemmArgs a) {
         }
     };
     constexpr int NMF = 2 * KU * OI * SI * (NW == 3 ? 6 : NP);  // MFMAs per step
+    // BYP: plane 1 of this step while plane 0 of the step before is added to
+    // `sum`, then plane 0 while plane 1 is added.
+    auto by_plane = [&](auto pc) {
+        constexpr int p = decltype(pc)::value;
+        constexpr int NM = 2 * KU * OI * SI, V = (OI * SI * 16 + NM - 1) / NM + 1;
+        static_for<0, 2 * KU>([&](auto hc) {
+            constexpr int h = decltype(hc)::value;
+#pragma unroll
+            for (int i = 0; i < OI; i++)
+#pragma unroll
+                for (int j = 0; j < SI; j++)
+                    acc[p][i][j] = mfma32<T>(fw[h][0][i], fx[h][p][j], h == 0 ? f32x16{} : acc[p][i][j]);
+        });
+#pragma unroll
+        for (int i = 0; i < OI; i++)
+#pragma unroll
+            for (int j = 0; j < SI; j++) {
+                if constexpr (p == 1) sum[i][j] += acc[0][i][j];
+                else sum[i][j] += acc[1][i][j] * kLowPlane;
+            }
+        static_for<0, NM>([&](auto) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, V, 0);
+        });
+    };
     auto multiply = [&](auto nc) {
         constexpr int n = decltype(nc)::value;
         __builtin_amdgcn_s_setprio(1);
+        if constexpr (BYP) {
+            by_plane(Int<1>{});
+            by_plane(Int<0>{});
+            __builtin_amdgcn_s_setprio(0);
+            return;
+        }
         // products of plane weight 2, 1, 0 (FOLD), or plane by plane
         static_for<0, FOLD ? 3 : 1>([&](auto oc) {
             constexpr int ord = 2 - decltype(oc)::value;
@@ -290,7 +325,7 @@ __global__ __launch_bounds__(512) void qkv_gemm_kernel(GemmArgs a) {
     // acc[i][j][4 g + e] = Y[s, o]: s = s0 + (wm SI + j) 32 + c32,
     // o = o0 + (wn OI + i) 32 + 8 g + 4 h2 + e.
     if constexpr (FOLD) {  // the last step's sums are not added yet
-        const bool odd = (ke - kb) & 1;
+        const bool odd = BYP || ((ke - kb) & 1);
 #pragma unroll
         for (int i = 0; i < OI; i++)
 #pragma unroll
@@ -337,6 +372,8 @@ __device__ __forceinline__ void planes_of(float x, uint16_t (&o)[NP]) {
         float hf, z;
         unpack2<T>(h, hf, z);
         r -= hf;
+        // |r| <= half a step of a value below 2^15 (2^3): 2^15 at most
+        if constexpr (__is_same(T, F16)) r *= 1.f / kLowPlane;
     }
     if (!fin) o[NP - 1] = (uint16_t)(pack2<T>(x, 0.f) & 0xffffu);
 }
