@@ -100,6 +100,29 @@ def test_infinities_and_nans_stay_in_their_rows(dev, wdt, bits):
     assert bool(((y[9].double() - ref).abs() <= 1e-4 * ref.abs()).all())
 
 
+@pytest.mark.parametrize("wdt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("rows,in_dim,H,Hk,D", [(40, 96, 2, 1, 64), (33, 2560, 4, 2, 128), (130, 1032, 4, 2, 128)])
+def test_infinite_weights_stay_infinite(dev, wdt, rows, in_dim, H, Hk, D):
+    """Infinities and NaNs among the weights give what f32 products and sums
+    give, also for values of x with empty planes (1, 0)."""
+    print(f"[qkv-gemm-winf] {wdt} rows{rows} in{in_dim}", flush=True)
+    x, ws = _inputs(dev, rows, in_dim, H, Hk, D, wdt, 12)
+    x[:, 7], x[2, 7], x[5, 90] = 1.0, 0.0, float("-inf")
+    clean = _raw(x, ws, H, Hk, D, 24)
+    inf = float("inf")
+    for w in ws:
+        w[5, 7], w[5, 11], w[9, in_dim - 1], w[11, 3], w[13, 90] = inf, inf, -inf, float("nan"), inf
+    got, w = _raw(x, ws, H, Hk, D, 24)[2], ws[2]  # v: no RoPE (whose zero sines make NaN of an infinity)
+    want = x.double() @ w.double().t().contiguous()
+    odd = ~torch.isfinite(want)
+    assert int(odd.sum()) > rows and bool(torch.isinf(want).any())
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(got[torch.isinf(want)], want[torch.isinf(want)].float())
+    keep = ~odd
+    keep[:, [5, 9, 11, 13]] = False
+    assert torch.equal(got[keep], clean[2][keep])
+
+
 @pytest.mark.parametrize("kvdt", ["f32", "bf16"])
 @pytest.mark.parametrize("rows,D,wdt,neox,rd", [(11, 256, "f16", True, 256), (50, 128, "bf16", False, 128),
                                                 (70, 64, "f32", True, 32)])

@@ -45,6 +45,8 @@ struct GemmArgs {
     int n_q, n_kv, n;          // outputs: q, k (and v), all
     int in_dim, ldx, rows;     // ldx: in_dim padded
     int mt, nt, ks;            // tiles of tokens and outputs, key ranges
+    const float *x;            // the operands themselves: [rows][in_dim],
+    const char *w[3];          // W_q, W_k, W_v
 };
 
 // SI x OI blocks of 32 x 32 per wave, WS x WO waves, NP planes of X and NW of
@@ -62,6 +64,32 @@ struct GemmCfg {
 
 // 16-byte slot swizzle of a 64-byte row: 4 rows share a 256-byte bank line.
 __device__ __forceinline__ int gm_swz(int r) { return (r >> 2) & 3; }
+
+// Output o of token row s over input dims [d0, d1), in f32: NaN as soon as the sum is.
+template <class T, int NW>
+__device__ float plain_dot(const GemmArgs &a, int s, int o, int d0, int d1) {
+    const int m = o < a.n_q ? 0 : (o < a.n_q + a.n_kv ? 1 : 2);
+    const int64_t row = o - (m == 0 ? 0 : (m == 1 ? a.n_q : a.n_q + a.n_kv));
+    const float *xr = a.x + (int64_t)s * a.in_dim;
+    float sum = 0.f;
+    for (int d = d0; d < d1 && sum == sum; d += 4) {
+        const float4 v = *(const float4 *)(xr + d);
+        float w[4];
+        if constexpr (NW == 3) {
+            const float4 t = *(const float4 *)((const float *)a.w[m] + row * a.in_dim + d);
+            w[0] = t.x, w[1] = t.y, w[2] = t.z, w[3] = t.w;
+        } else {
+            const uint2 t = *(const uint2 *)((const uint16_t *)a.w[m] + row * a.in_dim + d);
+            unpack2<T>(t.x, w[0], w[1]);
+            unpack2<T>(t.y, w[2], w[3]);
+        }
+        sum = __builtin_fmaf(w[0], v.x, sum);
+        sum = __builtin_fmaf(w[1], v.y, sum);
+        sum = __builtin_fmaf(w[2], v.z, sum);
+        sum = __builtin_fmaf(w[3], v.w, sum);
+    }
+    return sum;
+}
 
 template <class T, int NW, int NP, int SI, int OI, int WS, int WO, int KU, int NST, bool FOLD>
 __global__ __launch_bounds__(512) void qkv_gemm_kernel(GemmArgs a) {
@@ -337,6 +365,7 @@ __global__ __launch_bounds__(512) void qkv_gemm_kernel(GemmArgs a) {
             }
     }
     float *yp = a.y + (int64_t)part * a.rows * a.n;
+    bool nan = false;
 #pragma unroll
     for (int j = 0; j < SI; j++) {
         const int s = s0 + (wm * SI + j) * 32 + c32;
@@ -348,12 +377,30 @@ __global__ __launch_bounds__(512) void qkv_gemm_kernel(GemmArgs a) {
             const int ob = o0 + (wn * OI + i) * 32 + 4 * h2;
 #pragma unroll
             for (int g = 0; g < 4; g++)
-                if (ob + 8 * g < a.n)
-                    *(f32x4 *)(yr + ob + 8 * g) =
-                        f32x4{acc[0][i][j][4 * g] * f, acc[0][i][j][4 * g + 1] * f,
-                              acc[0][i][j][4 * g + 2] * f, acc[0][i][j][4 * g + 3] * f};
+                if (ob + 8 * g < a.n) {
+                    const f32x4 v = f32x4{acc[0][i][j][4 * g] * f, acc[0][i][j][4 * g + 1] * f,
+                                          acc[0][i][j][4 * g + 2] * f, acc[0][i][j][4 * g + 3] * f};
+                    *(f32x4 *)(yr + ob + 8 * g) = v;
+                    if constexpr (FOLD) nan |= v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3];
+                }
         }
     }
+    // An infinite weight times a plane of x that is zero, or of the other sign,
+    // makes NaN of what is an infinity: outputs that are NaN are summed again
+    // from the operands (rarely any; a real NaN ends its sum where it is met).
+    if constexpr (FOLD)
+        if (nan) {
+            const int d0 = kb * KD, d1 = min(ke * KD, a.in_dim);
+#pragma unroll 1
+            for (int b = 0; b < SI * OI * 16; b++) {
+                const int j = b / (OI * 16), i = b / 16 % OI;
+                const int s = s0 + (wm * SI + j) * 32 + c32;
+                const int o = o0 + (wn * OI + i) * 32 + 4 * h2 + (b % 16 / 4) * 8 + b % 4;
+                if (s >= a.rows || o >= a.n) continue;
+                float *yo = yp + (int64_t)s * a.n + o;
+                if (*yo != *yo) *yo = plain_dot<T, NW>(a, s, o, d0, d1);
+            }
+        }
 }
 
 // x = the sum of NP values of T.  An infinity or NaN goes to the last plane
@@ -590,7 +637,8 @@ extern "C" int ullm_hip_qkv_gemm_append(const float *x, int in_dim, const void *
     float *inv = (float *)(ws + pl.inv_off), *y = (float *)(ws + pl.y_off);
     const bool f16 = w_dtype == ULLM_DT_F16;
     GemmArgs a{(const char *)w_q, (const char *)w_k, (const char *)w_v, (const char *)xp,
-               f16 ? inv : nullptr, y, n_q, n_kv, n, in_dim, ld, rows, pl.mt, pl.nt, pl.ks};
+               f16 ? inv : nullptr, y, n_q, n_kv, n, in_dim, ld, rows, pl.mt, pl.nt, pl.ks,
+               x, {(const char *)w_q, (const char *)w_k, (const char *)w_v}};
     const dim3 xg((unsigned)rows), b(256);
     if (f16)
         launch_kernel((split_rows_kernel<F16, 2, true>), xg, b, 0, st, x, x, x, rows, rows, in_dim, ld, rows, xp, inv);
