@@ -66,6 +66,8 @@ unsafe extern "C" {
         head_dim: c_int, q_out: *mut c_void, q_dtype: c_int, k_cache: *mut c_void,
         v_cache: *mut c_void, kv_dtype: c_int, kv_stride: i64, workspace: *mut c_void,
         workspace_bytes: usize, stream: *mut c_void) -> c_int;
+    pub fn ullm_hip_qkv_gemm_plan(rows: c_int, in_dim: c_int, w_dtype: c_int, x_bits: c_int,
+        n_head: c_int, n_kv_head: c_int, head_dim: c_int, plan: *mut i32) -> c_int;
     pub fn ullm_hip_qkv_gemm_workspace_bytes(rows: c_int, in_dim: c_int, w_dtype: c_int,
         x_bits: c_int, n_head: c_int, n_kv_head: c_int, head_dim: c_int) -> usize;
     pub fn ullm_hip_paged_decode_workspace_bytes(batch: c_int, n_head: c_int, n_kv_head: c_int,

@@ -230,6 +230,10 @@ int ullm_hip_qkv_gemm_append(const float *x, int in_dim, const void *w_q, const 
                              void *stream);
 size_t ullm_hip_qkv_gemm_workspace_bytes(int rows, int in_dim, int w_dtype, int x_bits, int n_head,
                                          int n_kv_head, int head_dim);
+/* How such a call is cut (host only): plan[0] tokens and plan[1] outputs of a
+ * workgroup's tile, plan[2] ranges of in_dim. */
+int ullm_hip_qkv_gemm_plan(int rows, int in_dim, int w_dtype, int x_bits, int n_head, int n_kv_head,
+                           int head_dim, int32_t plan[3]);
 
 /* One decoded token from its raw q, k and v rows: the bias, norm and RoPE and
  * the cache store of ullm_hip_qkv_append (one row at position pos, full-width

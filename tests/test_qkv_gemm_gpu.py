@@ -4,6 +4,7 @@ that chooses it against the matvec path."""
 import pytest
 import torch
 
+from tests.test_gemm_rule import MODES, SHAPES
 from ullm_amd import attention as A
 
 pytestmark = pytest.mark.gpu
@@ -34,14 +35,10 @@ def _raw(x, ws, H, Hk, D, bits, start=0):
     return q, kc[start:start + rows], vc[start:start + rows]
 
 
-# Rows on both sides of the token tiles (32, 64, 128), outputs that leave part
-# of every output tile (128, 256, 384) empty, in_dim below a step, with a tail
-# of 8, 24 and 40 dims, and long enough to be split over several key ranges.
-@pytest.mark.parametrize("wdt,bits", [("bf16", 16), ("bf16", 24), ("f16", 24), ("f32", 24)])
-@pytest.mark.parametrize("rows,in_dim,H,Hk,D", [
-    (1, 8, 1, 1, 64), (31, 40, 3, 1, 64), (33, 264, 4, 2, 64), (64, 1048, 2, 2, 256),
-    (65, 2560, 8, 4, 128), (129, 1032, 9, 3, 128), (383, 544, 32, 8, 64), (1025, 512, 16, 4, 128),
-])
+# Shapes that reach every tile, whole and split, with its edges (shown on the
+# host: test_gemm_rule.py).
+@pytest.mark.parametrize("wdt,bits", MODES)
+@pytest.mark.parametrize("rows,in_dim,H,Hk,D", SHAPES)
 def test_projection_vs_f64(dev, rows, in_dim, H, Hk, D, wdt, bits):
     print(f"[qkv-gemm] rows{rows} in{in_dim} H{H} Hk{Hk} D{D} {wdt} bits{bits}", flush=True)
     x, ws = _inputs(dev, rows, in_dim, H, Hk, D, wdt, 5)

@@ -54,6 +54,7 @@ SIGNATURES = {
          _i, _i, _vp, _i, _vp, _vp, _i, _i64, _vp, _sz, _vp],
     ),
     "ullm_hip_qkv_gemm_workspace_bytes": (_sz, [_i, _i, _i, _i, _i, _i, _i]),
+    "ullm_hip_qkv_gemm_plan": (_i, [_i, _i, _i, _i, _i, _i, _i, _vp]),
     "ullm_hip_decode_token": (
         _i,
         [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _f, _vp, _i, _i, _i, _vp, _i, _i, _i, _i, _f,

@@ -574,15 +574,29 @@ static void launch_gemm(int tile, const GemmArgs &a, hipStream_t st) {
 
 using namespace ullm;
 
+static bool plan_call(int rows, int in_dim, int w_dtype, int x_bits, int n_head, int n_kv_head, int head_dim,
+                      GemmPlan &pl) {
+    return rows >= 1 && in_dim >= 8 && in_dim % 8 == 0 && dtype_ok(w_dtype) && (x_bits == 16 || x_bits == 24) &&
+           n_head >= 1 && n_kv_head >= 1 && (head_dim == 64 || head_dim == 128 || head_dim == 256) &&
+           ((int64_t)n_head + 2 * (int64_t)n_kv_head) * head_dim <= 0x7fffffff &&
+           gemm_plan(rows, in_dim, w_dtype, x_bits, (n_head + 2 * n_kv_head) * head_dim, pl);
+}
+
 extern "C" size_t ullm_hip_qkv_gemm_workspace_bytes(int rows, int in_dim, int w_dtype, int x_bits,
                                                     int n_head, int n_kv_head, int head_dim) {
     GemmPlan pl;
-    if (rows < 1 || in_dim < 8 || in_dim % 8 || !dtype_ok(w_dtype) || (x_bits != 16 && x_bits != 24) ||
-        n_head < 1 || n_kv_head < 1 || (head_dim != 64 && head_dim != 128 && head_dim != 256) ||
-        ((int64_t)n_head + 2 * (int64_t)n_kv_head) * head_dim > 0x7fffffff ||
-        !gemm_plan(rows, in_dim, w_dtype, x_bits, (n_head + 2 * n_kv_head) * head_dim, pl))
-        return 0;
-    return pl.bytes;
+    return plan_call(rows, in_dim, w_dtype, x_bits, n_head, n_kv_head, head_dim, pl) ? pl.bytes : 0;
+}
+
+extern "C" int ullm_hip_qkv_gemm_plan(int rows, int in_dim, int w_dtype, int x_bits, int n_head, int n_kv_head,
+                                      int head_dim, int32_t *plan) {
+    GemmPlan pl;
+    if (!plan) return set_error(ULLM_HIP_E_INVALID, "qkv_gemm_plan: null pointer");
+    if (!plan_call(rows, in_dim, w_dtype, x_bits, n_head, n_kv_head, head_dim, pl))
+        return set_error(ULLM_HIP_E_UNSUPPORTED, "qkv_gemm_plan: %d rows, %d -> %d/%d heads x %d, dtype %d", rows,
+                         in_dim, n_head, n_kv_head, head_dim, w_dtype);
+    plan[0] = kGmTile[pl.tile].bs, plan[1] = kGmTile[pl.tile].bo, plan[2] = pl.ks;
+    return ULLM_HIP_OK;
 }
 
 extern "C" int ullm_hip_qkv_gemm_append(const float *x, int in_dim, const void *w_q,
