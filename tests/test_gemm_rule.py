@@ -71,7 +71,8 @@ def test_plan_validation():
     ((16, 10240, 8192, 128, F32), 369, 293), ((2, 18432, 16384, 128, F32), 365, 1165), ((8, 18432, 16384, 128, F32), 1070, 1183),
     ((12, 18432, 16384, 128, F32), 1529, 1176), ((8, 8192, 3584, 256, F32), 203, 91), ((6, 8192, 3584, 256, F32), 62, 91),
     ((2, 32768, 8192, 256, F32), 508, 912), ((4, 32768, 8192, 256, F32), 1005, 915), ((2, 32768, 8192, 256, BF16), 530, 116),
-    ((1, 32768, 8192, 256, F16), 103, 123), ((16, 4096, 2560, 256, BF16), 150, 20),
+    ((1, 32768, 8192, 256, F16), 103, 123), ((8, 8192, 512, 256, F32), 27, 30),
+    ((9, 8192, 512, 256, F32), 45, 30), ((8, 8192, 768, 256, F32), 39, 31), ((16, 4096, 2560, 256, BF16), 150, 20),
 ])
 def test_rule_takes_the_faster_side(call, matvec, gemm):
     assert _gemm_pays(*call) == (gemm < matvec)

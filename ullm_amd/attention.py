@@ -195,9 +195,11 @@ def _gemm_pays(rows, n, in_dim, head_dim, w_dtype):
     294, 12 rows 302 / 293; 16384 -> 18432 2 rows 365 / 1165, 12 rows 1529 / 1176.
     head_dim 256 from 256 head vectors on, where the matvec is 4 to 9 times
     slower (3584 -> 8192 6 / 8 rows: bf16 37 / 223 against 26, f32 62 / 203
-    against 91); f32 8192 -> 32768: 2 rows 508 / 912, 3 rows 940 / 919."""
+    against 91); f32 8192 -> 32768: 2 rows 508 / 912, 3 rows 940 / 919; f32 512 ->
+    8192: 8 rows (one round of 256 workgroups) 27 / 30, 9 rows 45 / 30."""
     f32 = w_dtype == torch.float32
-    if head_dim == 256 and rows * (n // head_dim) >= 256 and not (f32 and rows < 3):
+    heads = rows * (n // head_dim)
+    if head_dim == 256 and heads >= 256 and not (f32 and (rows < 3 or (heads == 256 and in_dim < 768))):
         return True
     work = rows * n * in_dim
     if f32:
