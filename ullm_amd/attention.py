@@ -213,9 +213,12 @@ def qkv_proj_append(x, w_q, w_k, w_v, k_cache, v_cache, rope_cs, *, start_pos, n
                     kv_stride=None, workspace=None, stream=None):
     """Q/K/V projection (matvec_q, math.rs:9-21) with the append fused in
     (lib.rs:857-914).  x: [rows, in_dim] f32; w_*: [out, in_dim] f32/f16/bf16.
-    Returns q_out ([rows, n_head*D], q_dtype); K/V land in the cache.  The
-    workspace defaults to a cached one per shape (one caller at a time, as for
-    GpuForward)."""
+    Returns q_out ([rows, n_head*D], q_dtype); K/V land in the cache.  Few rows
+    run as a matvec per row, whose workspace defaults to a cached one per shape
+    (one caller at a time, as for GpuForward); more rows (`_gemm_pays`) as one
+    GEMM with scratch of its own (rows x outputs x 4 bytes per range of in_dim,
+    and x in planes: ullm_hip_qkv_gemm_workspace_bytes), `workspace` unused, or
+    row by row where that memory is not there."""
     rows, in_dim = x.shape
     n = (n_head + 2 * n_kv_head) * head_dim
     args = (x, w_q, w_k, w_v, k_cache, v_cache, start_pos)
@@ -389,8 +392,11 @@ class GpuAttention:
     def forward_proj(self, layer: int, xb, pos: int, wq, wk, wv, q_norm=None, k_norm=None,
                      q_bias=None, k_bias=None, v_bias=None):
         """Decode one token from the attention-normed hidden state xb [n_embd]
-        f32 (forward.rs:415-466): the Q/K/V matvecs with bias, norm, RoPE and
-        the cache store fused into one launch, then decode attention."""
+        f32 (forward.rs:415-466): the Q/K/V matvecs in one launch, then the
+        attention's two launches, which prepare q and the token's key (bias,
+        norm, RoPE) and store its cache row.  Where those do not take the shape
+        (the first 33 positions, head_dim 256, partial rotary, unaligned rows):
+        the projection with the append fused in, then decode attention."""
         p = self.p
         if not 0 <= pos < p.n_ctx:
             raise L.UllmHipError(L.E_INVALID, f"pos {pos} outside the context")
@@ -400,10 +406,11 @@ class GpuAttention:
     def forward_batch_proj(self, layer: int, xbs, wq, wk, wv, start_pos: int = 0, q_norm=None,
                            k_norm=None, q_bias=None, k_bias=None, v_bias=None):
         """Prefill S tokens from the attention-normed hidden states xbs
-        [S, n_embd] f32 (forward.rs:799-858): with bf16 weights the three
-        projections run as MFMA matmuls (forward.rs:799-801), then the fused
-        append and causal prefill attention; other weight dtypes use the
-        fused projection kernel over the S rows."""
+        [S, n_embd] f32 (forward.rs:799-858): the three projections
+        (forward.rs:799-801) as one MFMA GEMM with the append behind it, for few
+        rows as a matvec per row (`_gemm_pays`), then causal prefill attention.
+        bf16 weights take 16 significant bits of xbs, other weight dtypes 22 or
+        24 (ullm_hip_qkv_gemm_append)."""
         p = self.p
         S = xbs.shape[0]
         if start_pos + S > p.n_ctx:
@@ -446,7 +453,8 @@ class GpuAttention:
         projections come from the fused projection at position 0 with no
         norm or bias (RoPE at position 0 is the identity), then the bias,
         the Q/K norms and RoPE follow as appends into scratch rows, and the
-        last append writes the cache row exactly as forward_proj does.  The
+        last append writes the cache row as forward_proj does (which sums the
+        projections in another order: equal to f32 rounding).  The
         attention scores are never materialised by this path, so the report
         goes from rope_k to attn_out.  Returns (attention output, report:
         a list of (label, nan, inf, maxabs))."""

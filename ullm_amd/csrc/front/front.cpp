@@ -3,10 +3,10 @@
 //
 // A decode step is launch-bound: the kernels of one layer take 6 to 20 us and
 // the host has to queue them faster than that.  Host time of one call, us,
-// through ctypes and here: attn_decode 12.7 -> 7.0 (two launches 5.3; ctypes
-// spent 2.9 on the current stream, 1.4 on the output, the rest on arguments),
-// GpuAttention.forward 28.7 -> 10.8 and forward_proj 30.5 -> 11.3 (three
-// launches, one native call).  Functions take positional arguments only
+// through ctypes and here: attn_decode 12.7 -> 7.2 (two launches; ctypes spent
+// 2.9 on the current stream, 1.4 on the output, the rest on arguments),
+// GpuAttention.forward 28.7 -> 6.7 (three launches -> the fused step's two) and
+// forward_proj 30.5 -> 10.6 (three on both sides).  Functions take positional arguments only
 // (METH_FASTCALL); attention.py holds the signatures, defaults and documentation.
 // Nothing is kept between calls.
 #include <torch/csrc/autograd/python_variable.h>

@@ -6,12 +6,6 @@
 
 namespace ullm {
 
-template <int N>
-struct VecF;
-template <> struct VecF<1> { typedef float t; };
-template <> struct VecF<2> { typedef float2 t; };
-template <> struct VecF<4> { typedef float4 t; };
-
 template <int E>
 __device__ __forceinline__ void load_e(const float *p, float (&x)[E]) {
     if constexpr (E == 1) x[0] = p[0];

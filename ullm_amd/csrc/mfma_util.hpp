@@ -345,7 +345,7 @@ inline KeySplit split_at(const SplitPlan &pl, int tile, void *ws) {
 // Head_dim-256 prefill on 16-row waves, two per SIMD (prefill16.hip);
 // pgs.tab == nullptr for a contiguous cache.
 // ws: scratch for a split of the key ranges over workgroups, used where the
-// plan asks for one and ws_bytes holds it (prefill16_ws_bytes).
+// plan asks for one and ws_bytes holds it (ullm_hip_prefill_workspace_bytes).
 int launch_prefill16(int dtype, const void *q, const void *kc, const void *vc, int64_t kvs, int S,
                      int start_pos, int window, int n_head, int kv_mul, float qs, float *out,
                      hipStream_t st, KvPages pgs, void *ws = nullptr, size_t ws_bytes = 0);

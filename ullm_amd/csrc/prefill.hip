@@ -1223,10 +1223,11 @@ static SplitPlan prefill4_split(int S, int sp, int nh, int kv_mul, int D) {
 // cost 0.6 us per 32-key tile (32/8 heads x 64: 777 rows, 25 tiles, 21.1 us; 500
 // rows at 4000, 141 tiles, 84), one set 1.0; with more workgroups than CUs two
 // one-set workgroups share one and start their next unit on their own, which
-// is better for short units: 2000 rows, window 300 (504 units of 13 tiles) 27.7
+// is better for short units: 2000 rows, window 300 (504 units of 13 tiles) 24.8
 // us against 32.5, 100 rows (4 tiles) 8.2 against 9.1.  Measured (us, causal
-// pairs of units on one set -> this rule): 777 rows 33.9 -> 21.1, 1000 41.5 -> 24.9,
-// 2048 80 -> 57, 4096 216 -> 195, 500 at 4000 256 -> 55, 61 at 700 52 -> 13.
+// pairs of units on one set -> this rule): 777 rows 33.9 -> 21.0, 1000 41.5 -> 24.6,
+// 2048 80 -> 55, 4096 216 -> 165, 500 at 4000 256 -> 52 and 61 at 700 52 -> 12.5
+// (both split).
 static bool prefill_f32_two_sets(double wgs, double longest) {
     return longest > (wgs > 256 ? 16 : 4);
 }

@@ -508,7 +508,7 @@ struct GemmPlan {
 //   2048 rows: 128 x 384 129 (256 tiles: one round; the GEMM 105, 1.23
 //     PFLOP/s executed), 128 x 256 158, 128 x 128 179; the three
 //     ullm_hip_matmul launches and the append it replaces: 171;
-//   61 rows: 64 x 128 in 4 ranges 21.8, 5 ranges 22.1, 2 ranges 25.2, unsplit
+//   61 rows: 64 x 128 in 5 ranges (taken) 22.1, 4 ranges 21.8, 2 ranges 25.2, unsplit
 //     35.9, 32 x 256 23.3; replaced: 90.
 static bool gemm_plan(int rows, int in_dim, int w_dtype, int x_bits, int n, GemmPlan &pl) {
     const int ld = (in_dim + kGmPad - 1) / kGmPad * kGmPad, nk = ld / kGmK;
