@@ -122,6 +122,21 @@ def test_calls_do_without_scratch_they_cannot_have(dev, monkeypatch):
     assert torch.equal(out, whole) and torch.equal(qo, want)
 
 
+@pytest.mark.parametrize("window", [-1, N, 2 ** 31 - 1, 2 ** 31, 2 ** 63 - 1])
+def test_windows_that_hide_nothing(dev, window):
+    q, k, v, lens = _cache(dev)
+    qp = torch.randn(9, H * D, device=dev).half()
+    assert torch.equal(A.attn_decode(q, k, v, lens, N, Hk, window=window), A.attn_decode(q, k, v, lens, N, Hk))
+    assert torch.equal(A.attn_prefill(qp, k, v, H, Hk, D, start_pos=N - 9, window=window),
+                       A.attn_prefill(qp, k, v, H, Hk, D, start_pos=N - 9))
+    outs = []
+    for w in (0, window):
+        ga = A.GpuAttention(A.AttnParams(1, H, Hk, D, N, sliding_window=w))
+        ga.key_cache[0], ga.val_cache[0] = k, v
+        outs.append(ga.forward(0, q.view(-1), torch.ones(Hk * D, device=dev), torch.ones(Hk * D, device=dev), 200))
+    assert torch.equal(*outs)
+
+
 def test_layer_indices(dev):
     ga = A.GpuAttention(A.AttnParams(3, H, Hk, D, 16, kv_dtype=torch.float32))
     q, kk = torch.randn(H * D, device=dev), torch.randn(Hk * D, device=dev)

@@ -14,6 +14,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
+#include <climits>
 #include <cmath>
 #include <optional>
 
@@ -57,6 +58,11 @@ struct Args {
         const int64_t v = i64(i);
         if (v != (int)v) raise(PyExc_OverflowError, "integer argument out of range");
         return (int)v;
+    }
+    // A window; one past every position (2^31 and more) is none.
+    int window(int i) const {
+        const int64_t v = i64(i);
+        return v > INT_MAX || v < 0 ? 0 : (int)v;
     }
     double f(int i) const {
         const double v = PyFloat_AsDouble(a[i]);
@@ -150,7 +156,7 @@ at::Tensor decode(const Args &a) {
     const at::Tensor &q = a.t(0), &k = a.t(1), &v = a.t(2), &lens = a.t(3);
     if (q.dim() != 3) raise(PyExc_ValueError, "q must be [B, n_head, head_dim]");
     const int B = (int)q.size(0), H = (int)q.size(1), D = (int)q.size(2), max_len = a.i32(4), hk = a.i32(5),
-              win = a.i32(6);
+              win = a.window(6);
     need_cuda({&q, &k, &v, &lens});
     if (!f32_rows(q)) invalid("q must be contiguous f32 [B, n_head, head_dim]");
     if (lens.scalar_type() != at::kInt || lens.numel() != B) invalid("seq_lens must be int32 [B]");
@@ -175,7 +181,7 @@ at::Tensor decode_paged(const Args &a) {
     const at::Tensor &q = a.t(0), &k = a.t(1), &v = a.t(2), &tab = a.t(3), &lens = a.t(4);
     if (q.dim() != 3) raise(PyExc_ValueError, "q must be [B, n_head, head_dim]");
     const int B = (int)q.size(0), H = (int)q.size(1), D = (int)q.size(2), max_len = a.i32(5), hk = a.i32(6),
-              win = a.i32(7);
+              win = a.window(7);
     need_cuda({&q, &k, &v, &tab, &lens});
     if (!f32_rows(q)) invalid("q must be contiguous f32 [B, n_head, head_dim]");
     if (k.dim() != 3 || k.sizes() != v.sizes() || !k.is_contiguous() || !v.is_contiguous())
@@ -345,7 +351,7 @@ PyObject *proj(const Args &a) {
 at::Tensor prefill(const Args &a) {
     // q k_cache v_cache n_head n_kv head_dim start_pos window scale kv_stride out stream max_q_bytes
     const at::Tensor &q = a.t(0), &k = a.t(1), &v = a.t(2);
-    const int H = a.i32(3), hk = a.i32(4), D = a.i32(5), start = a.i32(6), win = a.i32(7);
+    const int H = a.i32(3), hk = a.i32(4), D = a.i32(5), start = a.i32(6), win = a.window(7);
     const int64_t S = q.size(0), row = (int64_t)H * D;
     need_cuda({&q, &k, &v});
     if (!q.is_contiguous() || q.numel() != S * row) invalid("q must be contiguous [S, n_head*head_dim]");
@@ -373,7 +379,7 @@ at::Tensor prefill(const Args &a) {
 at::Tensor prefill_paged(const Args &a) {
     // q k_pages v_pages block_table n_head n_kv head_dim start_pos window scale out stream
     const at::Tensor &q = a.t(0), &k = a.t(1), &v = a.t(2), &tab = a.t(3);
-    const int H = a.i32(4), hk = a.i32(5), D = a.i32(6), start = a.i32(7), win = a.i32(8);
+    const int H = a.i32(4), hk = a.i32(5), D = a.i32(6), start = a.i32(7), win = a.window(8);
     const int64_t S = q.size(0), row = (int64_t)H * D;
     need_cuda({&q, &k, &v, &tab});
     if (!q.is_contiguous() || q.numel() != S * row) invalid("q must be contiguous [S, n_head*head_dim]");
@@ -413,7 +419,7 @@ at::Tensor token(const Args &a) {
     // proj layer pos key_cache val_cache lens ws window scale <Prep> in0..in3 proj_ws
     const bool is_proj = a.truth(0);
     const int64_t layer = a.i64(1);
-    const int pos = a.i32(2), win = a.i32(7);
+    const int pos = a.i32(2), win = a.window(7);
     const at::Tensor &kc = a.t(3), &vc = a.t(4), &lens = a.t(5), &ws = a.t(6);
     const float scale = (float)a.f(8);
     const Prep p(a, 9);
