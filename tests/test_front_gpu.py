@@ -137,6 +137,42 @@ def test_windows_that_hide_nothing(dev, window):
     assert torch.equal(*outs)
 
 
+def test_calls_with_scratch_replay_from_a_graph(dev):
+    """Few-row and GEMM projections, a split prefill and the decode step
+    (fused, and with rows in the cache), captured together: each replay on new
+    inputs, with eager work between, gives what the calls give eagerly."""
+    H, Hk, D, E, n = 32, 8, 128, 2560, 4200
+    gen = torch.Generator(device=dev).manual_seed(8)
+    rn = lambda *s: torch.randn(*s, device=dev, generator=gen)  # noqa: E731
+    ga, gf = (A.GpuAttention(A.AttnParams(1, H, Hk, D, n, kv_dtype=t)) for t in (torch.bfloat16, torch.float32))
+    w = [(rn(m * D, E) / 50).bfloat16() for m in (H, Hk, Hk)]
+    x3, x70, q, kv = rn(3, E), rn(70, E), rn(H * D), rn(2, Hk * D)
+
+    def step():
+        gf.key_cache[0, 4100], gf.val_cache[0, 4100] = kv[0], kv[1]
+        return [ga.forward_batch_proj(0, x3, *w, 4000), ga.forward_batch_proj(0, x70, *w, 4010),
+                ga.forward(0, q, kv[0], kv[1], 4090), gf.forward(0, q, kv[0], kv[1], 4099),
+                gf.forward(0, q, gf.key_cache[0, 4100], gf.val_cache[0, 4100], 4100)]
+
+    step()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = step()
+    for _ in range(4):
+        for t in (x3, x70, q, kv):
+            t.copy_(rn(*t.shape))
+        want = [o.clone() for o in step()]
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(outs, want))
+
+
 def test_layer_indices(dev):
     ga = A.GpuAttention(A.AttnParams(3, H, Hk, D, 16, kv_dtype=torch.float32))
     q, kk = torch.randn(H * D, device=dev), torch.randn(Hk * D, device=dev)
