@@ -181,12 +181,12 @@ __global__ __launch_bounds__(512) void qkv_gemm_kernel(GemmArgs a) {
     }
 
     // FOLD: the matrix cores sum one step from zero, smallest products first,
-    // into acc[0] and acc[1] in turn (BYP: each plane of X into its own).  The step before is added to `sum` in
-    // f32 in the shadow of the MFMAs, and every eight steps `sum` goes to
-    // `top`, so that few additions round at the size of the whole result.
-    // Relative error at in_dim 2048..2560 (f64 reference): 1.0e-7..1.1e-7,
-    // against 1.2e-7..1.3e-7 of qkv_proj_kernel's f32 sums and 2.5e-7..5.6e-7
-    // of one chain of MFMAs.
+    // into acc[0] and acc[1] in turn (BYP: each plane of X into its own).  The
+    // step before is added to `sum` in f32 in the shadow of the MFMAs, and every
+    // eight steps `sum` goes to `top`, so that few additions round at the size of
+    // the whole result.  Relative error at in_dim 2048..2560 (f64 reference):
+    // 0.9e-7..1.1e-7, against 1.2e-7..1.3e-7 of qkv_proj_kernel's f32 sums and
+    // 2.5e-7..5.6e-7 of one chain of MFMAs.
     constexpr bool BYP = FOLD && __is_same(T, F16);
     constexpr int NA = FOLD ? 2 : 1;
     f32x16 acc[NA][OI][SI], sum[FOLD ? OI : 1][FOLD ? SI : 1], top[FOLD ? OI : 1][FOLD ? SI : 1];
@@ -243,7 +243,8 @@ __global__ __launch_bounds__(512) void qkv_gemm_kernel(GemmArgs a) {
     };
     constexpr int NMF = 2 * KU * OI * SI * (NW == 3 ? 6 : NP);  // MFMAs per step
     // BYP: plane 1 of this step while plane 0 of the step before is added to
-    // `sum`, then plane 0 while plane 1 is added.
+    // `sum`, then plane 0 while plane 1 is added (twice the additions, under the
+    // same MFMAs: 1000 rows x 2048 -> 3072 38.6 -> 39.0 us, traced).
     auto by_plane = [&](auto pc) {
         constexpr int p = decltype(pc)::value;
         constexpr int NM = 2 * KU * OI * SI, V = (OI * SI * 16 + NM - 1) / NM + 1;
